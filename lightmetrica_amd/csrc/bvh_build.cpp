@@ -370,6 +370,22 @@ bool build_wide_bvh(const float* positions, uint32_t num_vertices, const uint32_
     return true;
 }
 
+uint32_t place_leaves(WideBVH& bvh) {
+    const bool pad = bvh.tris.size() + bvh.num_leaves <= size_t(kMaxLeafFirst);
+    uint32_t next = 0;
+    // In the order of the nodes' slots, which is the order of the records.
+    for (Node4& n : bvh.nodes)
+        for (int slot = 0; slot < 4; slot++) {
+            const uint32_t c = n.child[slot];
+            if (c == kEmptyChild || !(c & kLeafBit)) continue;
+            const uint32_t count = ((c >> 27) & 0xfu) + 1u;
+            if (pad && count > 1u) next = (next + 1u) & ~1u;
+            n.pad[slot] = next;
+            next += count;
+        }
+    return next;
+}
+
 std::vector<XformRecord> make_xform_records(const std::vector<TriRecord>& tris) {
     std::vector<XformRecord> out(tris.size());
     for (size_t k = 0; k < tris.size(); k++) {

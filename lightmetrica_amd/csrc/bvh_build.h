@@ -25,6 +25,15 @@ struct alignas(128) Node4 {
 };
 static_assert(sizeof(Node4) == 128, "Node4 must be one 128-byte line");
 
+// The node as the device keeps it: planes are 8-bit steps from `origin`, four children to a word
+// (planes[axis][0] the lower, planes[axis][1] the upper ones).
+struct alignas(64) NodeQ {
+    float origin[3], step[3];
+    uint32_t planes[3][2];
+    uint32_t child[4];
+};
+static_assert(sizeof(NodeQ) == 64, "NodeQ is half a 128-byte line");
+
 // Child reference encoding.
 constexpr uint32_t kLeafBit = 0x80000000u;
 constexpr uint32_t kEmptyChild = 0xffffffffu;
@@ -41,6 +50,24 @@ struct alignas(16) TriRecord {
     float v2[4];
 };
 static_assert(sizeof(TriRecord) == 48, "TriRecord is 48 bytes");
+
+// The triangle record as the BVH traversal reads it, two to a 128-byte line: v0.w the scene-order
+// triangle index, the rest of the fourth column and box_yz the box of the record's leaf as it
+// was built (v1.w, v2.w its x range).
+struct alignas(64) LeafTri {
+    float v0[4], v1[4], v2[4];
+    float box_yz[4];  // lo y, hi y, lo z, hi z
+};
+static_assert(sizeof(LeafTri) == 64, "LeafTri is half a 128-byte line");
+
+// What a traversal reads.  `exact` are the nodes as they were built and `reach` the largest
+// coordinate of the scene's box: for the rays that trace_exact (traverse.hpp) decides.
+struct BvhDev {
+    const NodeQ* nodes;
+    const LeafTri* tris;
+    const Node4* exact;
+    float reach;
+};
 
 // Affine-transform record of a triangle for the path tracer of scenes small enough to test
 // every triangle per ray (Baldwin and Weber, "Fast Ray-Triangle Intersections by Coordinate
@@ -83,6 +110,12 @@ struct WideBVH {
     double sah_cost = 0.0;
     double build_seconds = 0.0;
 };
+
+// Places the leaves of `bvh` for the device: pad[slot] of a node becomes the first LeafTri of the
+// leaf in that child slot.  A leaf of two or more records starts on a line, so that it takes no
+// more lines than it fills, unless the padded array would outgrow the 27-bit leaf offsets.
+// Returns the number of LeafTri.
+uint32_t place_leaves(WideBVH& bvh);
 
 // positions: 3 floats per vertex; faces: 3 indices per triangle.
 // Returns false with `err` set when the input cannot be built.  A tree deeper than

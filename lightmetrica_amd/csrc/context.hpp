@@ -100,8 +100,16 @@ struct lmgpu_ctx {
     bool has_camera = false;
 
     // Device scene
-    lmgpu::DevBuf<lmgpu::Node4> nodes;
-    lmgpu::DevBuf<lmgpu::TriRecord> tris;
+    // One allocation, nodes.ptr: the packed nodes, the nodes as built (as many) and the records.
+    lmgpu::DevBuf<lmgpu::NodeQ> nodes;
+    lmgpu::Node4* exact_nodes = nullptr;
+    float reach = 0.f;                        // the largest coordinate of the scene's box
+    lmgpu::DevBuf<lmgpu::TriRecord> tris;  // scenes of at most kBruteMaxTris triangles, else empty
+    struct {
+        lmgpu::LeafTri* ptr;
+        size_t count;
+    } leaf_tris{nullptr, 0};
+    uint32_t num_records = 0;  // triangle records of the built tree
     lmgpu::DevBuf<lmgpu::XformRecord> xform;  // scenes of at most kBruteMaxTrisPt triangles, else empty
     uint32_t bvh_max_depth = 0;
     bool has_bvh = false;
@@ -157,6 +165,10 @@ struct lmgpu_ctx {
 
 namespace lmgpu {
 
+inline BvhDev bvh_of(const lmgpu_ctx* ctx) {
+    return BvhDev{ctx->nodes.ptr, ctx->leaf_tris.ptr, ctx->exact_nodes, ctx->reach};
+}
+
 // Status helpers: set ctx->err and return a status.
 lmgpu_status fail(lmgpu_ctx* ctx, lmgpu_status s, const std::string& msg);
 lmgpu_status hip_fail(lmgpu_ctx* ctx, hipError_t e, const char* what);
@@ -182,6 +194,8 @@ template <class Fn> hipError_t timed(lmgpu_ctx* ctx, int cls, Fn&& launch) {
 }
 
 // Kernel launchers (trace_kernels.hip, pt_kernels.hip).
+// The traversal's nodes and triangle records from the uploaded ones.
+hipError_t launch_pack_nodes(lmgpu_ctx* ctx);
 // `next`: the work counter of the persistent traversal.
 hipError_t launch_trace_closest(lmgpu_ctx* ctx, const float* const* rays, uint32_t n, float* t, float* b0, float* b1,
                                 int32_t* prim, bool refine, uint32_t* next);

@@ -480,10 +480,35 @@ lmgpu_status lmgpu_bvh_build(lmgpu_ctx* ctx, const lmgpu_bvh_params* params, lmg
         return fail(ctx, LMGPU_ERR_BVH_TOO_DEEP, "lmgpu_bvh_build: tree depth " + std::to_string(w.max_depth) +
                                                      " exceeds the traversal stack (max 32)");
     ctx->has_bvh = false;
-    lmgpu_status s = upload(ctx, ctx->nodes, w.nodes.data(), w.nodes.size(), "BVH nodes");
+    // Nodes and records go up as they are built and are packed and placed on the device.
+    const size_t nn = w.nodes.size(), nt = place_leaves(w);
+    const size_t packed_bytes = sizeof(NodeQ) * nn, exact_bytes = sizeof(Node4) * nn, leaf_bytes = sizeof(LeafTri) * nt;
+    free_buf(ctx->nodes);
+    free_buf(ctx->tris);
+    void* block = nullptr;
+    const size_t packed_pad = (packed_bytes + 127) / 128 * 128;
+    lmgpu_status s = dev_alloc(ctx, &block, packed_pad + exact_bytes + leaf_bytes, "BVH");
     if (s != LMGPU_OK) return s;
+    ctx->nodes.ptr = static_cast<NodeQ*>(block);
+    ctx->nodes.count = nn;
+    ctx->exact_nodes = reinterpret_cast<Node4*>(static_cast<char*>(block) + packed_pad);
+    ctx->leaf_tris = {reinterpret_cast<LeafTri*>(static_cast<char*>(block) + packed_pad + exact_bytes), nt};
+    ctx->num_records = uint32_t(w.tris.size());
+    hipError_t e = hipMemcpyAsync(ctx->exact_nodes, w.nodes.data(), exact_bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e != hipSuccess) return hip_fail(ctx, e, "BVH nodes");
     s = upload(ctx, ctx->tris, w.tris.data(), w.tris.size(), "triangle records");
     if (s != LMGPU_OK) return s;
+    e = launch_pack_nodes(ctx);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess) return hip_fail(ctx, e, "k_pack_nodes");
+    if (w.tris.size() > kBruteMaxTris) free_buf(ctx->tris);
+    ctx->reach = 0.f;
+    const Node4& root = w.nodes[0];
+    for (int i = 0; i < 4; i++) {
+        if (root.child[i] == kEmptyChild) continue;
+        for (float v : {root.lo_x[i], root.hi_x[i], root.lo_y[i], root.hi_y[i], root.lo_z[i], root.hi_z[i]})
+            ctx->reach = std::max(ctx->reach, std::fabs(v));
+    }
     // The path tracer of a scene small enough to test every triangle per ray tests the
     // triangles' transform records.
     free_buf(ctx->xform);
@@ -501,7 +526,7 @@ lmgpu_status lmgpu_bvh_build(lmgpu_ctx* ctx, const lmgpu_bvh_params* params, lmg
         info->num_tri_records = uint32_t(w.tris.size());
         info->build_seconds = w.build_seconds;
         info->sah_cost = w.sah_cost;
-        info->device_bytes = uint64_t(w.nodes.size()) * sizeof(Node4) + uint64_t(w.tris.size()) * sizeof(TriRecord);
+        info->device_bytes = uint64_t(packed_bytes + exact_bytes + leaf_bytes);
     }
     return LMGPU_OK;
 }

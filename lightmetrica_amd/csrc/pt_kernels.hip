@@ -62,8 +62,7 @@ constexpr int kDiffuseReflection = 1 << 0;
 constexpr int kSpecularReflection = 1 << 2;
 
 struct PTConsts {
-    const Node4* nodes;
-    const TriRecord* tris;
+    BvhDev bvh;
     const XformRecord* xform;  // scenes of at most kBruteMaxTrisPt triangles: the records' transforms
     const ShadeTri* shade;
     const MaterialDev* mats;
@@ -803,7 +802,7 @@ struct QueueSource {
 };
 
 struct HitSink {
-    const TriRecord* tris;
+    const LeafTri* tris;
     float4* hits;
     __device__ __forceinline__ void operator()(uint32_t i, bool found, const HitOut& h, const RayIn& r) const {
         float4 out = make_float4(0.f, 0.f, 0.f, __uint_as_float(kMiss));
@@ -833,16 +832,15 @@ __device__ __forceinline__ void add_wave_counts(const TraceCounters& cnt, unsign
 // kCount (lmgpu_enable_counting): also counts node visits and triangle tests into `counts`.
 // 6 waves per SIMD, as the LDS stack allows (the bound keeps the kernel within 80 VGPRs).
 template <bool kCount = false>
-__global__ __launch_bounds__(kTraceBlock, 6) void k_extend(const Node4* __restrict__ nodes,
-                                                        const TriRecord* __restrict__ tris, Queue q,
+__global__ __launch_bounds__(kTraceBlock, 6) void k_extend(BvhDev bvh, Queue q,
                                                         const uint32_t* __restrict__ count, uint32_t* next,
                                                         float4* __restrict__ hits, unsigned long long* counts) {
     __shared__ TraceShared<true> sm;
     const uint32_t n = *count;
     QueueSource src{q};
-    HitSink sink{tris, hits};
+    HitSink sink{bvh.tris, hits};
     TraceCounters cnt{0, 0};
-    trace_persistent<false, kCount, false>(nodes, tris, n, next, sm, src, sink, cnt);
+    trace_persistent<false, kCount>(bvh, n, next, sm, src, sink, cnt);
     if (kCount) add_wave_counts(cnt, counts);
 }
 
@@ -1139,7 +1137,7 @@ __global__ __launch_bounds__(kTraceBlock, 7) void k_shadow(PTConsts c, ShadowQue
     ShadowSource src{sq};
     ShadowSink<kMode, kSplat> sink{c, sq};
     TraceCounters cnt{0, 0};
-    trace_persistent<true, kCount, false>(c.nodes, c.tris, n, next, sm, src, sink, cnt);
+    trace_persistent<true, kCount>(c.bvh, n, next, sm, src, sink, cnt);
     if (kCount) add_wave_counts(cnt, counts);
 }
 
@@ -1210,7 +1208,7 @@ struct RaycastSink {
         float4 hit = make_float4(0.f, 0.f, 0.f, __uint_as_float(kMiss));
         if (found) {
             float t, b0, b1;
-            winner_barycentrics(c.tris, r, h, false, t, b0, b1);
+            winner_barycentrics(c.bvh.tris, r, h, false, t, b0, b1);
             hit = make_float4(t, b0, b1, __uint_as_float(h.prim));
         }
         Surf s;
@@ -1228,7 +1226,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_raycast(PTConsts c, uint32_t n,
     RaycastSource src{c.cam};
     RaycastSink<Out> sink{c, out};
     TraceCounters cnt{0, 0};
-    trace_persistent<false, false, true>(c.nodes, c.tris, n, next, sm, src, sink, cnt);
+    trace_persistent<false, false>(c.bvh, n, next, sm, src, sink, cnt);
 }
 
 __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
@@ -1554,9 +1552,8 @@ struct Pipeline {
         ctx->pt_capacity = cap;
         carve(ctx->pt_buf, cap, b);
         c = PTConsts{};
-        c.nodes = ctx->nodes.ptr;
-        c.tris = ctx->tris.ptr;
-        c.xform = ctx->xform.ptr;
+        c.bvh = bvh_of(ctx);
+            c.xform = ctx->xform.ptr;
         c.shade = ctx->shade.ptr;
         c.mats = ctx->mats.ptr;
         c.lights = ctx->lights.ptr;
@@ -1581,13 +1578,13 @@ struct Pipeline {
         // Segments traced per path: at most max_path_vertices - 1 (pathtrace.cpp:196-199).
         segments = c.max_pv - 1;
         is_pt = p->renderer == LMGPU_PT;
-        brute = ctx->tris.count <= (is_pt ? kBruteMaxTrisPt : kBruteMaxTris);
-        c.ntris = uint32_t(ctx->tris.count);
+        brute = ctx->num_records <= (is_pt ? kBruteMaxTrisPt : kBruteMaxTris);
+        c.ntris = ctx->num_records;
         // A BVH larger than the caches: camera rays in screen-tile order (k_tile_keys), whose
         // raster numbers follow key_skip others in each stream.
         c.order = nullptr;
         key_skip = is_pt ? 0 : 4 + (p->rr_depth != -1 && p->rr_depth <= 1 ? 1 : 0);
-        const uint64_t bvh_bytes = uint64_t(ctx->nodes.count) * sizeof(Node4) + uint64_t(ctx->tris.count) * sizeof(TriRecord);
+        const uint64_t bvh_bytes = uint64_t(ctx->nodes.count) * sizeof(NodeQ) + uint64_t(ctx->leaf_tris.count) * sizeof(LeafTri);
         if (bvh_bytes >= kOrderMinBvhBytes) {
             const uint32_t tiles = uint32_t(std::max((ctx->cam.width + 7) / 8, (ctx->cam.height + 7) / 8));
             key_bits = 2;
@@ -1623,7 +1620,7 @@ struct Pipeline {
         const dim3 grid_t(std::min<uint32_t>(grid_c.x, trace_grid));
         // Brute-force traversal grids: 16 blocks of kTraceBlock per CU, walking the queue.
         const dim3 grid_r(std::min<uint32_t>((cap + kTraceBlock - 1) / kTraceBlock, 16u * uint32_t(std::max(ctx->num_cus, 1))));
-        const uint32_t ntris = uint32_t(ctx->tris.count);
+        const uint32_t ntris = ctx->num_records;
         // Shade grids: 16 blocks per CU; the gradient pass 4, each flushing its gradient table once.
         const dim3 grid_s(std::min<uint32_t>(grid_c.x, (kMode == kAdjGrad ? 4u : 16u) * uint32_t(std::max(ctx->num_cus, 1))));
         hipError_t sort_e = hipSuccess;
@@ -1711,10 +1708,10 @@ struct Pipeline {
             if (!brute) {
                 e = timed(ctx, kKExtend, [&]() {
                     if (counting)
-                        hipLaunchKernelGGL(k_extend<true>, grid_t, dim3(kTraceBlock), 0, s, c.nodes, c.tris, qi,
+                        hipLaunchKernelGGL(k_extend<true>, grid_t, dim3(kTraceBlock), 0, s, c.bvh, qi,
                                            b.counters + k, b.counters + 2 * kMaxSegments + k, b.hits, ext_counts);
                     else
-                        hipLaunchKernelGGL(k_extend<false>, grid_t, dim3(kTraceBlock), 0, s, c.nodes, c.tris, qi,
+                        hipLaunchKernelGGL(k_extend<false>, grid_t, dim3(kTraceBlock), 0, s, c.bvh, qi,
                                            b.counters + k, b.counters + 2 * kMaxSegments + k, b.hits, ext_counts);
                 });
                 if (e != hipSuccess) return hip_fail(ctx, e, "k_extend");
@@ -1767,8 +1764,7 @@ lmgpu_status run_raycast(lmgpu_ctx* ctx, lmgpu_film* film) {
         out_dev = ctx->film_out_staging;
     }
     PTConsts c{};
-    c.nodes = ctx->nodes.ptr;
-    c.tris = ctx->tris.ptr;
+    c.bvh = bvh_of(ctx);
     c.shade = ctx->shade.ptr;
     c.mats = ctx->mats.ptr;
     c.lights = ctx->lights.ptr;

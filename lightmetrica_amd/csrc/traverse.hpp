@@ -1,28 +1,33 @@
 // Closest-hit and any-hit traversal of the 4-wide BVH (bvh_build.h) on gfx950.
 //
 // Replaces QBVHScene::IntersectTriangles (src/liblightmetrica/scene.qbvh.cpp:837-960):
-//   * one ray per lane, 64-lane wavefronts;
-//   * the node (6 SoA box planes x 4 children + 4 child words) is fetched as seven
-//     16-byte loads from one 128-byte line, each lane taking per axis the plane it enters
-//     first and the plane it leaves last (byte offsets from its direction signs);
-//   * each block keeps the root and its inner children in LDS: a ray's first one or two
-//     node visits happen when it starts, in the refill step, from that copy;
-//   * leaves are tested one triangle per step, a lane moving on to its next leaf as soon
-//     as it finishes one;
+//   * one ray per lane, 64-lane wavefronts; every step of a wave is either one node visit or
+//     one leaf step (two triangles), whichever more of its lanes wait for, so that a step
+//     runs with 26 to 43 lanes instead of the 14 of separate node and leaf loops;
+//   * a node is 64 bytes (NodeQ: 8-bit planes of four children), fetched as four 16-byte
+//     loads; a leaf of two or more triangles starts on a 128-byte line (LeafTri, two a line)
+//     and its triangles are fetched two at a time: what bounds a large batch is the lines
+//     fetched beyond L1 and L2;
 //   * children hit by the ray are sorted by entry distance; the nearest is descended
 //     into and the others are pushed, farthest first (closest and any hit);
 //   * the traversal stack lives in LDS, [level][lane] so the 64 lanes of a wave hit
-//     distinct banks, and spills to per-lane private memory beyond kStackLDS levels;
+//     distinct banks, and spills to per-lane private memory beyond StackLevels::kLds levels;
 //     closest-hit entries carry their box's entry distance, and pops skip the boxes that
 //     lie beyond the nearest hit found since they were pushed;
 //   * boxes are tested with the reciprocal-direction slab test in fused form, one FMA
-//     per plane (plane * inv + offset); the per-ray offsets -o * inv are widened by the
-//     rounding that form adds, and the exit distance is scaled by 1 + 2*gamma(4), so
-//     rounding never culls a box the ray touches (Ize, "Robust BVH Ray Traversal",
-//     JCGT 2013, with the absolute error of the fused form and the 1-ulp hardware
-//     reciprocal accounted for);
+//     per plane (step * (scale * inv) + (origin * inv + offset)); the per-ray offsets -o * inv
+//     are widened by the rounding that form adds, packed planes are moved out by more than
+//     theirs, and the exit distance is scaled by 1 + 2*gamma(6), so rounding never culls a
+//     box the ray touches (Ize, "Robust BVH Ray Traversal", JCGT 2013, with the absolute
+//     error of the fused form and the 1-ulp hardware reciprocal accounted for);
 //   * triangles use the watertight test of Woop, Benthin and Wald (JCGT 2013), with
 //     the FP64 fallback for edge functions that evaluate to exactly zero.
+// Measured on 16M incoherent rays against 1M triangles (closest hit with the FP64 pass):
+// 3.98 ms with separate node and leaf loops over 128-byte nodes and unaligned leaves, 3.06 ms
+// so; 4M any-hit segments 1.75 -> 1.31 ms; the extension rays of a 96k-triangle room (8.4M
+// paths, 8 segments, twice) 15.2 -> 12.0 ms, of which 0.4 ms buys the built boxes' order and
+// ends (LeafTri::box_yz, trace_exact).  With 128-byte nodes in the same loop: 3.35, 1.65 and
+// 13.8 ms.
 // Acceptance follows the reference's QBVH: t strictly inside (tmin, tmax), the first
 // triangle found wins an exact tie (scene.qbvh.cpp:124-133).
 #pragma once
@@ -33,9 +38,7 @@
 namespace lmgpu {
 
 constexpr int kTraceBlock = 256;
-constexpr int kStackLDS = 16;
-constexpr int kStackPriv = 80;
-constexpr int kStackTotal = kStackLDS + kStackPriv;  // supports 4-wide trees of depth <= 32
+constexpr int kStackTotal = 96;  // supports 4-wide trees of depth <= 32
 
 struct RayIn {
     float ox, oy, oz, dx, dy, dz, tmin, tmax;
@@ -46,6 +49,7 @@ struct HitOut {
     uint32_t rec;  // leaf-order triangle record of the winner
     uint32_t prim; // scene-order triangle index, 0xffffffff = miss
     float b0, b1;  // FP32 barycentric weights of v1 and v2 (closest hit)
+    float det;     // what b0 and b1 still have to be divided by (hit_weights)
 };
 
 struct TraceCounters {
@@ -90,20 +94,50 @@ __device__ __forceinline__ bool watertight_tail(float ax, float ay, float bx, fl
                                                 float zb, float zc, float tmin, float tmax, float& t, float& U,
                                                 float& V, float& W, float& det);
 
-// Watertight ray/triangle test.  Returns true with t strictly inside (tmin, tmax);
+// The shear of the BVH traversal, whose vertices differ from lane to lane: the axes are
+// permuted cyclically (kz the largest direction component) and two selects per component
+// apply the permutation.  make_shear also swaps kx and ky when the ray points down kz; the
+// swap negates U, V, W and det exactly and leaves t and the barycentric weights as they are,
+// so it is left out here.
+struct ShearCyclic {
+    uint32_t kz;
+    float Sx, Sy, Sz;
+    float ox, oy, oz;  // origin permuted into (kx, ky, kz)
+};
+
+__device__ __forceinline__ void permute(uint32_t kz, float x, float y, float z, float& px, float& py, float& pz) {
+    const bool k2 = kz == 2u, k1 = kz == 1u;
+    px = k2 ? x : (k1 ? z : y);
+    py = k2 ? y : (k1 ? x : z);
+    pz = k2 ? z : (k1 ? y : x);
+}
+
+__device__ __forceinline__ ShearCyclic make_shear_cyclic(const RayIn& r) {
+    ShearCyclic s;
+    const float ax = fabsf(r.dx), ay = fabsf(r.dy), az = fabsf(r.dz);
+    s.kz = (ax > ay) ? (ax > az ? 0u : 2u) : (ay > az ? 1u : 2u);
+    float dx, dy, dz;
+    permute(s.kz, r.dx, r.dy, r.dz, dx, dy, dz);
+    permute(s.kz, r.ox, r.oy, r.oz, s.ox, s.oy, s.oz);
+    s.Sz = __builtin_amdgcn_rcpf(dz);
+    s.Sx = dx * s.Sz;
+    s.Sy = dy * s.Sz;
+    return s;
+}
+
+// Watertight ray/triangle test.  Returns true with t in (tmin, tmax] (a hit has t < tmax: the
+// caller sees a tie with the hit it has);
 // U, V, W are the scaled barycentric weights of v0, v1, v2 and det = U + V + W.
-__device__ __forceinline__ bool watertight(const Shear& s, float4 v0, float4 v1, float4 v2, float tmin, float tmax,
-                                           float& t, float& U, float& V, float& W, float& det) {
+__device__ __forceinline__ bool watertight(const ShearCyclic& s, float4 v0, float4 v1, float4 v2, float tmin,
+                                           float tmax, float& t, float& U, float& V, float& W, float& det) {
 #pragma clang fp contract(off)
-    const float Ax = pick3(v0.x, v0.y, v0.z, s.kx) - s.ox;
-    const float Ay = pick3(v0.x, v0.y, v0.z, s.ky) - s.oy;
-    const float Az = pick3(v0.x, v0.y, v0.z, s.kz) - s.oz;
-    const float Bx = pick3(v1.x, v1.y, v1.z, s.kx) - s.ox;
-    const float By = pick3(v1.x, v1.y, v1.z, s.ky) - s.oy;
-    const float Bz = pick3(v1.x, v1.y, v1.z, s.kz) - s.oz;
-    const float Cx = pick3(v2.x, v2.y, v2.z, s.kx) - s.ox;
-    const float Cy = pick3(v2.x, v2.y, v2.z, s.ky) - s.oy;
-    const float Cz = pick3(v2.x, v2.y, v2.z, s.kz) - s.oz;
+    float Ax, Ay, Az, Bx, By, Bz, Cx, Cy, Cz;
+    permute(s.kz, v0.x, v0.y, v0.z, Ax, Ay, Az);
+    permute(s.kz, v1.x, v1.y, v1.z, Bx, By, Bz);
+    permute(s.kz, v2.x, v2.y, v2.z, Cx, Cy, Cz);
+    Ax -= s.ox; Ay -= s.oy; Az -= s.oz;
+    Bx -= s.ox; By -= s.oy; Bz -= s.oz;
+    Cx -= s.ox; Cy -= s.oy; Cz -= s.oz;
     const float ax = Ax - s.Sx * Az, ay = Ay - s.Sy * Az;
     const float bx = Bx - s.Sx * Bz, by = By - s.Sy * Bz;
     const float cx = Cx - s.Sx * Cz, cy = Cy - s.Sy * Cz;
@@ -157,18 +191,18 @@ __device__ __forceinline__ bool watertight_tail(float ax, float ay, float bx, fl
     U = cx * by - cy * bx;
     V = ax * cy - ay * cx;
     W = bx * ay - by * ax;
-    if (U == 0.f || V == 0.f || W == 0.f) {
+    if (fminf(fminf(fabsf(U), fabsf(V)), fabsf(W)) == 0.f) {
         // Exact products in FP64 decide the sign on the edge (Woop et al., section 3.3).
         U = float(double(cx) * double(by) - double(cy) * double(bx));
         V = float(double(ax) * double(cy) - double(ay) * double(cx));
         W = float(double(bx) * double(ay) - double(by) * double(ax));
     }
-    if ((U < 0.f || V < 0.f || W < 0.f) && (U > 0.f || V > 0.f || W > 0.f)) return false;
+    if (fminf(fminf(U, V), W) < 0.f && fmaxf(fmaxf(U, V), W) > 0.f) return false;
     det = U + V + W;
     if (det == 0.f) return false;
     const float T = U * za + V * zb + W * zc;
     t = T * __builtin_amdgcn_rcpf(det);  // within 3 ulp of T / det
-    return t > tmin && t < tmax;
+    return t > tmin && t <= tmax;
 }
 
 // The winner re-evaluated in FP64 (Moeller-Trumbore form): t and the weights of v1, v2.  Reads
@@ -195,9 +229,12 @@ __device__ __forceinline__ bool refine_fp64(const RayIn& r, float4 v0, float4 v1
     return true;
 }
 
-// 1 + 2 gamma(4), gamma(n) = n u / (1 - n u), u = 2^-24: the fused plane distance rounds once,
-// the hardware reciprocal is within 1 ulp (2u), and the threshold product rounds once.
-constexpr float kBoxRobust = 1.0f + 2.0f * 2.4e-7f;
+// 1 + 2 gamma(6), gamma(n) = n u / (1 - n u), u = 2^-24: the hardware reciprocal is within 1 ulp
+// (2u), the node's offset fma(origin, inv, offset) and the plane distance round once each, and
+// so does the threshold product.
+constexpr float kBoxRobust = 1.0f + 2.0f * 3.6e-7f;
+// The same for a box whose planes are at hand: 1 + 2 gamma(4).
+constexpr float kBoxRobustExact = 1.0f + 2.0f * 2.4e-7f;
 
 // Hardware reciprocal (v_rcp_f32, within 1 ulp) of a direction component kept away from 0.
 __device__ __forceinline__ float safe_rcp(float d) {
@@ -212,22 +249,19 @@ __device__ __forceinline__ float safe_rcp(float d) {
 // earlier by e and the plane that is left last later by e leaves the entry and exit distances
 // with relative errors only, which kBoxRobust covers.  Coordinates are assumed below 1e8 in
 // magnitude so that o * inv stays finite for the clamped reciprocal (<= 1e30).
-// Per axis the ray knows which plane it enters first (lo when inv >= 0): `b` is the byte
-// offset (0 or 16) of that plane's four coordinates within the node's lo/hi pair, so each
-// lane fetches its near and far planes directly and needs no min / max to order them.
+// Per axis the ray knows which plane it enters first (lo when inv >= 0), so a select per axis
+// and node takes the near and far planes of all four children and no min / max orders them.
 struct Slab {
     float ix, iy, iz;
     float nx, fx, ny, fy, nz, fz;  // offsets of the near and far planes per axis
-    uint32_t bx, by, bz;           // byte offset of the near plane in the axis's lo/hi pair
 };
 
-__device__ __forceinline__ void slab_axis(float o, float inv, float& near_off, float& far_off, uint32_t& b) {
+__device__ __forceinline__ void slab_axis(float o, float inv, float& near_off, float& far_off) {
     const float e = fabsf(o * inv) * 2.384185791015625e-7f;  // 2^-22 |p|
     const float lo = fmaf(-o, inv, inv >= 0.f ? -e : e);       // lo plane, moved away from the box's inside
     const float hi = fmaf(-o, inv, inv >= 0.f ? e : -e);
     near_off = inv >= 0.f ? lo : hi;
     far_off = inv >= 0.f ? hi : lo;
-    b = inv >= 0.f ? 0u : 16u;
 }
 
 __device__ __forceinline__ Slab make_slab(const RayIn& r) {
@@ -235,10 +269,230 @@ __device__ __forceinline__ Slab make_slab(const RayIn& r) {
     s.ix = safe_rcp(r.dx);
     s.iy = safe_rcp(r.dy);
     s.iz = safe_rcp(r.dz);
-    slab_axis(r.ox, s.ix, s.nx, s.fx, s.bx);
-    slab_axis(r.oy, s.iy, s.ny, s.fy, s.by);
-    slab_axis(r.oz, s.iz, s.nz, s.fz, s.bz);
+    slab_axis(r.ox, s.ix, s.nx, s.fx);
+    slab_axis(r.oy, s.iy, s.ny, s.fy);
+    slab_axis(r.oz, s.iz, s.nz, s.fz);
     return s;
+}
+
+// Orders two (key, reference) pairs, nearer first.  A pair is one 64-bit value, the key in the
+// upper half: read as doubles such values order by key (floats order like the upper halves of
+// doubles, and the lower half only decides between equal keys), so the exchange is one
+// minimum and one maximum instead of a compare and four selects.
+__device__ __forceinline__ void cswap(double& a, double& b) {
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
+}
+
+__device__ __forceinline__ double pack_entry(float key, uint32_t ref) {
+    return __hiloint2double(int(__float_as_uint(key)), int(ref));
+}
+__device__ __forceinline__ uint32_t entry_ref(double e) { return uint32_t(__double2loint(e)); }
+__device__ __forceinline__ float entry_key(double e) { return __uint_as_float(uint32_t(__double2hiint(e))); }
+
+constexpr uint32_t kDone = 0xffffffffu;  // nothing left to visit
+constexpr uint32_t kPop = 0xfffffffeu;   // the next reference is on the stack (no leaf of 16 records starts at 2^27 - 2)
+__device__ __forceinline__ bool is_inner(uint32_t ref) { return int(ref) >= 0; }
+__device__ __forceinline__ bool is_leaf(uint32_t ref) { return ref >= kLeafBit && ref < kPop; }
+
+// A node of the built tree in the form the kernels read.  Along each axis the children's planes
+// are 8-bit steps of ext / 254.9 from the lowest plane, lo planes rounded down and hi planes up
+// and moved out by at least kPlaneMargin steps more, which exceeds what evaluating
+// origin + q * scale along a ray can lose against the extent (3 roundings of 255 steps).
+// Step 0 is the lowest plane itself.  An empty slot's box is inverted (255, 0) and its child
+// word a one-record leaf: where rounding or NaN lets a ray in, the record's own test decides.
+constexpr double kPlaneMargin = 1.0 / 512;
+__device__ __forceinline__ NodeQ pack_node(const Node4& n) {
+    NodeQ q;
+    const float* lo[3] = {n.lo_x, n.lo_y, n.lo_z};
+    const float* hi[3] = {n.hi_x, n.hi_y, n.hi_z};
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        float l = INFINITY, h = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (n.child[i] == kEmptyChild) continue;
+            l = fminf(l, lo[a][i]);
+            h = fmaxf(h, hi[a][i]);
+        }
+        const double ext = double(h) - double(l);
+        const float step = ext > 0.0 ? fmaxf(float(ext * (1.0 / 254.9)), 1.17549435e-38f) : 0.f;
+        uint32_t ql = 0u, qh = 0u;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t b0 = 255u, b1 = 0u;
+            if (n.child[i] != kEmptyChild) {
+                b0 = 0u;
+                if (step > 0.f) {
+                    const double s0 = (double(lo[a][i]) - double(l)) / double(step) - kPlaneMargin;
+                    const double s1 = (double(hi[a][i]) - double(l)) / double(step) + kPlaneMargin;
+                    b0 = uint32_t(fmax(floor(s0), 0.0));
+                    b1 = uint32_t(fmin(ceil(s1), 255.0));
+                }
+            }
+            ql |= b0 << (8 * i);
+            qh |= b1 << (8 * i);
+        }
+        q.origin[a] = l;
+        q.step[a] = step;
+        q.planes[a][0] = ql;
+        q.planes[a][1] = qh;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) q.child[i] = n.child[i] == kEmptyChild ? kLeafBit : n.child[i];
+    return q;
+}
+
+// Node words are fetched through a buffer resource over the node array: the
+// constant part of each fetch's offset goes into the instruction's offset field, so a fetch
+// costs one 32-bit address add (a global load needs 64-bit address arithmetic to fold it),
+// and the 64-bit temporaries' registers are freed.  The resource's record count, 2^32 - 1
+// bytes, lets every fetch of a tree within kMaxNodes nodes through (the last node's words
+// end 16 bytes before 2^32).
+struct NodeFetch {
+    __amdgpu_buffer_rsrc_t rsrc;
+    __device__ __forceinline__ explicit NodeFetch(const NodeQ* nodes)
+        // word 3 of a gfx9 raw buffer resource: 32-bit data format, no swizzle, no stride.
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<NodeQ*>(nodes), short(0), -1, 0x00020000)) {}
+    __device__ __forceinline__ float4 operator()(uint32_t off) const {
+        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+    }
+};
+
+// Slab tests of the four children of node `cur` (Node4 words read by `fetch`), sorted into
+// entries (key = entry distance, reference), nearest first; a missed child's key is +inf.  Each
+// lane fetches the plane it enters first and the plane it leaves last per axis (byte offsets
+// from the ray's direction signs), so the entry and exit distances need no min / max per axis;
+// for a non-empty box they equal what ordering the two planes would give (fma rounds
+// monotonically), and the inverted box of an empty slot is never entered.
+__device__ __forceinline__ void node_children(const NodeFetch& fetch, uint32_t cur, const Slab& s, float tmin, float tmax,
+                                              double e[4]) {
+    // 32-bit byte offsets from the node array (at most kMaxNodes nodes, checked by the builder).
+    const uint32_t o = cur * uint32_t(sizeof(NodeQ));
+    const float4 q0 = fetch(o), q1 = fetch(o + 16u), q2 = fetch(o + 32u), q3 = fetch(o + 48u);
+    // The planes are origin + q * scale: along the ray fma(q, scale * inv, fma(origin, inv, offset)).
+    const float ax = q0.w * s.ix, ay = q1.x * s.iy, az = q1.y * s.iz;
+    const float bnx = fmaf(q0.x, s.ix, s.nx), bfx = fmaf(q0.x, s.ix, s.fx);
+    const float bny = fmaf(q0.y, s.iy, s.ny), bfy = fmaf(q0.y, s.iy, s.fy);
+    const float bnz = fmaf(q0.z, s.iz, s.nz), bfz = fmaf(q0.z, s.iz, s.fz);
+    const uint32_t lx = __float_as_uint(q1.z), hx = __float_as_uint(q1.w);
+    const uint32_t ly = __float_as_uint(q2.x), hy = __float_as_uint(q2.y);
+    const uint32_t lz = __float_as_uint(q2.z), hz = __float_as_uint(q2.w);
+    const uint32_t nx = s.ix >= 0.f ? lx : hx, fx = s.ix >= 0.f ? hx : lx;
+    const uint32_t ny = s.iy >= 0.f ? ly : hy, fy = s.iy >= 0.f ? hy : ly;
+    const uint32_t nz = s.iz >= 0.f ? lz : hz, fz = s.iz >= 0.f ? hz : lz;
+    const float c[4] = {q3.x, q3.y, q3.z, q3.w};
+    auto plane = [](uint32_t q, int i) { return float((q >> (8 * i)) & 0xffu); };
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float tn = fmaxf(fmaxf(fmaf(plane(nx, i), ax, bnx), fmaf(plane(ny, i), ay, bny)),
+                               fmaxf(fmaf(plane(nz, i), az, bnz), tmin));
+        const float tf = fminf(fminf(fmaf(plane(fx, i), ax, bfx), fmaf(plane(fy, i), ay, bfy)),
+                               fminf(fmaf(plane(fz, i), az, bfz), tmax));
+        e[i] = pack_entry(tn <= tf * kBoxRobust ? tn : INFINITY, __float_as_uint(c[i]));
+    }
+    cswap(e[0], e[1]);
+    cswap(e[2], e[3]);
+    cswap(e[0], e[2]);
+    cswap(e[1], e[3]);
+    cswap(e[1], e[2]);
+}
+
+// Records an accepted triangle in h; closest hit also keeps the watertight test's scaled weights
+// V and W of v1 and v2 and their sum det, so the winner is never fetched again: hit_weights
+// turns them into barycentric weights once the ray is done.
+template <bool kAny>
+__device__ __forceinline__ void accept_hit(HitOut& h, float t, uint32_t rec, uint32_t prim, float V, float W,
+                                           float det) {
+    h.t = t;
+    h.rec = rec;
+    h.prim = prim;
+    if (!kAny) {
+        h.b0 = V;
+        h.b1 = W;
+        h.det = det;
+    }
+}
+__device__ __forceinline__ void hit_weights(HitOut& h) {
+    const float inv = 1.f / h.det;
+    h.b0 *= inv;
+    h.b1 *= inv;
+}
+
+// The LDS of one traversal block: the stacks' LDS levels ([level][thread]), for closest hit
+// with the entry distance in an entry's upper half.
+template <bool kKeys> struct StackLevels;
+template <> struct StackLevels<true> {
+    using Entry = double;
+    static constexpr uint32_t kLds = 12;
+};
+template <> struct StackLevels<false> {
+    using Entry = uint32_t;
+    static constexpr uint32_t kLds = 16;
+};
+template <bool kKeys> struct TraceShared {
+    typename StackLevels<kKeys>::Entry stack[StackLevels<kKeys>::kLds * kTraceBlock];
+};
+
+// The per-lane traversal stack: the first levels live in LDS (`lds` is this lane's column,
+// lds[level * kTraceBlock]), deeper ones in private memory.  The builder bounds
+// 3 * depth <= kStackTotal, so the guard in push never fires.
+// With kKeys (closest hit) every entry carries the entry distance of its box, and pop skips
+// entries whose distance exceeds the current tmax * kBoxRobust: the box test would reject
+// them now that a nearer hit shrank tmax, so they are never fetched.
+// The spill array is owned by the caller (a separate private array, so the stack pointer and
+// the LDS columns stay in registers).
+template <bool kKeys> struct TraceStack {
+    using Entry = typename StackLevels<kKeys>::Entry;
+    static constexpr uint32_t kLds = StackLevels<kKeys>::kLds;
+    // Spelled with its address space: from two generic pointers the compiler made one flat access
+    // of each push and pop, which goes through the vector memory path.
+    __attribute__((address_space(3))) Entry* lds;
+    Entry* spill;
+    uint32_t sp = 0;
+
+    static __device__ __forceinline__ Entry entry(double e) {
+        if constexpr (kKeys) return e;
+        else return entry_ref(e);
+    }
+    __device__ __forceinline__ void push(double e) {
+        if (sp < kLds) lds[sp * kTraceBlock] = entry(e);
+        else if (sp < uint32_t(kStackTotal)) spill[sp - kLds] = entry(e);
+        else return;
+        sp++;
+    }
+    // Pushes the hit ones of the sorted entries e[3], e[2], e[1], in that order.
+    __device__ __forceinline__ void push_sorted(const double e[4]) {
+        if (sp + 3u <= kLds) {
+#pragma unroll
+            for (int i = 3; i > 0; i--)
+                if (entry_key(e[i]) < INFINITY) lds[sp++ * kTraceBlock] = entry(e[i]);
+        } else {
+            for (int i = 3; i > 0; i--)
+                if (entry_key(e[i]) < INFINITY) push(e[i]);
+        }
+    }
+    // Takes the top entry: its reference, kPop when the entry is skipped, kDone when there is none.
+    __device__ __forceinline__ uint32_t pop(float tmax) {
+        if (sp == 0u) return kDone;
+        sp--;
+        Entry e;
+        if (sp < kLds) e = lds[sp * kTraceBlock];
+        else e = spill[sp - kLds];
+        if constexpr (kKeys) return entry_key(e) > fmaxf(tmax * kBoxRobust, 0.f) ? kPop : entry_ref(e);
+        else return e;
+    }
+};
+
+// Descends from a node: pushes the farther hit children (the keys matter for closest hit
+// only) and returns the nearest, or kPop when none is hit.
+// Any hit descends nearest first too: it finds an occluder sooner (any-hit batch -1.7 %).
+template <class Stack> __device__ __forceinline__ uint32_t descend(const double e[4], Stack& st) {
+    st.push_sorted(e);
+    return entry_key(e[0]) < INFINITY ? entry_ref(e[0]) : kPop;
 }
 
 __device__ __forceinline__ void cswap(float& ka, uint32_t& va, float& kb, uint32_t& vb) {
@@ -251,273 +505,161 @@ __device__ __forceinline__ void cswap(float& ka, uint32_t& va, float& kb, uint32
     va = tv;
 }
 
-constexpr uint32_t kDone = 0xffffffffu;
-
-// Node words in LDS (the root and its inner children).
-struct NodeFetchLds {
-    const char* p;
-    __device__ __forceinline__ float4 operator()(uint32_t off) const { return *reinterpret_cast<const float4*>(p + off); }
-};
-
-// Node words in global memory, fetched through a buffer resource over the node array: the
-// constant part of each fetch's offset goes into the instruction's offset field, so a fetch
-// costs one 32-bit address add (a global load needs 64-bit address arithmetic to fold it),
-// and the 64-bit temporaries' registers are freed.  The resource's record count, 2^32 - 1
-// bytes, lets every fetch of a tree within kMaxNodes nodes through (the last node's words
-// end 16 bytes before 2^32).
-struct NodeFetchGlobal {
-    __amdgpu_buffer_rsrc_t rsrc;
-    __device__ __forceinline__ explicit NodeFetchGlobal(const Node4* nodes)
-        // word 3 of a gfx9 raw buffer resource: 32-bit data format, no swizzle, no stride.
-        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<Node4*>(nodes), short(0), -1, 0x00020000)) {}
-    __device__ __forceinline__ float4 operator()(uint32_t off) const {
-        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
-    }
-};
-
-// Slab tests of the four children of node `cur` (Node4 words read by `fetch`).  Returns how many
-// the ray enters within [tmin, tmax], the hit children first in (key, val), nearest first
-// (a missed child's key is +inf).  Each lane fetches the plane it enters first and the plane it leaves last
-// per axis (byte offsets from the ray's direction signs), so the entry and exit distances need
-// no min / max per axis; for a non-empty box they equal what ordering the two planes would
-// give (fma rounds monotonically), and an empty child is rejected by its reference.
-template <class Fetch>
-__device__ __forceinline__ int node_children(const Fetch& fetch, uint32_t cur, const Slab& s, float tmin, float tmax,
-                                             float key[4], uint32_t val[4]) {
-    // 32-bit byte offsets from the node array (at most kMaxNodes nodes, checked by the builder).
-    const uint32_t o = cur << 7;
-    const float4 nxv = fetch(o + s.bx);
-    const float4 fxv = fetch(o + (16u - s.bx));
-    const float4 nyv = fetch(o + (32u + s.by));
-    const float4 fyv = fetch(o + (48u - s.by));
-    const float4 nzv = fetch(o + (64u + s.bz));
-    const float4 fzv = fetch(o + (80u - s.bz));
-    const float4 chf = fetch(o + 96u);
-    const uint4 ch = make_uint4(__float_as_uint(chf.x), __float_as_uint(chf.y), __float_as_uint(chf.z),
-                                __float_as_uint(chf.w));
-    const float nx[4] = {nxv.x, nxv.y, nxv.z, nxv.w}, fx[4] = {fxv.x, fxv.y, fxv.z, fxv.w};
-    const float ny[4] = {nyv.x, nyv.y, nyv.z, nyv.w}, fy[4] = {fyv.x, fyv.y, fyv.z, fyv.w};
-    const float nz[4] = {nzv.x, nzv.y, nzv.z, nzv.w}, fz[4] = {fzv.x, fzv.y, fzv.z, fzv.w};
-    const uint32_t c[4] = {ch.x, ch.y, ch.z, ch.w};
-    int nhit = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float tn = fmaxf(fmaxf(fmaf(nx[i], s.ix, s.nx), fmaf(ny[i], s.iy, s.ny)),
-                               fmaxf(fmaf(nz[i], s.iz, s.nz), tmin));
-        const float tf = fminf(fminf(fmaf(fx[i], s.ix, s.fx), fmaf(fy[i], s.iy, s.fy)),
-                               fminf(fmaf(fz[i], s.iz, s.fz), tmax));
-        const bool hit = c[i] != kEmptyChild && tn <= tf * kBoxRobust;
-        key[i] = hit ? tn : INFINITY;
-        val[i] = c[i];
-        nhit += hit ? 1 : 0;
-    }
-    cswap(key[0], val[0], key[1], val[1]);
-    cswap(key[2], val[2], key[3], val[3]);
-    cswap(key[0], val[0], key[2], val[2]);
-    cswap(key[1], val[1], key[3], val[3]);
-    cswap(key[1], val[1], key[2], val[2]);
-    return nhit;
-}
-
-// Records an accepted triangle in h; closest hit also keeps the watertight test's barycentric
-// weights of v1 and v2 (V / det, W / det), so the winner is never fetched again.
-template <bool kAny>
-__device__ __forceinline__ void accept_hit(HitOut& h, float t, uint32_t rec, uint32_t prim, float V, float W,
-                                           float det) {
-    h.t = t;
-    h.rec = rec;
-    h.prim = prim;
-    if (!kAny) {
-        const float inv = 1.f / det;
-        h.b0 = V * inv;
-        h.b1 = W * inv;
-    }
-}
-
-// The LDS of one traversal block: the stacks' LDS levels ([level][thread]) and, for closest
-// hit, their keys.
-template <bool kKeys>
-struct TraceShared {
-    uint32_t ref[kStackLDS * kTraceBlock];
-    uint16_t key[kKeys ? kStackLDS * kTraceBlock : 1];
-    // The root node's words, then those of its inner children by child slot: every ray's
-    // first one or two node visits read them here.
-    float4 top[5 * 8];
-};
-
-// Entry-distance keys of closest-hit stack entries in LDS: the upper 16 bits of the float,
-// i.e. the distance rounded toward zero, so a key never exceeds the distance it stands for;
-// distances <= 0 are kept as -inf.
-__device__ __forceinline__ uint16_t key_down16(float t) {
-    return t > 0.f ? uint16_t(__float_as_uint(t) >> 16) : uint16_t(0xff80u);
-}
-__device__ __forceinline__ float key_up(uint16_t k) { return __uint_as_float(uint32_t(k) << 16); }
-
-// The per-lane traversal stack: levels [0, kStackLDS) live in LDS (`ref` and `key` are this
-// lane's columns of the block's __shared__ arrays, ref[level * kTraceBlock]), deeper levels in
-// private memory as 64-bit slots (reference, and the full float key in the upper half).  The
-// builder bounds 3 * depth <= kStackTotal, so the guard in push never fires.
-// With kKeys (closest hit) every entry carries the entry distance of its box, and pop skips
-// entries whose distance exceeds the current tmax * kBoxRobust: the box test would reject
-// them now that a nearer hit shrank tmax, so they are never fetched.
-// The spill array is owned by the caller (a separate private array, so the stack pointer and
-// the LDS columns stay in registers).
-template <bool kKeys>
-struct TraceStack {
-    uint32_t* ref;
-    uint16_t* key;
-    uint64_t* spill;
-    int sp = 0;
-
-    __device__ __forceinline__ void push(uint32_t v, float k) {
-        if (sp < kStackLDS) {
-            ref[sp * kTraceBlock] = v;
-            if (kKeys) key[sp * kTraceBlock] = key_down16(k);
-        } else if (sp < kStackTotal) {
-            spill[sp - kStackLDS] = kKeys ? uint64_t(v) | (uint64_t(__float_as_uint(k)) << 32) : uint64_t(v);
-        } else {
-            return;
-        }
-        sp++;
-    }
-    // The next entry to visit, or kDone when the stack is empty.
-    __device__ __forceinline__ uint32_t pop(float tmax) {
-        while (sp > 0) {
-            sp--;
-            uint32_t v;
-            float k;
-            if (sp < kStackLDS) {
-                v = ref[sp * kTraceBlock];
-                k = kKeys ? key_up(key[sp * kTraceBlock]) : -INFINITY;
-            } else {
-                const uint64_t e = spill[sp - kStackLDS];
-                v = uint32_t(e);
-                k = __uint_as_float(uint32_t(e >> 32));
-            }
-            if (!kKeys || !(k > tmax * kBoxRobust)) return v;
-        }
-        return kDone;
-    }
-    // Pushes v3 (n > 3), v2 (n > 2), v1 (n > 1) in that order, with their keys.  While three
-    // LDS levels are free it stores three slots without branches and raises sp by n - 1;
-    // slots above the new top are free levels of this lane.
-    __device__ __forceinline__ void push_sorted(int n, uint32_t v1, uint32_t v2, uint32_t v3, float k1, float k2,
-                                                float k3) {
-        if (sp + 3 <= kStackLDS) {
-            ref[sp * kTraceBlock] = n > 3 ? v3 : (n > 2 ? v2 : v1);
-            ref[(sp + 1) * kTraceBlock] = n > 3 ? v2 : v1;
-            ref[(sp + 2) * kTraceBlock] = v1;
-            if (kKeys) {
-                key[sp * kTraceBlock] = key_down16(n > 3 ? k3 : (n > 2 ? k2 : k1));
-                key[(sp + 1) * kTraceBlock] = key_down16(n > 3 ? k2 : k1);
-                key[(sp + 2) * kTraceBlock] = key_down16(k1);
-            }
-            sp += n - 1;
-        } else {
-            if (n > 3) push(v3, k3);
-            if (n > 2) push(v2, k2);
-            if (n > 1) push(v1, k1);
-        }
-    }
-};
-
-// Descends from the node on top: pushes the farther hit children (the keys matter for closest
-// hit only) and returns the nearest, or the next reference on the stack when none is hit.
-// Any hit descends nearest first too: it finds an occluder sooner (any-hit batch -1.7 %).
+// The packed boxes hold every hit, but the order in which a ray meets them is the built boxes' to
+// say: of two triangles at the same t the one found first wins.  A ray whose nearest hit is
+// such a tie (1 in 10^6 of a city's) is traced again here, one node or leaf after the other
+// in the order of the built boxes.
 template <class Stack>
-__device__ __forceinline__ uint32_t descend(int nhit, const float key[4], const uint32_t val[4], float tmax,
-                                            Stack& st) {
-    if (nhit == 0) return st.pop(tmax);
-    st.push_sorted(nhit, val[1], val[2], val[3], key[1], key[2], key[3]);
-    return val[0];
+__device__ __forceinline__ HitOut trace_exact(const BvhDev& bvh, const RayIn& r, Stack& st) {
+    const Slab s = make_slab(r);
+    const ShearCyclic sh = make_shear_cyclic(r);
+    HitOut h{r.tmax, 0u, 0xffffffffu, 0.f, 0.f, 1.f};
+    float tmax = r.tmax;
+    uint32_t cur = 0u;
+    st.sp = 0u;
+    while (cur != kDone) {
+        if (is_inner(cur)) {
+            const float4* n = reinterpret_cast<const float4*>(bvh.exact + cur);
+            const uint32_t x = s.ix >= 0.f ? 0u : 1u, y = s.iy >= 0.f ? 0u : 1u, z = s.iz >= 0.f ? 0u : 1u;
+            const float4 nxv = n[x], fxv = n[1u - x], nyv = n[2u + y], fyv = n[3u - y], nzv = n[4u + z], fzv = n[5u - z];
+            const float4 cv = n[6];
+            const float nx[4] = {nxv.x, nxv.y, nxv.z, nxv.w}, fx[4] = {fxv.x, fxv.y, fxv.z, fxv.w};
+            const float ny[4] = {nyv.x, nyv.y, nyv.z, nyv.w}, fy[4] = {fyv.x, fyv.y, fyv.z, fyv.w};
+            const float nz[4] = {nzv.x, nzv.y, nzv.z, nzv.w}, fz[4] = {fzv.x, fzv.y, fzv.z, fzv.w};
+            const float c[4] = {cv.x, cv.y, cv.z, cv.w};
+            float key[4];
+            uint32_t val[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float tn = fmaxf(fmaxf(fmaf(nx[i], s.ix, s.nx), fmaf(ny[i], s.iy, s.ny)),
+                                       fmaxf(fmaf(nz[i], s.iz, s.nz), r.tmin));
+                const float tf = fminf(fminf(fmaf(fx[i], s.ix, s.fx), fmaf(fy[i], s.iy, s.fy)),
+                                       fminf(fmaf(fz[i], s.iz, s.fz), tmax));
+                val[i] = __float_as_uint(c[i]);
+                key[i] = val[i] != kEmptyChild && tn <= tf * kBoxRobustExact ? tn : INFINITY;
+            }
+            cswap(key[0], val[0], key[1], val[1]);
+            cswap(key[2], val[2], key[3], val[3]);
+            cswap(key[0], val[0], key[2], val[2]);
+            cswap(key[1], val[1], key[3], val[3]);
+            cswap(key[1], val[1], key[2], val[2]);
+#pragma unroll
+            for (int i = 3; i > 0; i--)
+                if (key[i] < INFINITY) st.push(pack_entry(-INFINITY, val[i]));
+            cur = key[0] < INFINITY ? val[0] : st.pop(tmax);
+        } else {
+            const uint32_t first = cur & kMaxLeafFirst, end = first + ((cur >> 27) & 0xfu) + 1u;
+            for (uint32_t k = first; k < end; k++) {
+                const float4* tp = reinterpret_cast<const float4*>(bvh.tris + k);
+                const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
+                float t, U, V, W, det;
+                if (watertight(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det) && t < tmax) {
+                    tmax = t;
+                    accept_hit<false>(h, t, k, __float_as_uint(v0.w), V, W, det);
+                }
+            }
+            cur = st.pop(tmax);
+        }
+    }
+    return h;
 }
 
-// Lanes of a persistent traversal fetch new rays once this many lanes of the wave are idle:
-// kRefillIdle when every refill claims its rays with an atomic (the path tracer's queues),
-// kRefillIdleRanged when rays come from ranges claimed ahead of need (ray batches).
-constexpr int kRefillIdle = 40;
-constexpr int kRefillIdleRanged = 8;
+// A wave fetches new rays once this many of its lanes are idle: fetching costs the setup of the
+// rays' constants for the idle lanes only, waiting leaves lanes out of every step.  16M rays:
+// 12 idle lanes 3.65 ms, 20: 3.45, 28: 3.38; extension rays of the 96k-triangle room 11.6, 11.6, 11.8.
+constexpr uint32_t kRefillIdle = 20;
+// A wave takes a node step while at least this many times more lanes wait at nodes than hold a
+// leaf: a leaf step is shorter and frees its lanes to shrink tmax.  2 against 1: extension rays
+// 11.8 -> 11.5 ms, 1M-triangle city 2.65 -> 2.49 ms, 16M rays the same; 3: 11.8 ms.
+constexpr uint32_t kLeafWeight = 2;
 
 // Persistent traversal with per-lane ray refill (Aila & Laine, "Understanding the
 // efficiency of ray traversal on GPUs", HPG 2009): every wave of the grid loops over
 // the batch.  The first 64 rays of a wave are assigned statically (wave w takes
 // [64 w, 64 w + 64)); after that lanes whose rays have finished fetch the next unclaimed
-// rays from `next` (counting from 64 x the number of waves) once enough of the wave's lanes
-// are idle: without kRanged with one atomic per refill, at kRefillIdle idle lanes; with
-// kRanged from 64-ray ranges claimed one range ahead, at kRefillIdleRanged idle lanes.  A
-// batch smaller than the grid therefore costs no atomics.
-// Leaves are processed speculatively (same paper): a lane that reaches a leaf postpones it
-// and keeps descending until every lane still descending holds a leaf, so the inner-node
-// and triangle loops each run with as many lanes as possible.
+// rays once kRefillIdle of the wave's lanes are idle, from ranges claimed from `next` (which
+// counts from 64 x the number of waves) one range ahead of need, so that a refill waits for no
+// atomic.  A batch smaller than the grid costs no atomics.
+// A lane visits nodes until it meets a leaf, and goes on visiting nodes while the leaf's
+// triangles are still to be tested (speculative traversal, same paper); a second leaf stops
+// it.  Each step of the wave serves the larger of the two groups.  A lane whose node left
+// nothing to descend into takes one entry off its stack a step: a loop until every lane had
+// one ran 102 times per 64 rays with 4 lanes each.
 // `src(i)` returns ray i, `sink(i, found, h, r)` consumes its result.  Every wave exits
 // once the batch is exhausted and its own lanes are done.  With kCount, `cnt` sums the
 // lane's node visits and triangle tests over all rays it traced.
-template <bool kAny, bool kCount, bool kRanged, class Source, class Sink>
-__device__ __forceinline__ void trace_persistent(const Node4* __restrict__ nodes, const TriRecord* __restrict__ tris,
-                                                 uint32_t n, uint32_t* next, TraceShared<!kAny>& sm, Source& src,
+// n is at most kMaxBatch: a claim past the end then never wraps the counter.
+constexpr uint32_t kMaxBatch = 0x80000000u;
+template <bool kAny, bool kCount, class Source, class Sink>
+__device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, uint32_t* next, TraceShared<!kAny>& sm, Source& src,
                                                  Sink& sink, TraceCounters& cnt) {
-    uint64_t spill[kStackPriv];
-    TraceStack<!kAny> st{sm.ref + threadIdx.x, kAny ? nullptr : sm.key + threadIdx.x, spill};
+    typename TraceStack<!kAny>::Entry spill[kStackTotal - TraceStack<!kAny>::kLds];
+    TraceStack<!kAny> st{(__attribute__((address_space(3))) typename TraceStack<!kAny>::Entry*)(sm.stack + threadIdx.x), spill};
     constexpr uint32_t kNone = 0xffffffffu;
     const uint32_t lane = __lane_id();
     uint32_t id = kNone;
     RayIn r{0.f, 0.f, 0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
     float tmax = 0.f;
     Slab sl = make_slab(r);
-    Shear sh = make_shear(r);
-    HitOut h{0.f, 0u, kNone, 0.f, 0.f};
+    ShearCyclic sh = make_shear_cyclic(r);
+    HitOut h{0.f, 0u, kNone, 0.f, 0.f, 1.f};
     bool found = false;
+    bool tie = false;  // closest hit: another triangle at the nearest distance (trace_exact decides)
+    // Distances beyond doubt: farther than 2^-21 of the coordinates involved from the ends, where a
+    // distance is known to a few units of 2^-24 of them.
+    float sure_lo = 0.f, sure_hi = 0.f;
+    // Closed rays with a tie, kTies at most; a lane with a full list takes no further ray.
+    constexpr uint32_t kTies = 4;
+    uint32_t ties[kAny ? 1 : kTies];
+    uint32_t num_ties = 0u;
     uint32_t cur = kDone;   // next node or leaf reference to visit
-    uint32_t leaf = kDone;  // postponed leaf
-    // The root node and its inner children into the block's LDS: a new ray's first visits
-    // read them there, in the refill step, instead of as dependent fetches of the node loop.
-    const float4* nodes4 = reinterpret_cast<const float4*>(nodes);
-    if (threadIdx.x < 8u) {
-        sm.top[threadIdx.x] = nodes4[threadIdx.x];
-    } else if (threadIdx.x < 40u) {
-        const uint32_t slot = (threadIdx.x - 8u) >> 3;
-        const uint32_t c = reinterpret_cast<const uint32_t*>(nodes4 + 6)[slot];  // the root's child refs
-        if (c != kEmptyChild && !(c & kLeafBit)) sm.top[threadIdx.x] = nodes4[8u * c + (threadIdx.x & 7u)];
-    }
-    __syncthreads();
-    const char* top = reinterpret_cast<const char*>(sm.top);
-    const NodeFetchLds lfetch{top};
-    const NodeFetchGlobal gfetch(nodes);
+    uint32_t tri = 0u, tri_end = 0u;  // records left of the leaf being tested
+    const NodeFetch fetch(bvh.nodes);
+    // A leaf next in line becomes the one being tested if there is none.
+    auto take_leaf = [&]() {
+        if (is_leaf(cur) && tri >= tri_end) {
+            tri = cur & kMaxLeafFirst;
+            tri_end = tri + ((cur >> 27) & 0xfu) + 1u;
+            cur = kPop;
+        }
+    };
     auto start = [&](uint32_t k) {
         id = k;
         r = src(k);
         sl = make_slab(r);
-        sh = make_shear(r);
+        sh = make_shear_cyclic(r);
         tmax = r.tmax;
-        h.prim = kNone;
-        h.rec = 0;
-        h.t = tmax;
-        found = false;
-        leaf = kDone;
-        st.sp = 0;
-        float key[4];
-        uint32_t val[4];
-        // The root; then, if the next node is one of its inner children (every entry on the
-        // stack is), that child from its slot.
-        if (kCount) cnt.nodes++;
-        int nhit = node_children(lfetch, 0u, sl, r.tmin, tmax, key, val);
-        cur = descend(nhit, key, val, tmax, st);
-        if (cur != kDone && (cur & kLeafBit)) {
-            leaf = cur;
-            cur = st.pop(tmax);
+        found = tie = false;
+        const float band = 4.76837158203125e-7f * fabsf(sh.Sz) *
+                           (fmaxf(fmaxf(fabsf(r.ox), fabsf(r.oy)), fabsf(r.oz)) + bvh.reach);
+        sure_lo = r.tmin + band;
+        if (kAny) sure_hi = fmaf(r.tmax, 1.f - 1e-6f, -band);
+        tri = tri_end = 0u;
+        st.sp = 0u;
+        cur = 0u;
+    };
+    // A triangle passed at t in (tmin, tmax].  So near an end of the interval that the FP32
+    // distance may lie inside where the leaf lies outside, the leaf's built box decides.
+    auto meet = [&](uint32_t k, float t, float id_bits, float V, float W, float det) {
+        if (t < tmax && (t < sure_lo || (kAny && t > sure_hi))) {
+            const LeafTri& rec = bvh.tris[k];
+            const float4 b = *reinterpret_cast<const float4*>(rec.box_yz);
+            const float lx = rec.v1[3], hx = rec.v2[3];
+            const float tn = fmaxf(fmaxf(fmaf(sl.ix >= 0.f ? lx : hx, sl.ix, sl.nx), fmaf(sl.iy >= 0.f ? b.x : b.y, sl.iy, sl.ny)),
+                                   fmaxf(fmaf(sl.iz >= 0.f ? b.z : b.w, sl.iz, sl.nz), r.tmin));
+            const float tf = fminf(fminf(fmaf(sl.ix >= 0.f ? hx : lx, sl.ix, sl.fx), fmaf(sl.iy >= 0.f ? b.y : b.x, sl.iy, sl.fy)),
+                                   fminf(fmaf(sl.iz >= 0.f ? b.w : b.z, sl.iz, sl.fz), tmax));
+            if (!(tn <= tf * kBoxRobustExact)) return;
         }
-        if (cur != kDone && !(cur & kLeafBit)) {
-            const uint4 rc = *reinterpret_cast<const uint4*>(top + 96);
-            const uint32_t slot = cur == rc.x ? 1u : (cur == rc.y ? 2u : (cur == rc.z ? 3u : (cur == rc.w ? 4u : 0u)));
-            if (slot != 0u) {
-                if (kCount) cnt.nodes++;
-                nhit = node_children(lfetch, slot, sl, r.tmin, tmax, key, val);
-                cur = descend(nhit, key, val, tmax, st);
-                if (cur != kDone && (cur & kLeafBit) && leaf == kDone) {
-                    leaf = cur;
-                    cur = st.pop(tmax);
-                }
-            }
+        if (kAny) {
+            found = found || t < tmax;
+        } else if (t < tmax) {
+            tie = false;
+            found = true;
+            tmax = t;
+            accept_hit<kAny>(h, 0.f, k, __float_as_uint(id_bits), V, W, det);  // t: tmax once the ray is done
+        } else {
+            tie = found;
         }
     };
     const uint32_t waves = gridDim.x * (blockDim.x >> 6);
@@ -532,120 +674,127 @@ __device__ __forceinline__ void trace_persistent(const Node4* __restrict__ nodes
         if (lane < chunk && k < n) start(k);
     }
     bool exhausted = static_total >= n;  // wave-uniform
-    bool first = true;
-    // kRanged: rays come from ranges -- the wave's static 64, then ranges claimed from `next`.
-    // While at least a grid's worth of rays remains beyond the current range, the next 64-ray
-    // range is claimed one ahead of need (lane 0 holds its base), so a refill waits for no
-    // atomic; otherwise a refill claims exactly the rays it lacks, so the end of the batch
-    // stays balanced across waves.
-    uint32_t cur_next = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64u + 64u;
-    uint32_t cur_end = cur_next;
-    uint32_t pend = 0u;
-    bool has_pend = false;  // wave-uniform
+    // Ranges: [cur_next, cur_end) is being handed out; `pend` (held by lane 0) is the base of the
+    // next one, of pend_size rays.  A range holds a share of what is left, between 64
+    // and kMaxRange rays, so a long batch costs few atomics and its end stays balanced.
+    constexpr uint32_t kMaxRange = 1024u;
+    const uint32_t share = 33u - uint32_t(__clz(int(waves)));  // log2 of 2 to 4 times the waves
+    uint32_t cur_next = static_total, cur_end = static_total;
+    uint32_t pend = 0u, pend_size = 0u;
+    auto range_size = [&](uint32_t at) {
+        const uint32_t left = at < n ? n - at : 0u;
+        return min(max((left >> share) & ~63u, 64u), kMaxRange);
+    };
+    auto refill = [&]() {
+        const bool need = id == kNone && num_ties < kTies;
+        const unsigned long long mask = __ballot(need);
+        const uint32_t want = uint32_t(__popcll(mask));
+        if (want == 0u) return;
+        const uint32_t rank = uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
+        const uint32_t avail = cur_end - cur_next;
+        uint32_t k = cur_next + rank;
+        if (want > avail) {
+            uint32_t base = 0u, size = pend_size;
+            if (size != 0u) {
+                base = __builtin_amdgcn_readfirstlane(pend);
+                pend_size = 0u;
+            } else {
+                size = range_size(cur_end);
+                if (lane == 0u) base = static_total + atomicAdd(next, size);
+                base = __builtin_amdgcn_readfirstlane(base);
+            }
+            if (rank >= avail) k = base + (rank - avail);
+            cur_next = base + (want - avail);
+            cur_end = base + size;
+        } else {
+            cur_next += want;
+        }
+        if (need && k < n) start(k);
+        if (cur_next >= n) {
+            exhausted = true;
+        } else if (pend_size == 0u && cur_end < n && n - cur_end > static_total) {
+            pend_size = range_size(cur_end);
+            if (lane == 0u) pend = static_total + atomicAdd(next, pend_size);
+        }
+    };
     for (;;) {
-        if (kRanged && !exhausted && !first) {
-            const bool need = id == kNone;
-            const unsigned long long mask = __ballot(need);
-            const uint32_t cnt_need = uint32_t(__popcll(mask));
-            if (cnt_need > 0) {
-                const uint32_t rank = uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
-                const uint32_t avail = cur_end - cur_next;
-                uint32_t k = cur_next + rank;
-                if (cnt_need > avail) {
-                    uint32_t base = 0u;
-                    if (has_pend) {
-                        base = __shfl(pend, 0, 64);
-                        cur_next = base + (cnt_need - avail);
-                        cur_end = base + 64u;
-                        has_pend = false;
-                    } else {
-                        if (lane == 0u) base = static_total + atomicAdd(next, cnt_need - avail);
-                        base = __shfl(base, 0, 64);
-                        cur_next = cur_end = base + (cnt_need - avail);
-                    }
-                    if (rank >= avail) k = base + (rank - avail);
-                } else {
-                    cur_next += cnt_need;
-                }
-                if (need && k < n) start(k);
-                if (cur_next >= n) {
-                    exhausted = true;
-                } else if (!has_pend && cur_end + static_total < n) {
-                    if (lane == 0u) pend = static_total + atomicAdd(next, 64u);
-                    has_pend = true;
-                }
-            }
-        }
-        if (!kRanged && !exhausted && !first) {
-            const bool need = id == kNone;
-            const unsigned long long mask = __ballot(need);
-            const uint32_t cnt_need = uint32_t(__popcll(mask));
-            if (cnt_need > 0) {
-                const int leader = __ffsll((long long)mask) - 1;
-                uint32_t base = 0;
-                if (int(lane) == leader) base = atomicAdd(next, cnt_need);
-                base = __shfl(base, leader, 64) + static_total;
-                if (base + cnt_need >= n) exhausted = true;
-                if (need) {
-                    const uint32_t k = base + uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
-                    if (k < n) start(k);
-                }
-            }
-        }
-        first = false;
-        if (__ballot(id != kNone) == 0ull) break;
         for (;;) {
-            // Inner nodes, until every lane still descending holds a postponed leaf.
-            while (cur != kDone && !(cur & kLeafBit)) {
-                if (kCount) cnt.nodes++;
-                float key[4];
-                uint32_t val[4];
-                const int nhit = node_children(gfetch, cur, sl, r.tmin, tmax, key, val);
-                cur = descend(nhit, key, val, tmax, st);
-                if (cur != kDone && (cur & kLeafBit) && leaf == kDone) {
-                    leaf = cur;
-                    cur = st.pop(tmax);
-                }
-                if (__ballot(leaf == kDone) == 0ull) break;
-            }
-            // Postponed leaves, then any leaf that is next in line, one triangle per step: a
-            // lane that finishes a leaf moves on to its next one at once instead of waiting for
-            // the wave's longest leaf.  Per lane the triangles are tested in the same order as
-            // leaf by leaf.
-            uint32_t tri = 0u, tri_end = 0u;
-            if (leaf != kDone) {
-                tri = leaf & kMaxLeafFirst;
-                tri_end = tri + ((leaf >> 27) & 0xfu) + 1u;
-            }
-            while (tri < tri_end) {
-                if (kCount) cnt.tris++;
-                const float4* tp = reinterpret_cast<const float4*>(tris + tri);
-                const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
-                float t, U, V, W, det;
-                if (watertight(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det)) {
-                    found = true;
-                    tmax = t;
-                    accept_hit<kAny>(h, t, tri, __float_as_uint(v0.w), V, W, det);
-                    if (kAny) {
-                        cur = kDone;
-                        tri_end = tri;
+            const unsigned long long nm = __ballot(is_inner(cur)), lm = __ballot(tri < tri_end);
+            const unsigned long long pm = __ballot(cur == kPop);
+            const uint32_t nn = uint32_t(__popcll(nm)), nl = uint32_t(__popcll(lm)), busy = uint32_t(__popcll(nm | lm | pm));
+            if (busy == 0u || (!exhausted && busy <= 64u - kRefillIdle)) {
+                if (id != kNone && cur == kDone && tri >= tri_end) {
+                    if (!kAny && tie) {
+                        ties[num_ties++] = id;
+                    } else {
+                        h.t = tmax;
+                        if (!kAny && found) hit_weights(h);
+                        sink(id, found, h, r);
                     }
+                    id = kNone;
                 }
-                tri++;
-                if (tri >= tri_end && cur != kDone && (cur & kLeafBit)) {
-                    tri = cur & kMaxLeafFirst;
-                    tri_end = tri + ((cur >> 27) & 0xfu) + 1u;
-                    cur = st.pop(tmax);
+                if (busy == 0u && (exhausted || (!kAny && __ballot(num_ties < kTies) == 0ull))) break;
+                refill();
+            } else if (nn >= nl * kLeafWeight) {
+                if (is_inner(cur)) {
+                    if (kCount) cnt.nodes++;
+                    double e[4];
+                    node_children(fetch, cur, sl, r.tmin, tmax, e);
+                    cur = descend(e, st);
+                    take_leaf();
+                }
+            } else {
+                if (tri < tri_end) {
+                    // Two records a step: they share a line unless the second starts the next one.
+                    const bool two = tri + 1u < tri_end;
+                    const float4* ap = reinterpret_cast<const float4*>(bvh.tris + tri);
+                    const float4* bp = ap + (two ? sizeof(LeafTri) / 16 : 0);
+                    const float4 a0 = ap[0], a1 = ap[1], a2 = ap[2];
+                    const float4 b0 = bp[0], b1 = bp[1], b2 = bp[2];
+                    float t, U, V, W, det;
+                    if (kCount) cnt.tris++;
+                    if (watertight(sh, a0, a1, a2, r.tmin, tmax, t, U, V, W, det))
+                        meet(tri, t, a0.w, V, W, det);
+                    if (two && !(kAny && found)) {
+                        if (kCount) cnt.tris++;
+                        if (watertight(sh, b0, b1, b2, r.tmin, tmax, t, U, V, W, det))
+                            meet(tri + 1u, t, b0.w, V, W, det);
+                    }
+                    tri += 2u;
+                    if (kAny && found) {
+                        cur = kDone;
+                        tri_end = 0u;
+                    }
+                    take_leaf();
                 }
             }
-            leaf = kDone;
-            if (id != kNone && cur == kDone) {
-                sink(id, found, h, r);
-                id = kNone;
+            if (cur == kPop) {
+                cur = st.pop(tmax);
+                take_leaf();
             }
-            const uint32_t idle = uint32_t(__popcll(__ballot(id == kNone)));
-            if (idle == 64u || (!exhausted && idle >= uint32_t(kRanged ? kRefillIdleRanged : kRefillIdle))) break;
         }
+        if constexpr (kAny) break;
+        // All lanes are idle: nothing of the loop above is live here.
+        while (num_ties > 0u) {
+            num_ties--;
+            const RayIn q = src(ties[num_ties]);
+            HitOut hx = trace_exact(bvh, q, st);
+            const bool hit = hx.prim != kNone;
+            if (hit) hit_weights(hx);
+            sink(ties[num_ties], hit, hx, q);
+        }
+        if (exhausted) break;
+        r = RayIn{0.f, 0.f, 0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
+        sl = Slab{};
+        sh = ShearCyclic{};
+        h = HitOut{};
+        tmax = sure_lo = sure_hi = 0.f;
+        found = tie = false;
+        id = kNone;
+        cur = kDone;
+        tri = tri_end = 0u;
+        st.sp = 0u;
+        refill();
     }
 }
 
@@ -679,13 +828,13 @@ __device__ __forceinline__ void trace_brute(const TriRecord* __restrict__ tris, 
         const RayIn r = src(w);
         const ShearRows sh = make_shear_rows(r, make_shear(r));
         float tmax = r.tmax;
-        HitOut h{tmax, 0u, 0xffffffffu, 0.f, 0.f};
+        HitOut h{tmax, 0u, 0xffffffffu, 0.f, 0.f, 1.f};
         bool found = false;
         for (uint32_t j = lane; j < ntris; j += 64u) {
             const float4* tp = reinterpret_cast<const float4*>(tris + j);
             const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
             float t, U, V, W, det;
-            if (!(kAny && found) && watertight_rows(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det)) {
+            if (!(kAny && found) && watertight_rows(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det) && t < tmax) {
                 found = true;
                 tmax = t;
                 accept_hit<kAny>(h, t, j, __float_as_uint(v0.w), V, W, det);
@@ -707,7 +856,10 @@ __device__ __forceinline__ void trace_brute(const TriRecord* __restrict__ tris, 
             for (int off = 32; off > 0; off >>= 1) rec = min(rec, uint32_t(__shfl_xor(int(rec), off, 64)));
             winner = __ffsll(static_cast<long long>(__ballot(found && h.t == best && h.rec == rec))) - 1;
         }
-        if (int(lane) == winner) sink(w, true, h, r);
+        if (int(lane) == winner) {
+            if (!kAny) hit_weights(h);
+            sink(w, true, h, r);
+        }
         return;
     }
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
@@ -716,19 +868,20 @@ __device__ __forceinline__ void trace_brute(const TriRecord* __restrict__ tris, 
         const RayIn r = active ? src(i) : RayIn{0.f, 0.f, 0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
         const ShearRows sh = make_shear_rows(r, make_shear(r));
         float tmax = r.tmax;
-        HitOut h{tmax, 0u, 0xffffffffu, 0.f, 0.f};
+        HitOut h{tmax, 0u, 0xffffffffu, 0.f, 0.f, 1.f};
         bool found = false;
         for (uint32_t j = 0; j < ntris; j++) {
             const float4* tp = reinterpret_cast<const float4*>(tris + j);
             const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
             float t, U, V, W, det;
-            if (active && !(kAny && found) && watertight_rows(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det)) {
+            if (active && !(kAny && found) && watertight_rows(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det) && t < tmax) {
                 found = true;
                 tmax = t;
                 accept_hit<kAny>(h, t, j, __float_as_uint(v0.w), V, W, det);
             }
             if (kAny && __ballot(active && !found) == 0ull) break;
         }
+        if (!kAny && found) hit_weights(h);
         if (active) sink(i, found, h, r);
     }
 }
@@ -856,7 +1009,8 @@ __device__ __forceinline__ bool xform_any(const XformRecord* __restrict__ xf, ui
 
 // Barycentrics of the recorded winner (weights of v1 and v2): the FP32 weights kept at
 // acceptance, or the winner re-evaluated in FP64.
-__device__ __forceinline__ void winner_barycentrics(const TriRecord* __restrict__ tris, const RayIn& r,
+template <class Tri>
+__device__ __forceinline__ void winner_barycentrics(const Tri* __restrict__ tris, const RayIn& r,
                                                     const HitOut& h, bool fp64, float& t, float& b0, float& b1) {
     t = h.t;
     b0 = h.b0;

@@ -1,0 +1,103 @@
+"""The traversal's device layout -- packed nodes, leaves placed on lines, pairs of triangles a
+step, rays handed out in ranges -- at the sizes where it can go wrong, against every triangle
+tested in float64 on the CPU.
+
+A ray may differ from the float64 answer only where its FP32 arithmetic cannot decide: coordinates
+reach 3 units from the ray's origin, triangles measure about 0.05, so an edge function is known to
+about 16 * 2^-24 * 3 / 0.05 = 6e-5 of its triangle, rounded up to 1e-4; distances are compared to
+1e-6 relative between two candidate triangles."""
+import numpy as np
+import pytest
+
+from lightmetrica_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+NEAR_EDGE, NEAR_TIE = 1e-4, 1e-6
+NRAYS = 6000
+
+
+def make(kind, ntri, seed):
+    r = np.random.default_rng(seed)
+    c = r.uniform(0.0, 1.0, (ntri, 1, 3))
+    v = c + r.normal(0.0, 0.05, (ntri, 3, 3))
+    if kind == "flat":      # every box has no extent along z
+        v[:, :, 2] = 0.25
+    elif kind == "grid":    # shared planes: many equal box faces, half the boxes flat
+        v = np.round(v * 16.0) / 16.0
+        v = v[np.linalg.norm(np.cross(v[:, 1] - v[:, 0], v[:, 2] - v[:, 0]), axis=1) > 0]
+    P = v.reshape(-1, 3).astype(np.float32)
+    F = np.arange(P.shape[0], dtype=np.uint32).reshape(-1, 3)
+    o = r.uniform(-0.5, 1.5, (NRAYS, 3))
+    d = r.normal(size=(NRAYS, 3))
+    d[: NRAYS // 8, 0] = 0.0          # parallel to a plane of every box
+    d[NRAYS // 8: NRAYS // 4, 1:] = 0.0  # along an axis
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = scenes.Rays(o.astype(np.float32), d.astype(np.float32), np.zeros(NRAYS, np.float32),
+                       np.full(NRAYS, scenes.FLT_MAX, np.float32))
+    return scenes.Scene(kind, P, np.zeros_like(P), F), rays
+
+
+def brute(sc, rays):
+    """Per ray: the sorted distances and edge margins of the triangles it may hit, in float64."""
+    T = sc.positions.astype(np.float64)[sc.faces]
+    e1, e2 = T[:, 1] - T[:, 0], T[:, 2] - T[:, 0]
+    out = []
+    for a in range(0, NRAYS, 500):
+        o, d = rays.o[a:a + 500].astype(np.float64), rays.d[a:a + 500].astype(np.float64)
+        s1 = np.cross(d[:, None], e2[None])
+        det = (s1 * e1[None]).sum(-1)
+        with np.errstate(divide="ignore", invalid="ignore"):
+            q = o[:, None] - T[None, :, 0]
+            u = (q * s1).sum(-1) / det
+            s2 = np.cross(q, e1[None])
+            w = (d[:, None] * s2).sum(-1) / det
+            t = (e2[None] * s2).sum(-1) / det
+        margin = np.minimum(np.minimum(u, w), 1 - u - w)
+        ok = np.isfinite(t) & (t > 0)
+        out.append((np.where(ok, t, np.inf), np.where(ok, margin, -np.inf)))
+    return np.concatenate([x[0] for x in out]), np.concatenate([x[1] for x in out])
+
+
+@pytest.mark.parametrize("kind,ntri,leaf", [("soup", 129, 1), ("soup", 131, 2), ("soup", 257, 3), ("soup", 1000, 4),
+                                            ("soup", 1001, 5), ("soup", 999, 16), ("flat", 300, 4), ("grid", 700, 4),
+                                            ("grid", 700, 16)])
+def test_layout_finds_every_hit(gpu, kind, ntri, leaf):
+    sc, rays = make(kind, ntri, 1000 * leaf + ntri)
+    gpu.upload(sc)
+    gpu.build_bvh(max_leaf_size=leaf)
+    t, b0, b1, prim = gpu.trace_closest(rays, refine_fp64=True)
+    occluded = gpu.trace_any(rays)
+    T, M = brute(sc, rays)
+    rows = np.arange(NRAYS)
+    inside = np.where(M >= 0, T, np.inf)
+    best = inside.argmin(1)
+    hit = np.isfinite(inside[rows, best])
+    sure = np.where(M >= NEAR_EDGE, T, np.inf).min(1)  # the nearest triangle hit beyond doubt
+    found = prim >= 0
+    # a reported triangle is one the ray passes, up to the margin, and none beyond doubt is nearer
+    k = np.where(found, prim, 0)
+    assert np.all(M[rows, k][found] > -NEAR_EDGE)
+    assert np.all(np.abs(t - T[rows, k])[found] <= 1e-5 * np.maximum(T[rows, k][found], 1e-3))
+    assert np.all(T[rows, k][found] <= sure[found] * (1 + NEAR_TIE))
+    assert not np.any(~found & np.isfinite(sure))
+    same = (prim == best) & hit & found
+    assert (hit & ~same & ~np.isclose(np.where(found, T[rows, k], 0), inside[rows, best], rtol=NEAR_TIE)).sum() <= 20
+    np.testing.assert_array_equal(occluded, found)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 5000, 327_681, 700_001])
+def test_batches_of_any_size_agree(gpu, n):
+    """Rays handed out singly, in chunks and in ranges: a ray's result does not depend on its batch."""
+    sc, rays = make("soup", 1000, 5)
+    gpu.upload(sc)
+    gpu.build_bvh()
+    ref = gpu.trace_closest(rays, refine_fp64=False)
+    rep = np.arange(n) % NRAYS
+    many = scenes.Rays(rays.o[rep], rays.d[rep], rays.tmin[rep], rays.tmax[rep])
+    for refine in (False, True):
+        out = gpu.trace_closest(many, refine_fp64=refine)
+        np.testing.assert_array_equal(out[3], ref[3][rep])
+        if not refine:
+            np.testing.assert_array_equal(out[0], ref[0][rep])
+    np.testing.assert_array_equal(gpu.trace_any(many), ref[3][rep] >= 0)
