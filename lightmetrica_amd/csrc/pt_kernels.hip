@@ -815,6 +815,15 @@ struct HitSink {
     }
 };
 
+// The LDS of a stage that traces a queue, whatever the number of rays makes of it: late bounces
+// hold few rays, which several lanes follow each (trace_grouped).
+template <bool kKeys> union QueueShared {
+    TraceShared<kKeys> lane;
+    GroupShared<64> group64;
+    GroupShared<16> group16;
+    __device__ QueueShared() {}
+};
+
 // The traversal counters of a wave added to counts[0] (node visits) and counts[1] (triangle
 // tests), one atomic per wave each (the counting forms of the extension and shadow stages).
 __device__ __forceinline__ void add_wave_counts(const TraceCounters& cnt, unsigned long long* counts) {
@@ -835,12 +844,14 @@ template <bool kCount = false>
 __global__ __launch_bounds__(kTraceBlock, 6) void k_extend(BvhDev bvh, Queue q,
                                                         const uint32_t* __restrict__ count, uint32_t* next,
                                                         float4* __restrict__ hits, unsigned long long* counts) {
-    __shared__ TraceShared<true> sm;
+    __shared__ QueueShared<true> sm;
     const uint32_t n = *count;
     QueueSource src{q};
     HitSink sink{bvh.tris, hits};
     TraceCounters cnt{0, 0};
-    trace_persistent<false, kCount>(bvh, n, next, sm, src, sink, cnt);
+    if (n <= kGroup64Rays) trace_grouped<false, kCount, 64>(bvh, n, sm.group64, src, sink, cnt);
+    else if (n <= kGroup16Closest) trace_grouped<false, kCount, 16>(bvh, n, sm.group16, src, sink, cnt);
+    else trace_persistent<false, kCount>(bvh, n, next, sm.lane, src, sink, cnt);
     if (kCount) add_wave_counts(cnt, counts);
 }
 
@@ -1132,12 +1143,14 @@ struct ShadowSink {
 template <int kMode, bool kSplat = false, bool kCount = false>
 __global__ __launch_bounds__(kTraceBlock, 7) void k_shadow(PTConsts c, ShadowQueue sq, const uint32_t* __restrict__ count,
                                                         uint32_t* next, unsigned long long* counts) {
-    __shared__ TraceShared<false> sm;
+    __shared__ QueueShared<false> sm;
     const uint32_t n = *count;
     ShadowSource src{sq};
     ShadowSink<kMode, kSplat> sink{c, sq};
     TraceCounters cnt{0, 0};
-    trace_persistent<true, kCount>(c.bvh, n, next, sm, src, sink, cnt);
+    if (n <= kGroup64Rays) trace_grouped<true, kCount, 64>(c.bvh, n, sm.group64, src, sink, cnt);
+    else if (n <= kGroup16Any) trace_grouped<true, kCount, 16>(c.bvh, n, sm.group16, src, sink, cnt);
+    else trace_persistent<true, kCount>(c.bvh, n, next, sm.lane, src, sink, cnt);
     if (kCount) add_wave_counts(cnt, counts);
 }
 
@@ -1221,12 +1234,14 @@ struct RaycastSink {
 };
 
 template <class Out>
-__global__ __launch_bounds__(kTraceBlock) void k_raycast(PTConsts c, uint32_t n, uint32_t* next, Out* out) {
-    __shared__ TraceShared<true> sm;
+__global__ __launch_bounds__(kTraceBlock, 5) void k_raycast(PTConsts c, uint32_t n, uint32_t* next, Out* out) {
+    __shared__ QueueShared<true> sm;
     RaycastSource src{c.cam};
     RaycastSink<Out> sink{c, out};
     TraceCounters cnt{0, 0};
-    trace_persistent<false, false>(c.bvh, n, next, sm, src, sink, cnt);
+    if (n <= kGroup64Rays) trace_grouped<false, false, 64>(c.bvh, n, sm.group64, src, sink, cnt);
+    else if (n <= kGroup16Closest) trace_grouped<false, false, 16>(c.bvh, n, sm.group16, src, sink, cnt);
+    else trace_persistent<false, false>(c.bvh, n, next, sm.lane, src, sink, cnt);
 }
 
 __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
@@ -1616,8 +1631,9 @@ struct Pipeline {
         c.batch = nb;
         hipLaunchKernelGGL(k_zero_u32, dim3(2), dim3(256), 0, s, b.counters, uint32_t(4 * kMaxSegments));
         const dim3 grid_b((nb + kPTBlock - 1) / kPTBlock), grid_c((cap + kPTBlock - 1) / kPTBlock);
-        // Persistent traversal grids: the device fill, never more than the queue capacity needs.
-        const dim3 grid_t(std::min<uint32_t>(grid_c.x, trace_grid));
+        // Persistent traversal grids: the device fill, never more than the queue capacity needs with a
+        // wave per ray.
+        const dim3 grid_t(std::min<uint32_t>((cap + kTraceBlock / 64 - 1) / (kTraceBlock / 64), trace_grid));
         // Brute-force traversal grids: 16 blocks of kTraceBlock per CU, walking the queue.
         const dim3 grid_r(std::min<uint32_t>((cap + kTraceBlock - 1) / kTraceBlock, 16u * uint32_t(std::max(ctx->num_cus, 1))));
         const uint32_t ntris = ctx->num_records;
@@ -1773,7 +1789,7 @@ lmgpu_status run_raycast(lmgpu_ctx* ctx, lmgpu_film* film) {
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_raycast<float>, kTraceBlock, 0) != hipSuccess || occ < 1)
         occ = 1;
-    const uint32_t grid = std::min<uint32_t>((n + kTraceBlock - 1) / kTraceBlock,
+    const uint32_t grid = std::min<uint32_t>((n + kTraceBlock / 64 - 1) / (kTraceBlock / 64),
                                              uint32_t(std::max(ctx->num_cus, 1)) * uint32_t(occ));
     hipStream_t s = ctx->stream;
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, ctx->next_counter, 1u);

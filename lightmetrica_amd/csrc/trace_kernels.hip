@@ -105,6 +105,30 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_closest_brute(const TriRe
     trace_brute<false>(tris, ntris, n, src, sink);
 }
 
+// Small batches, kLanes lanes per ray (trace_grouped): one launch, the FP64 evaluation included.
+template <bool kRefine, int kLanes>
+__global__ __launch_bounds__(kTraceBlock, 6) void k_trace_closest_grouped(BvhDev bvh, RaysSoA rays, uint32_t n,
+                                                                       float* __restrict__ t_out,
+                                                                       float* __restrict__ b0_out,
+                                                                       float* __restrict__ b1_out,
+                                                                       int32_t* __restrict__ prim_out) {
+    __shared__ GroupShared<kLanes> sm;
+    SoASource src{rays};
+    ClosestSink<kRefine, LeafTri> sink{bvh.tris, t_out, b0_out, b1_out, prim_out};
+    TraceCounters cnt{0, 0};
+    trace_grouped<false, false, kLanes>(bvh, n, sm, src, sink, cnt);
+}
+
+template <int kLanes>
+__global__ __launch_bounds__(kTraceBlock) void k_trace_any_grouped(BvhDev bvh, RaysSoA rays, uint32_t n,
+                                                                   uint8_t* __restrict__ occluded) {
+    __shared__ GroupShared<kLanes> sm;
+    SoASource src{rays};
+    OcclusionSink sink{occluded};
+    TraceCounters cnt{0, 0};
+    trace_grouped<true, false, kLanes>(bvh, n, sm, src, sink, cnt);
+}
+
 // The hits of k_trace_record, evaluated in FP64 (refine_fp64): prim holds the leaf-order record
 // of the winner (-1 for a miss), replaced here by its scene-order id.  Only the origin and
 // direction of a hit ray are read.  Where the FP64 determinant is 0 the traversal's FP32
@@ -236,6 +260,8 @@ template <class K> static uint32_t persistent_blocks(lmgpu_ctx* ctx, K kernel, u
     return uint32_t(std::max<uint64_t>(1, std::min(full, need)));
 }
 
+static dim3 group_blocks(uint32_t n, uint32_t lanes) { return dim3((n + kTraceBlock / lanes - 1) / (kTraceBlock / lanes)); }
+
 // Grid of the brute-force kernels: 16 blocks per CU at most, walking the batch.
 static uint32_t brute_blocks(lmgpu_ctx* ctx, uint32_t n) {
     const uint64_t need = (uint64_t(n) + kTraceBlock - 1) / kTraceBlock;
@@ -268,6 +294,14 @@ hipError_t launch_trace_closest(lmgpu_ctx* ctx, const float* const* rays, uint32
                 hipLaunchKernelGGL(k_trace_closest_brute<false>, dim3(brute_blocks(ctx, n)), block, 0, ctx->stream,
                                    ctx->tris.ptr, ntris, soa_of(rays), n, t, b0, b1, prim);
         });
+    if (n <= kGroup16Closest)
+        return timed(ctx, kKTraceClosest, [&]() {
+            const bool whole = n <= kGroup64Rays;
+            auto kernel = refine ? (whole ? k_trace_closest_grouped<true, 64> : k_trace_closest_grouped<true, 16>)
+                                 : (whole ? k_trace_closest_grouped<false, 64> : k_trace_closest_grouped<false, 16>);
+            hipLaunchKernelGGL(kernel, group_blocks(n, whole ? 64 : 16), block, 0, ctx->stream, bvh_of(ctx), soa_of(rays),
+                               n, t, b0, b1, prim);
+        });
     return timed(ctx, kKTraceClosest, [&]() {
         hipLaunchKernelGGL(k_zero_next, dim3(1), dim3(64), 0, ctx->stream, next);
         if (refine) {
@@ -293,6 +327,13 @@ hipError_t launch_trace_any(lmgpu_ctx* ctx, const float* const* rays, uint32_t n
         return timed(ctx, kKTraceAny, [&]() {
             hipLaunchKernelGGL(k_trace_any_brute, dim3(brute_blocks(ctx, n)), dim3(kTraceBlock), 0, ctx->stream,
                                ctx->tris.ptr, ntris, soa_of(rays), n, occluded);
+        });
+    if (n <= kGroup16Any)
+        return timed(ctx, kKTraceAny, [&]() {
+            const bool whole = n <= kGroup64Rays;
+            auto kernel = whole ? k_trace_any_grouped<64> : k_trace_any_grouped<16>;
+            hipLaunchKernelGGL(kernel, group_blocks(n, whole ? 64 : 16), dim3(kTraceBlock), 0, ctx->stream, bvh_of(ctx),
+                               soa_of(rays), n, occluded);
         });
     return timed(ctx, kKTraceAny, [&]() {
         hipLaunchKernelGGL(k_zero_next, dim3(1), dim3(64), 0, ctx->stream, next);

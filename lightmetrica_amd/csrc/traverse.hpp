@@ -798,6 +798,164 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
     }
 }
 
+// ---- Several lanes per ray ----------------------------------------------------------------
+// Batches with few rays for the chip -- a probe, a late bounce -- last as long as one ray's
+// chain of dependent fetches.  Here kLanes lanes follow one ray: each round takes up to
+// kLanes / 4 nodes off the ray's stack, nearest on top, and every lane tests one child of one
+// of them; the leaves found are tested at once, one triangle per lane.  With 64 lanes the chain
+// is about the tree's depth instead of every node and leaf the ray visits.  The boxes are the
+// built ones, so a leaf is met exactly if a depth-first descent could meet it; ties go to
+// trace_exact.  The lanes of a ray are consecutive and every branch is uniform among them.
+// Measured on device rays with the FP64 evaluation (1k to 1M triangles), us a batch: 81 rays 76-106
+// one lane each, 8-14 with 64 lanes each; 1000 rays 98-136 -> 9-14; 32768 rays 97-193 -> 22-33 with
+// 16 lanes each.  With three streams in flight the one-lane kernel overlaps its tails: 41-75 at 32768
+// rays, 35-87 at 65549 against 42-67 with 16 lanes, hence the bounds:
+constexpr uint32_t kGroup64Rays = 8192;     // 64 lanes per ray (4000 rays: 6-9 against 8-16 with 16 lanes; 16384: 18-24, 12-19)
+constexpr uint32_t kGroup16Closest = 65536;  // 16 lanes per ray, closest hit
+constexpr uint32_t kGroup16Any = 98304;      // any hit (65549 rays: 27-48 against 36-72; 131072: 53-94, 42-82)
+template <int kLanes> struct GroupShared {
+    static constexpr uint32_t kRays = kTraceBlock / kLanes;
+    // Entries that one node at a time can add (3 * depth), and as much again for kLanes / 4.
+    static constexpr uint32_t kDeep = 96, kRoom = kLanes == 64 ? 160 : 48;
+    uint2 node[kRays][kDeep + kRoom];  // reference, entry distance
+    uint32_t leaf[kRays][kLanes];
+};
+
+// The stack of trace_exact for a group's one ray.
+struct PrivateStack {
+    uint32_t* slot;
+    uint32_t sp = 0u;
+    __device__ __forceinline__ void push(double e) {
+        if (sp < uint32_t(kStackTotal)) slot[sp++] = entry_ref(e);
+    }
+    __device__ __forceinline__ uint32_t pop(float) { return sp > 0u ? slot[--sp] : kDone; }
+};
+
+// Orders a wave's LDS writes before its later reads (the hardware keeps them in order).
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Group g of the grid traces rays g, g + groups, ...; as in trace_persistent, `sink` is called once
+// per ray, by one lane.  With kCount the lanes count the children and triangles they test.
+template <bool kAny, bool kCount, int kLanes, class Source, class Sink>
+__device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, GroupShared<kLanes>& sm, Source& src,
+                                              Sink& sink, TraceCounters& cnt) {
+    constexpr uint32_t kNodes = kLanes / 4;
+    const uint32_t lane = __lane_id() & (kLanes - 1u), base = __lane_id() & ~(kLanes - 1u);
+    const uint32_t sub = lane & 3u, slot = lane >> 2, quad = lane & ~3u;
+    const uint32_t in_block = threadIdx.x / kLanes, groups = gridDim.x * (kTraceBlock / kLanes);
+    auto ballot = [&](bool p) -> unsigned long long {
+        const unsigned long long m = __ballot(p);
+        if constexpr (kLanes == 64) return m;
+        else return (m >> base) & ((1ull << kLanes) - 1ull);
+    };
+    uint2* stack = sm.node[in_block];
+    uint32_t* leaves = sm.leaf[in_block];
+    for (uint32_t i = blockIdx.x * (kTraceBlock / kLanes) + in_block; i < n; i += groups) {
+        const RayIn r = src(i);
+        const Slab sl = make_slab(r);
+        const ShearCyclic sh = make_shear_cyclic(r);
+        float tmax = r.tmax;
+        HitOut h{0.f, 0u, 0xffffffffu, 0.f, 0.f, 1.f};
+        bool mine = false;                // this lane met a triangle
+        bool found = false, tie = false;  // of the ray
+        uint32_t sp = 1u;
+        wave_fence();
+        if (lane == 0u) stack[0] = make_uint2(0u, 0xff800000u);
+        while (sp > 0u && !(kAny && found)) {
+            // As many nodes as their children are sure to fit for.
+            const uint32_t take = sp + 3u * kNodes <= GroupShared<kLanes>::kRoom ? min(sp, kNodes) : 1u;
+            wave_fence();
+            const uint2 e = stack[slot < take ? sp - 1u - slot : 0u];
+            sp -= take;
+            bool hit = false;
+            float tn = INFINITY;
+            uint32_t child = kEmptyChild;
+            if (slot < take && !(__uint_as_float(e.y) > tmax * kBoxRobustExact)) {
+                if (kCount) cnt.nodes += sub == 0u ? 1u : 0u;
+                const float* nd = reinterpret_cast<const float*>(bvh.exact + e.x) + sub;
+                const float lx = nd[0], hx = nd[4], ly = nd[8], hy = nd[12], lz = nd[16], hz = nd[20];
+                child = __float_as_uint(nd[24]);
+                tn = fmaxf(fmaxf(fmaf(sl.ix >= 0.f ? lx : hx, sl.ix, sl.nx), fmaf(sl.iy >= 0.f ? ly : hy, sl.iy, sl.ny)),
+                           fmaxf(fmaf(sl.iz >= 0.f ? lz : hz, sl.iz, sl.nz), r.tmin));
+                const float tf = fminf(fminf(fmaf(sl.ix >= 0.f ? hx : lx, sl.ix, sl.fx), fmaf(sl.iy >= 0.f ? hy : ly, sl.iy, sl.fy)),
+                                       fminf(fmaf(sl.iz >= 0.f ? hz : lz, sl.iz, sl.fz), tmax));
+                hit = child != kEmptyChild && tn <= tf * kBoxRobustExact;
+            }
+            const bool inner = hit && is_inner(child), leaf = hit && !is_inner(child);
+            // Inner children: the top node's on top, each node's nearest uppermost.
+            const unsigned long long im = ballot(inner);
+            const uint32_t key = inner ? __float_as_uint(fmaxf(tn, 0.f)) : 0x7f800000u;
+            uint32_t rank = 0u;
+#pragma unroll
+            for (uint32_t k = 1; k < 4u; k++) {
+                const uint32_t other = uint32_t(__shfl_xor(int(key), int(k), 64));
+                rank += other < key || (other == key && (sub ^ k) < sub) ? 1u : 0u;
+            }
+            const uint32_t below = uint32_t(__popcll(im >> quad));  // in this node and the ones under it
+            wave_fence();
+            if (inner) stack[sp + below - 1u - rank] = make_uint2(child, __float_as_uint(tn));
+            sp += uint32_t(__popcll(im));
+            const unsigned long long lm = ballot(leaf);
+            const uint32_t nl = uint32_t(__popcll(lm));
+            if (nl == 0u) continue;
+            if (leaf) leaves[__popcll(lm & ((1ull << lane) - 1ull))] = child;
+            wave_fence();
+            for (uint32_t l = 0; l < nl && !(kAny && found); l += kNodes) {
+                const uint32_t ref = l + slot < nl ? leaves[l + slot] : kDone;
+                uint32_t tri = (ref & kMaxLeafFirst) + sub, end = tri - sub + ((ref >> 27) & 0xfu) + 1u;
+                if (ref == kDone) end = tri = 0u;
+                for (; ballot(tri < end) != 0ull; tri += 4u) {
+                    float t = INFINITY, U, V, W, det;
+                    bool met = false, same = false;
+                    if (tri < end) {
+                        if (kCount) cnt.tris++;
+                        const float4* tp = reinterpret_cast<const float4*>(bvh.tris + tri);
+                        const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
+                        if (watertight(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det)) {
+                            met = t < tmax;
+                            same = !met && found;
+                            if (met) accept_hit<kAny>(h, t, tri, __float_as_uint(v0.w), V, W, det);
+                        }
+                    }
+                    const bool any_met = ballot(met) != 0ull;
+                    if (kAny) {
+                        found = found || any_met;
+                        if (found) break;
+                        continue;
+                    }
+                    tie = tie || ballot(same) != 0ull;
+                    if (any_met) {
+                        mine = mine || met;
+                        found = true;
+                        float m = met ? t : INFINITY;
+#pragma unroll
+                        for (int off = kLanes / 2; off > 0; off >>= 1) m = fminf(m, __shfl_xor(m, off, 64));
+                        tmax = m;
+                        tie = __popcll(ballot(met && t == tmax)) > 1;
+                    }
+                }
+            }
+        }
+        if (kAny) {
+            if (lane == 0u) sink(i, found, h, r);
+            continue;
+        }
+        const unsigned long long holders = ballot(mine && h.t == tmax);
+        const bool lead = found ? lane == uint32_t(__ffsll(static_cast<long long>(holders)) - 1) : lane == 0u;
+        if (!lead) continue;
+        if (tie) {
+            uint32_t slots[kStackTotal];
+            PrivateStack st{slots};
+            h = trace_exact(bvh, r, st);
+        }
+        if (found) hit_weights(h);
+        sink(i, found, h, r);
+    }
+}
+
 // Scenes of at most kBruteMaxTris triangles skip the BVH: every lane tests every triangle
 // record, in the same order, so the records are read at wave-uniform addresses and no lane
 // idles in a divergent descent -- the loop of the reference's NaiveScene

@@ -101,3 +101,23 @@ def test_batches_of_any_size_agree(gpu, n):
         if not refine:
             np.testing.assert_array_equal(out[0], ref[0][rep])
     np.testing.assert_array_equal(gpu.trace_any(many), ref[3][rep] >= 0)
+
+
+@pytest.mark.parametrize("n", [1, 8192, 8193, 65_536, 65_537, 98_304, 98_305, 400_001])
+def test_kernels_by_batch_size_agree(gpu, n):
+    """64 and 16 lanes per ray, one lane per ray: at the bounds between them a ray's result is the
+    same, ties included -- every triangle is there twice, so every hit is one."""
+    sc, rays = make("soup", 500, 7)
+    sc = scenes.Scene("twice", np.concatenate([sc.positions, sc.positions]), np.concatenate([sc.normals, sc.normals]),
+                      np.concatenate([sc.faces, sc.faces + sc.positions.shape[0]]))
+    gpu.upload(sc)
+    gpu.build_bvh()
+    ref = gpu.trace_closest(rays, refine_fp64=True)
+    T, M = brute(sc, rays)
+    sure = np.where(M >= NEAR_EDGE, T, np.inf).min(1)
+    assert np.all(np.isfinite(sure) <= (ref[3] >= 0))
+    rep = np.arange(n) % NRAYS
+    many = scenes.Rays(rays.o[rep], rays.d[rep], rays.tmin[rep], rays.tmax[rep])
+    for a, b in zip(gpu.trace_closest(many, refine_fp64=True), ref):
+        np.testing.assert_array_equal(a, b[rep])
+    np.testing.assert_array_equal(gpu.trace_any(many), ref[3][rep] >= 0)
