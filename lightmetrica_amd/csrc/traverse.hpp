@@ -565,21 +565,20 @@ __device__ __forceinline__ HitOut trace_exact(const BvhDev& bvh, const RayIn& r,
 }
 
 // A wave fetches new rays once this many of its lanes are idle: fetching costs the setup of the
-// rays' constants for the idle lanes only, waiting leaves lanes out of every step.  16M rays:
-// 12 idle lanes 3.65 ms, 20: 3.45, 28: 3.38; extension rays of the 96k-triangle room 11.6, 11.6, 11.8.
-constexpr uint32_t kRefillIdle = 20;
+// rays' constants for the idle lanes only, waiting leaves lanes out of every step.  16M rays: 12
+// idle lanes 3.14 ms, 16: 3.08, 28: 3.25; extension rays of the 96k-triangle room 10.6, 10.6, 10.9.
+constexpr uint32_t kRefillIdle = 16;
 // A wave takes a node step while at least this many times more lanes wait at nodes than hold a
 // leaf: a leaf step is shorter and frees its lanes to shrink tmax.  2 against 1: extension rays
 // 11.8 -> 11.5 ms, 1M-triangle city 2.65 -> 2.49 ms, 16M rays the same; 3: 11.8 ms.
 constexpr uint32_t kLeafWeight = 2;
 
 // Persistent traversal with per-lane ray refill (Aila & Laine, "Understanding the
-// efficiency of ray traversal on GPUs", HPG 2009): every wave of the grid loops over
-// the batch.  The first 64 rays of a wave are assigned statically (wave w takes
-// [64 w, 64 w + 64)); after that lanes whose rays have finished fetch the next unclaimed
-// rays once kRefillIdle of the wave's lanes are idle, from ranges claimed from `next` (which
-// counts from 64 x the number of waves) one range ahead of need, so that a refill waits for no
-// atomic.  A batch smaller than the grid costs no atomics.
+// efficiency of ray traversal on GPUs", HPG 2009): every wave of the grid loops over its rays,
+// and lanes whose rays have finished fetch new ones once kRefillIdle of the wave's lanes are
+// idle.  A batch of up to kEvenRounds rays per lane is dealt out beforehand; a larger one gives
+// each wave 64 rays and the rest in ranges claimed from `next` (which counts from 64 x the
+// number of waves) one range ahead of need, so that a refill waits for no atomic.
 // A lane visits nodes until it meets a leaf, and goes on visiting nodes while the leaf's
 // triangles are still to be tested (speculative traversal, same paper); a second leaf stops
 // it.  Each step of the wave serves the larger of the two groups.  A lane whose node left
@@ -590,6 +589,11 @@ constexpr uint32_t kLeafWeight = 2;
 // lane's node visits and triangle tests over all rays it traced.
 // n is at most kMaxBatch: a claim past the end then never wraps the counter.
 constexpr uint32_t kMaxBatch = 0x80000000u;
+// Up to this many rays per lane of the grid a wave's rays are fixed beforehand, consecutive and as
+// many for each: 0.9M camera rays 240 -> 153 us, extension rays of the 96k-triangle room 12.0 ->
+// 10.6 ms, shadow rays of a 1M-triangle city 1.10 -> 0.85 ms.  Beyond, ranges claimed as they are
+// needed balance better (24 instead of 16: extension rays 11.3 ms; 64: 16M rays 3.09 -> 3.25 ms).
+constexpr uint32_t kEvenRounds = 16;
 template <bool kAny, bool kCount, class Source, class Sink>
 __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, uint32_t* next, TraceShared<!kAny>& sm, Source& src,
                                                  Sink& sink, TraceCounters& cnt) {
@@ -663,23 +667,21 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
         }
     };
     const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     const uint32_t static_total = waves * 64u;
-    {
-        // A batch of at most 64 rays per wave is spread evenly over all waves, in chunks of
-        // ceil(n / waves) consecutive rays: a wave runs as long as the slowest of its rays
-        // (and the four-cycle issue of each instruction does not shrink with the lanes in
-        // use), so fewer rays per wave end a small batch -- a late bounce -- sooner.
-        const uint32_t chunk = static_total >= n ? (n + waves - 1u) / waves : 64u;
-        const uint32_t k = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * chunk + lane;
-        if (lane < chunk && k < n) start(k);
-    }
-    bool exhausted = static_total >= n;  // wave-uniform
+    // A batch of up to kEvenRounds rays per lane is spread evenly over all waves, each taking
+    // ceil(n / waves) consecutive ones: ranges would give some waves a round more than others.
+    const bool even = n <= static_total * kEvenRounds;
+    const uint32_t chunk = even ? (n + waves - 1u) / waves : 64u;
+    uint32_t cur_next = min(wave * chunk + min(chunk, 64u), n);
+    uint32_t cur_end = even ? uint32_t(min(uint64_t(wave + 1u) * chunk, uint64_t(n))) : cur_next;
+    if (lane < min(chunk, 64u) && wave * chunk + lane < n) start(wave * chunk + lane);
+    bool exhausted = cur_next >= (even ? cur_end : n);  // wave-uniform
     // Ranges: [cur_next, cur_end) is being handed out; `pend` (held by lane 0) is the base of the
     // next one, of pend_size rays.  A range holds a share of what is left, between 64
     // and kMaxRange rays, so a long batch costs few atomics and its end stays balanced.
     constexpr uint32_t kMaxRange = 1024u;
     const uint32_t share = 33u - uint32_t(__clz(int(waves)));  // log2 of 2 to 4 times the waves
-    uint32_t cur_next = static_total, cur_end = static_total;
     uint32_t pend = 0u, pend_size = 0u;
     auto range_size = [&](uint32_t at) {
         const uint32_t left = at < n ? n - at : 0u;
@@ -693,13 +695,19 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
         const uint32_t rank = uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
         const uint32_t avail = cur_end - cur_next;
         uint32_t k = cur_next + rank;
+        if (even) {
+            if (need && rank < avail) start(k);
+            cur_next = min(cur_next + want, cur_end);
+            exhausted = cur_next >= cur_end;
+            return;
+        }
         if (want > avail) {
             uint32_t base = 0u, size = pend_size;
             if (size != 0u) {
                 base = __builtin_amdgcn_readfirstlane(pend);
                 pend_size = 0u;
             } else {
-                size = range_size(cur_end);
+                size = range_size(max(cur_end, static_total));
                 if (lane == 0u) base = static_total + atomicAdd(next, size);
                 base = __builtin_amdgcn_readfirstlane(base);
             }
@@ -713,7 +721,7 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
         if (cur_next >= n) {
             exhausted = true;
         } else if (pend_size == 0u && cur_end < n && n - cur_end > static_total) {
-            pend_size = range_size(cur_end);
+            pend_size = range_size(max(cur_end, static_total));
             if (lane == 0u) pend = static_total + atomicAdd(next, pend_size);
         }
     };
