@@ -616,6 +616,7 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
     constexpr uint32_t kTies = 4;
     uint32_t ties[kAny ? 1 : kTies];
     uint32_t num_ties = 0u;
+    unsigned long long full = 0ull;  // the lanes whose list is
     uint32_t cur = kDone;   // next node or leaf reference to visit
     uint32_t tri = 0u, tri_end = 0u;  // records left of the leaf being tested
     const NodeFetch fetch(bvh.nodes);
@@ -730,7 +731,9 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
             const unsigned long long nm = __ballot(is_inner(cur)), lm = __ballot(tri < tri_end);
             const unsigned long long pm = __ballot(cur == kPop);
             const uint32_t nn = uint32_t(__popcll(nm)), nl = uint32_t(__popcll(lm)), busy = uint32_t(__popcll(nm | lm | pm));
-            if (busy == 0u || (!exhausted && busy <= 64u - kRefillIdle)) {
+            // A lane with a full list cannot be served: it counts as busy, or the wave would come here
+            // for it again and again and take no step.
+            if (busy == 0u || (!exhausted && uint32_t(__popcll(nm | lm | pm | full)) <= 64u - kRefillIdle)) {
                 if (id != kNone && cur == kDone && tri >= tri_end) {
                     if (!kAny && tie) {
                         ties[num_ties++] = id;
@@ -741,7 +744,8 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
                     }
                     id = kNone;
                 }
-                if (busy == 0u && (exhausted || (!kAny && __ballot(num_ties < kTies) == 0ull))) break;
+                if (!kAny) full = __ballot(num_ties == kTies);
+                if (busy == 0u && (exhausted || full == ~0ull)) break;
                 refill();
             } else if (nn >= nl * kLeafWeight) {
                 if (is_inner(cur)) {
@@ -792,6 +796,7 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
             sink(ties[num_ties], hit, hx, q);
         }
         if (exhausted) break;
+        full = 0ull;
         r = RayIn{0.f, 0.f, 0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
         sl = Slab{};
         sh = ShearCyclic{};

@@ -121,3 +121,26 @@ def test_kernels_by_batch_size_agree(gpu, n):
     for a, b in zip(gpu.trace_closest(many, refine_fp64=True), ref):
         np.testing.assert_array_equal(a, b[rep])
     np.testing.assert_array_equal(gpu.trace_any(many), ref[3][rep] >= 0)
+
+
+@pytest.mark.parametrize("n", [2_500_001, 6_000_001])
+def test_many_ties_a_lane(gpu, n):
+    """Every ray's nearest hit is a tie, more of them than a lane keeps for later, in batches dealt
+    out beforehand and in ranges."""
+    torch = pytest.importorskip("torch")
+    sc, rays = make("soup", 500, 7)
+    sc = scenes.Scene("twice", np.concatenate([sc.positions, sc.positions]), np.concatenate([sc.normals, sc.normals]),
+                      np.concatenate([sc.faces, sc.faces + sc.positions.shape[0]]))
+    gpu.upload(sc)
+    gpu.build_bvh()
+    ref = gpu.trace_closest(rays, refine_fp64=False)
+    hits = np.flatnonzero(ref[3] >= 0)
+    rep = hits[np.arange(n) % len(hits)]
+    cols = [torch.from_numpy(np.ascontiguousarray(a[rep])).cuda() for a in
+            (*rays.o.T, *rays.d.T, rays.tmin, rays.tmax)]
+    out = [torch.empty(n, device="cuda") for _ in range(3)] + [torch.empty(n, dtype=torch.int32, device="cuda")]
+    torch.cuda.synchronize()
+    gpu.trace_closest_device([c.data_ptr() for c in cols], [c.data_ptr() for c in out], n, refine_fp64=False)
+    gpu.synchronize()
+    for a, b in zip(out, ref):
+        np.testing.assert_array_equal(a.cpu().numpy(), b[rep])
