@@ -10,6 +10,7 @@
 #include "../../include/lmgpu.h"
 #include "bvh_build.h"
 #include "device_math.hpp"
+#include "host_io.hpp"
 
 namespace lmgpu {
 
@@ -127,8 +128,8 @@ struct lmgpu_ctx {
     // Staging of host rays / hits for the trace entry points.
     void* trace_staging = nullptr;
     size_t trace_staging_bytes = 0;
-    void* host_pinned = nullptr;  // pinned host chunks of large host-buffer traces
-    size_t host_pinned_bytes = 0;
+    lmgpu::HostIo* io = nullptr;  // acquired by ensure_pinned
+    hipEvent_t io_events[7] = {};
     hipStream_t copy_streams[2] = {nullptr, nullptr};  // their uploads and read-backs
     uint64_t* count_buf = nullptr;  // 2 x u64 for lmgpu_trace_count
     uint32_t* next_counter = nullptr;  // work counter of the persistent traversal kernels
@@ -161,6 +162,7 @@ struct lmgpu_ctx {
     double kernel_ms[lmgpu::kKNumClasses] = {};
     uint64_t kernel_launches[lmgpu::kKNumClasses] = {};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipEvent_t run0 = nullptr, run1 = nullptr;  // of a whole render or adjoint
 };
 
 namespace lmgpu {
@@ -174,6 +176,16 @@ lmgpu_status fail(lmgpu_ctx* ctx, lmgpu_status s, const std::string& msg);
 lmgpu_status hip_fail(lmgpu_ctx* ctx, hipError_t e, const char* what);
 lmgpu_status dev_alloc(lmgpu_ctx* ctx, void** p, size_t bytes, const char* what);
 void dev_free(void* p);
+
+// Grows the context's pinned memory to at least `bytes` (its contents are lost); false if it cannot
+// be had.
+bool ensure_pinned(lmgpu_ctx* ctx, size_t bytes);
+bool ensure_io_events(lmgpu_ctx* ctx);
+constexpr size_t kReadSlot = size_t(2) << 20;
+constexpr size_t kReadSlots = 4;
+// Copies device results to a host array, behind the work on the context's stream; returns when
+// they are there.
+hipError_t read_back(lmgpu_ctx* ctx, void* dst, const void* src, size_t bytes);
 
 // Times `launch` with HIP events on the context stream when timing is enabled.
 template <class Fn> hipError_t timed(lmgpu_ctx* ctx, int cls, Fn&& launch) {

@@ -5,10 +5,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <atomic>
 #include <mutex>
 #include <new>
-#include <thread>
 #include <vector>
 
 using namespace lmgpu;
@@ -69,6 +67,112 @@ lmgpu_status dev_alloc(lmgpu_ctx* ctx, void** p, size_t bytes, const char* what)
 
 void dev_free(void* p) {
     if (p) (void)hipFree(p);
+}
+
+// Left to the process at its end: the runtime may be gone before static objects are.
+struct HostIoPool {
+    std::mutex m;
+    std::vector<HostIo*> idle;
+    size_t contexts = 0;
+};
+static HostIoPool& host_io_pool() {
+    static HostIoPool* pool = new HostIoPool;
+    return *pool;
+}
+static void host_io_free(HostIo* io) {
+    if (io->pinned) (void)hipHostFree(io->pinned);
+    delete io;
+}
+
+void host_io_context() {
+    HostIoPool& pool = host_io_pool();
+    std::lock_guard<std::mutex> lock(pool.m);
+    pool.contexts++;
+}
+
+HostIo* host_io_acquire() {
+    HostIoPool& pool = host_io_pool();
+    std::lock_guard<std::mutex> lock(pool.m);
+    if (pool.idle.empty()) return new (std::nothrow) HostIo;
+    HostIo* io = pool.idle.back();
+    pool.idle.pop_back();
+    return io;
+}
+
+void host_io_release(HostIo* io) {
+    HostIoPool& pool = host_io_pool();
+    std::vector<HostIo*> gone;
+    {
+        std::lock_guard<std::mutex> lock(pool.m);
+        if (io && pool.idle.size() < kIdleIos && io->bytes <= kIdlePinned) pool.idle.push_back(io);
+        else if (io) gone.push_back(io);
+        if (--pool.contexts == 0) {
+            gone.insert(gone.end(), pool.idle.begin(), pool.idle.end());
+            pool.idle.clear();
+        }
+    }
+    for (HostIo* g : gone) host_io_free(g);
+}
+
+bool ensure_pinned(lmgpu_ctx* ctx, size_t bytes) {
+    if (!ctx->io && !(ctx->io = host_io_acquire())) return false;
+    HostIo& io = *ctx->io;
+    if (bytes <= io.bytes) return true;
+    size_t room = size_t(64) << 10;  // small needs in powers of two, to grow seldom
+    while (room < bytes && room < (size_t(4) << 20)) room *= 2;
+    bytes = std::max(bytes, room);
+    if (io.pinned) (void)hipHostFree(io.pinned);
+    io.pinned = nullptr;
+    io.bytes = 0;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocPortable) != hipSuccess || !p) {
+        (void)hipGetLastError();
+        return false;
+    }
+    io.pinned = p;
+    io.bytes = bytes;
+    return true;
+}
+
+bool ensure_io_events(lmgpu_ctx* ctx) {
+    for (hipEvent_t& ev : ctx->io_events)
+        if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+            ev = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
+    return true;
+}
+
+// Results on their way to the caller: a ring of kReadSlots pinned slots of kReadSlot bytes, each
+// copied out by the host threads while the next ones are on the link (57 GB/s).  Into pageable
+// memory the runtime copies with one thread: the FP64 film of a 1920 x 1080 render (50 MB) took
+// 4.8 ms, 1 to 3 so (the caller's pages are made on the way); a raycast of 1280 x 720 (11 MB), its
+// kernel included, 0.89 -> 0.51 ms.  Slots of 512 KB: 0.83 ms, a copy has its own cost on the link.
+hipError_t read_back(lmgpu_ctx* ctx, void* dst, const void* src, size_t bytes) {
+    const hipStream_t s = ctx->stream;
+    const size_t chunks = (bytes + kReadSlot - 1) / kReadSlot;
+    if (!ensure_pinned(ctx, kPinnedWords + std::min(bytes, kReadSlots * kReadSlot)) || !ensure_io_events(ctx)) {
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    }
+    char* pin = static_cast<char*>(ctx->io->pinned) + kPinnedWords;
+    auto size = [&](size_t c) { return std::min(kReadSlot, bytes - c * kReadSlot); };
+    size_t sent = 0;
+    hipError_t e = hipSuccess;
+    for (size_t c = 0; c < chunks && e == hipSuccess; c++) {
+        for (; sent < chunks && sent < c + kReadSlots && e == hipSuccess; sent++) {
+            e = hipMemcpyAsync(pin + sent % kReadSlots * kReadSlot, static_cast<const char*>(src) + sent * kReadSlot,
+                               size(sent), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipEventRecord(ctx->io_events[sent % kReadSlots], s);
+        }
+        if (e == hipSuccess) e = hipEventSynchronize(ctx->io_events[c % kReadSlots]);
+        if (e != hipSuccess) break;
+        const CopyJob job{static_cast<char*>(dst) + c * kReadSlot, pin + c % kReadSlots * kReadSlot, size(c)};
+        ctx->io->team.run(&job, 1);
+    }
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);
+    return e;
 }
 
 }  // namespace lmgpu
@@ -184,11 +288,14 @@ lmgpu_status lmgpu_create(int device, lmgpu_ctx** out) {
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev0);
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev1);
+    if (e == hipSuccess) e = hipEventCreate(&ctx->run0);
+    if (e == hipSuccess) e = hipEventCreate(&ctx->run1);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&ctx->num_cus, hipDeviceAttributeMultiprocessorCount, device);
     if (e != hipSuccess) {
         delete ctx;
         return LMGPU_ERR_HIP;
     }
+    host_io_context();
     ctx->stream = ctx->own_stream;
     ctx->env.index = -1;
     void* counters = nullptr;
@@ -221,7 +328,8 @@ lmgpu_status lmgpu_destroy(lmgpu_ctx* ctx) {
     free_buf(ctx->lights);
     free_buf(ctx->light_tris);
     dev_free(ctx->trace_staging);
-    if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
+    for (hipEvent_t ev : ctx->io_events)
+        if (ev) (void)hipEventDestroy(ev);
     for (hipStream_t cs : ctx->copy_streams)
         if (cs) (void)hipStreamDestroy(cs);
     dev_free(ctx->count_buf);
@@ -233,7 +341,10 @@ lmgpu_status lmgpu_destroy(lmgpu_ctx* ctx) {
     dev_free(ctx->order_buf);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
+    if (ctx->run0) (void)hipEventDestroy(ctx->run0);
+    if (ctx->run1) (void)hipEventDestroy(ctx->run1);
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
+    host_io_release(ctx->io);
     delete ctx;
     return LMGPU_OK;
 }
@@ -571,60 +682,22 @@ lmgpu_status prepare_rays(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uint32_t n
     return LMGPU_OK;
 }
 
-// Batches of at least kPipeMinRays host rays with host results move through the device in
-// chunks of a quarter of the batch (between kPipeMinChunk and kPipeChunk rays, so that a
-// batch always has chunks to overlap), double-buffered in pinned host memory and in the
-// device staging, on three streams: uploads on one copy stream, the kernels on the context's
-// stream, read-backs on the other copy stream, so the two transfer directions and the kernels
-// overlap, while the host threads copy chunk c + 1 in from the caller's arrays and chunk
-// c - 1 out to them.  Copies
-// from pageable memory otherwise run at one host thread's memcpy rate inside the runtime,
-// one direction at a time.  Each ray is traced by the same kernels as in one batch, so the
-// results are the same.
-constexpr uint32_t kPipeChunk = 1u << 21;
+// Host rays with host results go through pinned memory.  Up to kDirectRays the kernels read and
+// write it themselves: a copy costs more than they wait for the link.  Up to kPipeMinChunk are
+// copied to the device and back in one piece each.  More move through the device in chunks of a
+// quarter of the batch (between kPipeMinChunk and kPipeChunk rays), two of them at a time in pinned memory and in the device staging, on three streams: uploads on one
+// copy stream, the kernels on the context's stream, read-backs on the other copy stream, so the
+// two transfer directions and the kernels overlap, while the host threads copy chunk c + 1 in from
+// the caller's arrays and chunk c - 1 out to them.  Each ray is traced by the same kernels as in
+// one batch, so the results are the same.
+// 81 rays 210 -> 34 us (eight copies in and four out before); 512 rays direct 36 us, copied 39; 4000
+// rays 63 and 61.  65536 rays 445 -> 255 us, 1M rays 2.7 -> 1.6 ms.
+constexpr uint32_t kDirectRays = 1024;
+constexpr uint32_t kPipeChunk = 1u << 19;
 constexpr uint32_t kPipeMinChunk = 1u << 16;
-constexpr uint32_t kPipeMinRays = 1u << 20;
-constexpr unsigned kCopyThreads = 8;
 
-struct CopyJob {
-    char* dst;
-    const char* src;
-    size_t bytes;
-};
-
-// Runs the copies with up to kCopyThreads host threads, each job cut into pieces of at
-// most 4 MB that the threads take in turn; if no thread can be started (or the piece list
-// cannot be allocated) the calling thread copies everything.
-void par_copy(const CopyJob* jobs, int njobs) {
-    constexpr size_t kPiece = size_t(4) << 20;
-    std::vector<CopyJob> pieces;
-    try {
-        for (int j = 0; j < njobs; j++)
-            for (size_t off = 0; off < jobs[j].bytes; off += kPiece)
-                pieces.push_back({jobs[j].dst + off, jobs[j].src + off, std::min(kPiece, jobs[j].bytes - off)});
-    } catch (...) {
-        for (int j = 0; j < njobs; j++) std::memcpy(jobs[j].dst, jobs[j].src, jobs[j].bytes);
-        return;
-    }
-    const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    const unsigned nt = unsigned(std::min<size_t>(pieces.size(), std::min(kCopyThreads, hw)));
-    std::atomic<size_t> next{0};
-    auto work = [&]() {
-        for (size_t i = next.fetch_add(1); i < pieces.size(); i = next.fetch_add(1))
-            std::memcpy(pieces[i].dst, pieces[i].src, pieces[i].bytes);
-    };
-    std::vector<std::thread> team;
-    try {
-        for (unsigned t = 1; t < nt; t++) team.emplace_back(work);
-    } catch (...) {
-        // fewer helpers: the pieces left over are taken by the threads that did start
-    }
-    work();
-    for (auto& th : team) th.join();
-}
-
-// Pinned host memory of at least `bytes` and the two copy streams for the pipelined path;
-// false if they cannot be had (the caller then takes the plain staged copies).
+// Pinned host memory of at least `bytes` and what the pipelined path needs besides; false if it
+// cannot be had (the caller then takes the plain staged copies).
 bool ensure_pipeline(lmgpu_ctx* ctx, size_t bytes) {
     for (hipStream_t& cs : ctx->copy_streams)
         if (!cs && hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess) {
@@ -632,18 +705,7 @@ bool ensure_pipeline(lmgpu_ctx* ctx, size_t bytes) {
             (void)hipGetLastError();
             return false;
         }
-    if (bytes <= ctx->host_pinned_bytes) return true;
-    if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
-    ctx->host_pinned = nullptr;
-    ctx->host_pinned_bytes = 0;
-    void* p = nullptr;
-    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess || !p) {
-        (void)hipGetLastError();
-        return false;
-    }
-    ctx->host_pinned = p;
-    ctx->host_pinned_bytes = bytes;
-    return true;
+    return ensure_pinned(ctx, bytes) && ensure_io_events(ctx);
 }
 
 // One result column of the pipelined path: the caller's host array and its element size.
@@ -662,27 +724,54 @@ lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, ui
     const float* src[8] = {rays->ox, rays->oy, rays->oz, rays->dx, rays->dy, rays->dz, rays->tmin, rays->tmax};
     for (int k = 0; k < 8; k++)
         if (!src[k]) return fail(ctx, LMGPU_ERR_INVALID_ARGUMENT, "ray array is NULL");
+    size_t elems = 0;
+    for (int j = 0; j < nout; j++) elems += outs[j].elem;
+    if (n <= kPipeMinChunk) {
+        const size_t in = size_t(n) * 32, out = size_t(n) * elems;
+        if (!ensure_pinned(ctx, in + out)) return LMGPU_ERR_UNSUPPORTED;
+        char* const pinned = static_cast<char*>(ctx->io->pinned);
+        char* dev = pinned;
+        CopyJob jobs[8];
+        for (int k = 0; k < 8; k++)
+            jobs[k] = {pinned + size_t(k) * n * 4, reinterpret_cast<const char*>(src[k]), size_t(n) * 4};
+        ctx->io->team.run(jobs, 8);
+        hipError_t e = hipSuccess;
+        if (n > kDirectRays) {
+            const lmgpu_status st = stage(ctx, in + out);
+            if (st != LMGPU_OK) return st;
+            dev = static_cast<char*>(ctx->trace_staging);
+            e = hipMemcpyAsync(dev, pinned, in, hipMemcpyHostToDevice, ctx->stream);
+        }
+        const float* dr[8];
+        for (int k = 0; k < 8; k++) dr[k] = reinterpret_cast<const float*>(dev + size_t(k) * n * 4);
+        char* dout[4] = {nullptr, nullptr, nullptr, nullptr};
+        size_t off = in;
+        for (int j = 0; j < nout; j++) {
+            dout[j] = dev + off;
+            jobs[j] = {static_cast<char*>(outs[j].dst), pinned + off, size_t(n) * outs[j].elem};
+            off += size_t(n) * outs[j].elem;
+        }
+        if (e == hipSuccess) e = launch(dr, n, dout);
+        if (e == hipSuccess && dev != pinned) e = hipMemcpyAsync(pinned + in, dev + in, out, hipMemcpyDeviceToHost, ctx->stream);
+        const hipError_t done = hipStreamSynchronize(ctx->stream);
+        if (e == hipSuccess) e = done;
+        if (e != hipSuccess) return hip_fail(ctx, e, what);
+        ctx->io->team.run(jobs, nout);
+        return LMGPU_OK;
+    }
     const size_t quarter = (size_t(n) + 4 * kPipeMinChunk - 1) / (4 * kPipeMinChunk) * kPipeMinChunk;
     const size_t chunk = std::min<size_t>(kPipeChunk, std::max<size_t>(kPipeMinChunk, quarter));
-    size_t out_bytes = 0;
-    for (int j = 0; j < nout; j++) out_bytes += chunk * outs[j].elem;
-    const size_t in_bytes = chunk * 4 * 8;
-    const size_t slot = (in_bytes + out_bytes + 255) / 256 * 256;
+    const size_t slot = (chunk * (32 + elems) + 255) / 256 * 256;
     if (!ensure_pipeline(ctx, 2 * slot)) return LMGPU_ERR_UNSUPPORTED;
     lmgpu_status st = stage(ctx, 2 * slot);
     if (st != LMGPU_OK) return st;
-    char* pin = static_cast<char*>(ctx->host_pinned);
+    char* pin = static_cast<char*>(ctx->io->pinned);
     char* dev = static_cast<char*>(ctx->trace_staging);
     const hipStream_t sk = ctx->stream, sin = ctx->copy_streams[0], sout = ctx->copy_streams[1];
     // start: the caller's earlier work on the context's stream; up / kdone / down: slot s's
     // upload, kernels and read-back of its latest chunk.
-    hipEvent_t start = nullptr, up[2] = {nullptr, nullptr}, kdone[2] = {nullptr, nullptr}, down[2] = {nullptr, nullptr};
-    hipError_t e = hipEventCreateWithFlags(&start, hipEventDisableTiming);
-    for (int k = 0; k < 2 && e == hipSuccess; k++) {
-        e = hipEventCreateWithFlags(&up[k], hipEventDisableTiming);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&kdone[k], hipEventDisableTiming);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&down[k], hipEventDisableTiming);
-    }
+    const hipEvent_t start = ctx->io_events[0], *up = ctx->io_events + 1, *kdone = up + 2, *down = kdone + 2;
+    hipError_t e = hipSuccess;
     // The staging buffers may still be in use by work queued earlier on the context's stream.
     if (e == hipSuccess) e = hipEventRecord(start, sk);
     if (e == hipSuccess) e = hipStreamWaitEvent(sin, start, 0);
@@ -691,14 +780,14 @@ lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, ui
     uint64_t down_first[2] = {0, 0}, down_m[2] = {0, 0};
     // Copies a finished chunk's results from pinned slot s to the caller's arrays.
     auto copy_out = [&](int s) {
-        std::vector<CopyJob> jobs;
-        size_t off = in_bytes;
+        CopyJob jobs[4];
+        size_t off = down_m[s] * 32;
         for (int j = 0; j < nout; j++) {
-            jobs.push_back({static_cast<char*>(outs[j].dst) + down_first[s] * outs[j].elem, pin + s * slot + off,
-                            size_t(down_m[s]) * outs[j].elem});
-            off += chunk * outs[j].elem;
+            jobs[j] = {static_cast<char*>(outs[j].dst) + down_first[s] * outs[j].elem, pin + s * slot + off,
+                       size_t(down_m[s]) * outs[j].elem};
+            off += down_m[s] * outs[j].elem;
         }
-        par_copy(jobs.data(), int(jobs.size()));
+        ctx->io->team.run(jobs, nout);
         down_pending[s] = false;
     };
     const uint64_t chunks = (uint64_t(n) + chunk - 1) / chunk;
@@ -716,11 +805,11 @@ lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, ui
         }
         CopyJob in[8];
         for (int k = 0; k < 8; k++)
-            in[k] = {ps + size_t(k) * chunk * 4, reinterpret_cast<const char*>(src[k] + first), size_t(m) * 4};
-        par_copy(in, 8);
+            in[k] = {ps + size_t(k) * m * 4, reinterpret_cast<const char*>(src[k] + first), size_t(m) * 4};
+        ctx->io->team.run(in, 8);
         // Upload once the slot's previous kernels have read its device rays.
         if (used[s]) e = hipStreamWaitEvent(sin, kdone[s], 0);
-        if (e == hipSuccess) e = hipMemcpyAsync(ds, ps, in_bytes, hipMemcpyHostToDevice, sin);
+        if (e == hipSuccess) e = hipMemcpyAsync(ds, ps, size_t(m) * 32, hipMemcpyHostToDevice, sin);
         if (e == hipSuccess) e = hipEventRecord(up[s], sin);
         if (e != hipSuccess) break;
         up_pending[s] = true;
@@ -729,12 +818,12 @@ lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, ui
         if (e == hipSuccess && used[s]) e = hipStreamWaitEvent(sk, down[s], 0);
         if (e != hipSuccess) break;
         const float* dr[8];
-        for (int k = 0; k < 8; k++) dr[k] = reinterpret_cast<const float*>(ds + size_t(k) * chunk * 4);
+        for (int k = 0; k < 8; k++) dr[k] = reinterpret_cast<const float*>(ds + size_t(k) * m * 4);
         char* dout[4] = {nullptr, nullptr, nullptr, nullptr};
-        size_t off = in_bytes;
+        size_t off = size_t(m) * 32;
         for (int j = 0; j < nout; j++) {
             dout[j] = ds + off;
-            off += chunk * outs[j].elem;
+            off += size_t(m) * outs[j].elem;
         }
         e = launch(dr, m, dout);
         if (e == hipSuccess) e = hipEventRecord(kdone[s], sk);
@@ -748,7 +837,7 @@ lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, ui
             copy_out(t);
         }
         e = hipStreamWaitEvent(sout, kdone[s], 0);
-        if (e == hipSuccess) e = hipMemcpyAsync(ps + in_bytes, ds + in_bytes, out_bytes, hipMemcpyDeviceToHost, sout);
+        if (e == hipSuccess) e = hipMemcpyAsync(ps + size_t(m) * 32, ds + size_t(m) * 32, m * elems, hipMemcpyDeviceToHost, sout);
         if (e == hipSuccess) e = hipEventRecord(down[s], sout);
         if (e != hipSuccess) break;
         down_pending[s] = true;
@@ -765,12 +854,6 @@ lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, ui
         (void)hipStreamSynchronize(sin);
         (void)hipStreamSynchronize(sk);
         (void)hipStreamSynchronize(sout);
-    }
-    if (start) (void)hipEventDestroy(start);
-    for (int k = 0; k < 2; k++) {
-        if (up[k]) (void)hipEventDestroy(up[k]);
-        if (kdone[k]) (void)hipEventDestroy(kdone[k]);
-        if (down[k]) (void)hipEventDestroy(down[k]);
     }
     if (e != hipSuccess) return hip_fail(ctx, e, what);
     return LMGPU_OK;
@@ -796,7 +879,7 @@ lmgpu_status lmgpu_trace_closest(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uin
     if (!hits->t || !hits->b0 || !hits->b1 || !hits->prim)
         return fail(ctx, LMGPU_ERR_INVALID_ARGUMENT, "lmgpu_trace_closest: NULL hit array");
     const bool refine = (flags & LMGPU_TRACE_REFINE_FP64) != 0;
-    if (!rays->device && !hits->device && n >= kPipeMinRays) {
+    if (!rays->device && !hits->device) {
         const HostOut outs[4] = {{hits->t, 4}, {hits->b0, 4}, {hits->b1, 4}, {hits->prim, 4}};
         s = trace_host_pipelined(
             ctx, rays, n, outs, 4,
@@ -873,7 +956,7 @@ lmgpu_status lmgpu_trace_any(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uint32_
     lmgpu_status s = check_trace(ctx, rays, occluded);
     if (s != LMGPU_OK) return s;
     if (n == 0) return LMGPU_OK;
-    if (!rays->device && !occluded_on_device && n >= kPipeMinRays) {
+    if (!rays->device && !occluded_on_device) {
         const HostOut outs[1] = {{occluded, 1}};
         s = trace_host_pipelined(
             ctx, rays, n, outs, 1,

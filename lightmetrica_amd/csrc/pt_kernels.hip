@@ -1761,6 +1761,10 @@ struct Pipeline {
     }
 };
 
+// A film of up to this many bytes is resolved into pinned host memory: the link takes it as fast as
+// a copy would, without the copy's launch.
+constexpr size_t kDirectFilm = (size_t(1) << 20) - kPinnedWords;
+
 lmgpu_status run_raycast(lmgpu_ctx* ctx, lmgpu_film* film) {
     if (!ctx->has_bvh) return fail(ctx, LMGPU_ERR_NO_BVH, "lmgpu_raycast_render: build the BVH first");
     if (!ctx->has_shading || !ctx->has_camera)
@@ -1802,12 +1806,8 @@ lmgpu_status run_raycast(lmgpu_ctx* ctx, lmgpu_film* film) {
                                static_cast<float*>(out_dev));
     });
     if (e != hipSuccess) return hip_fail(ctx, e, "k_raycast");
-    if (!film->device) {
-        e = hipMemcpyAsync(film->data, out_dev, out_bytes, hipMemcpyDeviceToHost, s);
-        if (e != hipSuccess) return hip_fail(ctx, e, "raycast readback");
-    }
-    e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return hip_fail(ctx, e, "raycast synchronize");
+    e = film->device ? hipStreamSynchronize(s) : read_back(ctx, film->data, out_dev, out_bytes);
+    if (e != hipSuccess) return hip_fail(ctx, e, "raycast readback");
     return LMGPU_OK;
 }
 
@@ -1833,7 +1833,15 @@ lmgpu_status run_pt(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_film* film, 
     const size_t out_elem = film->precision == LMGPU_FILM_FP64 ? 8 : 4;
     const size_t out_bytes = nval * out_elem;
     void* out_dev = film->data;
-    if (!film->device) {
+    // The pinned memory is grown here, before it holds the words.
+    const bool small = !film->device && out_bytes <= kDirectFilm;
+    const bool pinned = ensure_pinned(ctx, kPinnedWords + (film->device ? 0 : std::min(out_bytes, kReadSlots * kReadSlot)));
+    const bool direct = small && pinned;
+    unsigned long long words_here[4];
+    void* const words = pinned ? ctx->io->pinned : words_here;
+    if (direct) {
+        out_dev = static_cast<char*>(ctx->io->pinned) + kPinnedWords;
+    } else if (!film->device) {
         st = ensure(ctx, &ctx->film_out_staging, &ctx->film_out_staging_bytes, out_bytes, "film staging");
         if (st != LMGPU_OK) return st;
         out_dev = ctx->film_out_staging;
@@ -1868,10 +1876,7 @@ lmgpu_status run_pt(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_film* film, 
     }
 
     hipStream_t s = ctx->stream;
-    hipEvent_t r0, r1;
-    (void)hipEventCreate(&r0);
-    (void)hipEventCreate(&r1);
-    (void)hipEventRecord(r0, s);
+    (void)hipEventRecord(ctx->run0, s);
     hipLaunchKernelGGL(k_zero_bytes, dim3(uint32_t((acc_bytes / 16 + 255) / 256)), dim3(256), 0, s,
                        static_cast<uint4*>(ctx->film_acc), acc_bytes / 16);
     if (splat_bytes)
@@ -1919,18 +1924,20 @@ lmgpu_status run_pt(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_film* film, 
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) st = hip_fail(ctx, e, "k_resolve");
     }
-    (void)hipEventRecord(r1, s);
+    (void)hipEventRecord(ctx->run1, s);
     unsigned long long totals[2] = {0, 0};
     if (st == LMGPU_OK) {
-        hipError_t e = hipMemcpyAsync(totals, pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess && !film->device) e = hipMemcpyAsync(film->data, out_dev, out_bytes, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        hipError_t e = hipMemcpyAsync(words, pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = film->device || direct ? hipStreamSynchronize(s) : read_back(ctx, film->data, out_dev, out_bytes);
         if (e != hipSuccess) st = hip_fail(ctx, e, "pt readback");
+        else std::memcpy(totals, words, sizeof(totals));
+        if (e == hipSuccess && direct) {
+            const CopyJob job{static_cast<char*>(film->data), static_cast<const char*>(out_dev), out_bytes};
+            ctx->io->team.run(&job, 1);
+        }
     }
     float ms = 0.f;
-    if (st == LMGPU_OK) (void)hipEventElapsedTime(&ms, r0, r1);
-    (void)hipEventDestroy(r0);
-    (void)hipEventDestroy(r1);
+    if (st == LMGPU_OK) (void)hipEventElapsedTime(&ms, ctx->run0, ctx->run1);
     if (st != LMGPU_OK) return st;
     if (stats) {
         stats->closest_rays = totals[0];
@@ -1978,10 +1985,7 @@ lmgpu_status run_pt_backward(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_adj
     }
     pl.c.film_mode = LMGPU_FILM_FP32;
 
-    hipEvent_t r0, r1;
-    (void)hipEventCreate(&r0);
-    (void)hipEventCreate(&r1);
-    (void)hipEventRecord(r0, s);
+    (void)hipEventRecord(ctx->run0, s);
     hipLaunchKernelGGL(k_zero_bytes, dim3(uint32_t(((g_bytes + 16) / 16 + 255) / 256)), dim3(256), 0, s,
                        reinterpret_cast<uint4*>(grad), (g_bytes + 16) / 16);
     hipLaunchKernelGGL(k_zero_u32, dim3(5), dim3(256), 0, s, pl.b.counters, (4096u + 64u) / 4u);
@@ -2017,23 +2021,28 @@ lmgpu_status run_pt_backward(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_adj
         e = hipGetLastError();
         if (e != hipSuccess) st = hip_fail(ctx, e, "k_scale_f64");
     }
-    (void)hipEventRecord(r1, s);
+    (void)hipEventRecord(ctx->run1, s);
     unsigned long long totals[2] = {0, 0};
     double hs[2] = {0.0, 0.0};
+    char words_here[sizeof(hs) + sizeof(totals)];
+    char* const words = ensure_pinned(ctx, kPinnedWords) ? static_cast<char*>(ctx->io->pinned) : words_here;
     if (st == LMGPU_OK) {
         const hipMemcpyKind k = adj->grad_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
         e = hipMemcpyAsync(adj->d_albedo, grad, size_t(ctx->num_materials) * 24, k, s);
         if (e == hipSuccess && ctx->num_lights > 0)
             e = hipMemcpyAsync(adj->d_emission, pl.c.grad_light, size_t(ctx->num_lights) * 24, k, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(hs, sums, sizeof(hs), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(totals, pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(words, sums, sizeof(hs), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(words + sizeof(hs), pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) st = hip_fail(ctx, e, "adjoint readback");
+        else {
+            std::memcpy(hs, words, sizeof(hs));
+            std::memcpy(totals, words + sizeof(hs), sizeof(totals));
+        }
     }
     float ms = 0.f;
-    if (st == LMGPU_OK) (void)hipEventElapsedTime(&ms, r0, r1);
-    (void)hipEventDestroy(r0);
-    (void)hipEventDestroy(r1);
+    if (st == LMGPU_OK) (void)hipEventElapsedTime(&ms, ctx->run0, ctx->run1);
     if (st != LMGPU_OK) return st;
     adj->replay_residual = hs[0] > 0.0 ? hs[1] / hs[0] : 0.0;
     if (stats) {
