@@ -56,6 +56,7 @@ constexpr uint32_t kMiss = 0xffffffffu;
 constexpr uint32_t kBlackMat = 0xffffffffu;  // the black diffuse BSDF of the environment sphere
 constexpr uint32_t kFlagDegenerate = 1u;     // previous vertex is the pinhole camera
 constexpr uint32_t kFlagSpecular = 2u;       // previous BSDF sample was specular
+constexpr uint32_t kFlagLit = 4u;            // pt render: the path has gathered light (aux)
 
 // GeneralizedBSDFType bits (include/lightmetrica/generalizedbsdf.h:34-72)
 constexpr int kDiffuseReflection = 1 << 0;
@@ -95,14 +96,22 @@ struct PTConsts {
     int renderer;
 };
 
-// Path queue: structure of arrays of 16-byte records.
+// Path queue: structure of arrays of 16-byte records.  The shading stages are bound by their traffic,
+// so a vertex moves 48 bytes in and 48 out beside its hit, and `aux` only where it holds something:
+// with five full records each the shading of a training step (59M vertices, twice) took 4.29 ms, now
+// 4.09, the camera stage 0.80 -> 0.57, the whole step 16.8 -> 15.9 ms.  A segment's rays have one tmin, which the host passes.
 struct Queue {
-    float4* ray_o;  // o.xyz, tmin
-    float4* ray_d;  // d.xyz, pdf of the BSDF sample that produced the ray
-    float4* thr;    // throughput.xyz
-    float4* aux;    // pt: L.xyz;  pt.direct / pt.mis: shading normal of the ray origin
-    uint4* meta;    // sample index in batch, vertex count n | flags << 16, stream dimension, pixel
+    float4* ray_o;  // o.xyz, throughput x
+    float4* ray_d;  // d.xyz, throughput y
+    uint4* meta;    // sample index in batch, path_bits, pixel, throughput z
+    float4* aux;    // pt render: L.xyz of a path that has kFlagLit;  pt.mis: shading normal of the ray
+                    // origin, pdf of the BSDF sample that produced the ray
 };
+
+// Vertex count n <= kMaxSegments, flags and stream dimension (at most a dozen numbers a vertex).
+__device__ __forceinline__ uint32_t path_bits(uint32_t n, uint32_t flags, uint32_t dim) {
+    return n | flags << 8 | dim << 16;
+}
 
 struct ShadowQueue {
     float4* o;      // origin, tmax
@@ -665,13 +674,11 @@ __device__ __forceinline__ const XformRecord* stage_xform(const PTConsts& c, Xfo
     return lds;
 }
 
-__device__ __forceinline__ void store_path(const Queue& q, uint32_t slot, V3 o, float tmin, V3 d, float pdf, V3 T,
-                                           V3 aux, uint32_t sid, uint32_t n_flags, uint32_t dim, uint32_t pixel) {
-    q.ray_o[slot] = make_float4(o.x, o.y, o.z, tmin);
-    q.ray_d[slot] = make_float4(d.x, d.y, d.z, pdf);
-    q.thr[slot] = make_float4(T.x, T.y, T.z, 0.f);
-    q.aux[slot] = make_float4(aux.x, aux.y, aux.z, 0.f);
-    q.meta[slot] = make_uint4(sid, n_flags, dim, pixel);
+__device__ __forceinline__ void store_path(const Queue& q, uint32_t slot, V3 o, V3 d, V3 T, uint32_t sid, uint32_t bits,
+                                           uint32_t pixel) {
+    q.ray_o[slot] = make_float4(o.x, o.y, o.z, T.x);
+    q.ray_d[slot] = make_float4(d.x, d.y, d.z, T.y);
+    q.meta[slot] = make_uint4(sid, bits, pixel, __float_as_uint(T.z));
 }
 
 // Interleaves the bits of x and y (each < 2^16): the Z-order (Morton) index of (x, y).
@@ -737,8 +744,8 @@ __global__ __launch_bounds__(kPTBlock) void k_gen(PTConsts c, Queue out, uint32_
         float pdf;
         const V3 d = cam_direction(c.cam, r0, r1, pdf);
         const uint32_t pixel = pixel_of(c.cam, r0, r1);
-        store_path(out, slot0, cam_p, 0.f, d, pdf, v3s(1.f), v3s(0.f), i, 1u, rng.dim, pixel);
-        if (kMode == kRender && c.record) c.record[i] = make_float4(0.f, 0.f, 0.f, __uint_as_float(pixel));
+        // The path's record is written where it ends.
+        store_path(out, slot0, cam_p, d, v3s(1.f), i, path_bits(1u, 0u, rng.dim), pixel);
         return;
     }
     const bool mis = c.renderer == LMGPU_PT_MIS;
@@ -777,8 +784,10 @@ __global__ __launch_bounds__(kPTBlock) void k_gen(PTConsts c, Queue out, uint32_
         pixel = pixel_of(c.cam, rx, ry);
     }
     const uint32_t slot = block_append<1>(live_count, alive);
-    if (alive)
-        store_path(out, slot, cam_p, kEps, d, pdf, T, v3s(0.f), i, 1u | (kFlagDegenerate << 16), rng.dim, pixel);
+    if (alive) {
+        store_path(out, slot, cam_p, d, T, i, path_bits(1u, kFlagDegenerate, rng.dim), pixel);
+        if (mis) out.aux[slot] = make_float4(0.f, 0.f, 0.f, pdf);
+    }
     if (kMode == kRender && c.record && valid) {
         c.record[2ull * i] = make_float4(0.f, 0.f, 0.f, __uint_as_float(alive ? pixel : kNoPixel));
         c.record[2ull * i + 1] = make_float4(0.f, 0.f, 0.f, __uint_as_float(kNoPixel));
@@ -795,9 +804,10 @@ __global__ __launch_bounds__(kPTBlock) void k_gen(PTConsts c, Queue out, uint32_
 // Extension rays: closest hit of every live path (persistent, refilling lanes).
 struct QueueSource {
     Queue q;
+    float tmin;
     __device__ __forceinline__ RayIn operator()(uint32_t i) const {
         const float4 o = q.ray_o[i], d = q.ray_d[i];
-        return RayIn{o.x, o.y, o.z, d.x, d.y, d.z, o.w, kInf};
+        return RayIn{o.x, o.y, o.z, d.x, d.y, d.z, tmin, kInf};
     }
 };
 
@@ -841,12 +851,12 @@ __device__ __forceinline__ void add_wave_counts(const TraceCounters& cnt, unsign
 // kCount (lmgpu_enable_counting): also counts node visits and triangle tests into `counts`.
 // 6 waves per SIMD, as the LDS stack allows (the bound keeps the kernel within 80 VGPRs).
 template <bool kCount = false>
-__global__ __launch_bounds__(kTraceBlock, 6) void k_extend(BvhDev bvh, Queue q,
+__global__ __launch_bounds__(kTraceBlock, 6) void k_extend(BvhDev bvh, Queue q, float tmin,
                                                         const uint32_t* __restrict__ count, uint32_t* next,
                                                         float4* __restrict__ hits, unsigned long long* counts) {
     __shared__ QueueShared<true> sm;
     const uint32_t n = *count;
-    QueueSource src{q};
+    QueueSource src{q, tmin};
     HitSink sink{bvh.tris, hits};
     TraceCounters cnt{0, 0};
     if (n <= kGroup64Rays) trace_grouped<false, kCount, 64>(bvh, n, sm.group64, src, sink, cnt);
@@ -934,7 +944,7 @@ __device__ __forceinline__ uint32_t lanes_per_path(uint32_t count) {
 // block's gradient table collects many paths before it is flushed): a late segment's
 // nearly empty queue then costs a launch of that grid, not of one block per queue slot.
 template <int kMode, bool kFuse = false>
-__global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, const uint32_t* __restrict__ in_count,
+__global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, float tmin, const uint32_t* __restrict__ in_count,
                                                        const float4* __restrict__ hits, Queue out,
                                                        uint32_t* out_count) {
     const uint32_t count = *in_count;
@@ -952,33 +962,40 @@ __global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, con
     const bool valid = i < count;
     const bool lead = sub == 0u;  // the lane of the group that applies the path's effects
     const uint32_t j = valid ? i : 0u;  // invalid lanes read slot 0 and discard it
-    const float4 ro = in.ray_o[j], rd = in.ray_d[j], th = in.thr[j], ax = in.aux[j];
+    const float4 ro = in.ray_o[j], rd = in.ray_d[j];
     const uint4 meta = in.meta[j];
     const V3 o = v3(ro.x, ro.y, ro.z), d = v3(rd.x, rd.y, rd.z);
-    V3 T = v3(th.x, th.y, th.z), L = v3(ax.x, ax.y, ax.z);
-    int n = int(meta.y & 0xffffu);
+    V3 T = v3(ro.w, rd.w, __uint_as_float(meta.w)), L = v3s(0.f);
+    int n = int(meta.y & 0xffu);
+    if (kMode == kRender && (meta.y >> 8 & kFlagLit)) {
+        const float4 ax = in.aux[j];
+        L = v3(ax.x, ax.y, ax.z);
+    }
     SampleStream rng;
-    rng.init(c.seed, c.base + meta.x, meta.z);
+    rng.init(c.seed, c.base + meta.x, meta.y >> 16);
     // kFuse (scenes of at most kBruteMaxTris triangles): the segment's ray is traced here
     // instead of by a separate extension launch.
-    const RayIn ray{ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, ro.w, kInf};
+    const RayIn ray{ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, tmin, kInf};
     const float4 hit = kFuse ? xform_closest(xf, c.ntris, ray, valid, group, sub) : hits[j];
     // Every lane of a group shades the same path the same way; the lead lane applies it.
-    const PtVertex v = pt_vertex(c, o, d, ro.w, hit, valid, T, n, rng);
+    const PtVertex v = pt_vertex(c, o, d, tmin, hit, valid, T, n, rng);
     if (v.emits) {
         if (kMode == kRender) L = L + v.emit;
-        else if (lead) contribute<kMode>(c, meta.x, meta.w, v.emit);
+        else if (lead) contribute<kMode>(c, meta.x, meta.z, v.emit);
     }
     const bool alive = v.alive && lead;
     if (kMode == kAdjGrad && lead) {
-        if (v.emits) grad_emission(gc, c, meta.w, v.Le_w, v.s.light);
+        if (v.emits) grad_emission(gc, c, meta.z, v.Le_w, v.s.light);
         if (alive && v.s.mat != kBlackMat) grad_material(gc, c, meta.x, v.s.mat, v.m.R);
     }
     const uint32_t slot = block_append<0>(out_count, alive);
-    if (alive) store_path(out, slot, v.s.p, kEps, v.wo, v.pdf, T, L, meta.x, uint32_t(n), rng.dim, meta.w);
-    else if (kMode == kRender && valid && lead) {
-        film_add(c, meta.w, L);
-        if (c.record) c.record[meta.x] = make_float4(L.x, L.y, L.z, __uint_as_float(meta.w));
+    if (alive) {
+        const bool lit = kMode == kRender && (L.x != 0.f || L.y != 0.f || L.z != 0.f);
+        store_path(out, slot, v.s.p, v.wo, T, meta.x, path_bits(uint32_t(n), lit ? kFlagLit : 0u, rng.dim), meta.z);
+        if (lit) out.aux[slot] = make_float4(L.x, L.y, L.z, 0.f);
+    } else if (kMode == kRender && valid && lead) {
+        film_add(c, meta.z, L);
+        if (c.record) c.record[meta.x] = make_float4(L.x, L.y, L.z, __uint_as_float(meta.z));
     }
     };
     for (uint32_t tile = blockIdx.x; tile * per_tile < count; tile += gridDim.x) tile_body(tile);
@@ -991,7 +1008,7 @@ __global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, con
 // 5 waves per SIMD: the bound keeps the kernel within 96 VGPRs (it needed 97, i.e. 4 waves;
 // the room's pt.direct / pt.mis renders 3 % faster).
 template <int kMode, bool kFuse = false>
-__global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in, const uint32_t* __restrict__ in_count,
+__global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in, float tmin, const uint32_t* __restrict__ in_count,
                                                         const float4* __restrict__ hits, Queue out,
                                                         uint32_t* out_count, ShadowQueue sq, uint32_t* shadow_count) {
     const uint32_t count = *in_count;
@@ -1011,20 +1028,21 @@ __global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in,
     const bool lead = sub == 0u;
     const uint32_t j = valid ? i : 0u;  // invalid lanes read slot 0 and discard it
     const bool mis = c.renderer == LMGPU_PT_MIS;
-    const float4 ro = in.ray_o[j], rd = in.ray_d[j], th = in.thr[j], ax = in.aux[j];
+    const float4 ro = in.ray_o[j], rd = in.ray_d[j];
     const uint4 meta = in.meta[j];
     const V3 o = v3(ro.x, ro.y, ro.z), d = v3(rd.x, rd.y, rd.z);
-    V3 T = v3(th.x, th.y, th.z);
-    int n = int(meta.y & 0xffffu);
-    const uint32_t flags = meta.y >> 16;
+    V3 T = v3(ro.w, rd.w, __uint_as_float(meta.w));
+    const uint32_t pixel = meta.z;
+    int n = int(meta.y & 0xffu);
+    const uint32_t flags = meta.y >> 8 & 0xffu;
     SampleStream rng;
-    rng.init(c.seed, c.base + meta.x, meta.z);
+    rng.init(c.seed, c.base + meta.x, meta.y >> 16);
     Surf s;
     s.mat = kBlackMat;
     s.light = -1;
-    const RayIn ray{ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, ro.w, kInf};
+    const RayIn ray{ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, tmin, kInf};
     const float4 hit = kFuse ? xform_closest(xf, c.ntris, ray, valid, group, sub) : hits[j];
-    bool alive = valid && surface_at(c, o, d, ro.w, hit, s);
+    bool alive = valid && surface_at(c, o, d, tmin, hit, s);
     bool emits = false;
     V3 Le_w = v3s(0.f);
     if (alive && s.light >= 0) {
@@ -1035,6 +1053,7 @@ __global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in,
             Le_w = T * v3s(LeD) * kPi;
         } else if (mis) {
             // GeneralizedGeometryTerm(previous vertex, hit) and the light-sampling pdf
+            const float4 ax = in.aux[j];
             V3 dv = s.p - o;
             const float l2 = dot(dv, dv);
             const float l = sqrtf(l2);
@@ -1046,13 +1065,13 @@ __global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in,
             const float pos_pdf = s.light == c.env.index ? c.env.inv_area
                                                          : reinterpret_cast<const float4*>(c.lights)[2 * s.light + 1].z;
             const float pdf_dl = G == 0.f ? 0.f : (1.f / float(c.num_lights)) * pos_pdf / G;
-            const float w = rd.w / (rd.w + pdf_dl);
+            const float w = ax.w / (ax.w + pdf_dl);
             emits = true;
             Le_w = T * v3s(LeD) * kPi * w;
         }
-        if (emits && lead) contribute<kMode>(c, meta.x, meta.w, Le_w * Le);
+        if (emits && lead) contribute<kMode>(c, meta.x, pixel, Le_w * Le);
     }
-    if (kMode == kAdjGrad && emits && lead) grad_emission(gc, c, meta.w, Le_w, s.light);
+    if (kMode == kAdjGrad && emits && lead) grad_emission(gc, c, pixel, Le_w, s.light);
     if (alive) {
         n++;
         if (c.max_pv != -1 && n >= c.max_pv) alive = false;
@@ -1063,7 +1082,7 @@ __global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in,
     v.camera = false;
     v.wi = -d;
     v.m = alive ? mat_info(c, s.mat) : MatInfo{LMGPU_BSDF_MIRROR, v3s(0.f)};
-    const ShadowRec rec = nee(c, v, T, n, meta.w, rng, mis, alive && mat_nondelta(v.m), kMode != kRender);
+    const ShadowRec rec = nee(c, v, T, n, pixel, rng, mis, alive && mat_nondelta(v.m), kMode != kRender);
     if constexpr (kMode == kRender && kFuse) {
         (void)block_append<0>(shadow_count, rec.emit && lead);  // counts the shadow rays traced
         if (shadow_visible(c, xf, rec, group, sub) && lead) add_connection<false>(c, rec, meta.x);
@@ -1090,8 +1109,9 @@ __global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in,
     alive = alive && lead;
     const uint32_t slot = block_append<1>(out_count, alive);
     if (alive) {
-        const uint32_t nf = uint32_t(n) | ((type & (1 << 2)) ? (kFlagSpecular << 16) : 0u);
-        store_path(out, slot, s.p, kEps, wo, pdf, T, s.f.sn, meta.x, nf, rng.dim, meta.w);
+        const uint32_t bits = path_bits(uint32_t(n), (type & (1 << 2)) ? kFlagSpecular : 0u, rng.dim);
+        store_path(out, slot, s.p, wo, T, meta.x, bits, pixel);
+        if (mis) out.aux[slot] = make_float4(s.f.sn.x, s.f.sn.y, s.f.sn.z, pdf);
     }
     };
     for (uint32_t tile = blockIdx.x; tile * per_tile < count; tile += gridDim.x) tile_body(tile);
@@ -1451,14 +1471,13 @@ static void connection_rect(const lmgpu_ctx* ctx, uint32_t r[4]) {
     }
 }
 
-static size_t queue_bytes(uint32_t cap) { return size_t(cap) * 16 * 5; }
+static size_t queue_bytes(uint32_t cap) { return size_t(cap) * 16 * 4; }
 
 static void carve(void* base, uint32_t cap, PTBuffers& b) {
     char* p = static_cast<char*>(base);
     for (int k = 0; k < 2; k++) {
         b.q[k].ray_o = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
         b.q[k].ray_d = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
-        b.q[k].thr = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
         b.q[k].aux = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
         b.q[k].meta = reinterpret_cast<uint4*>(p); p += size_t(cap) * 16;
     }
@@ -1475,7 +1494,7 @@ static void carve(void* base, uint32_t cap, PTBuffers& b) {
 static size_t pt_bytes(uint32_t cap) { return 2 * queue_bytes(cap) + size_t(cap) * (16 * 4 + 8) + 4096 + 64; }
 
 // Paths in flight per batch when the caller leaves it to the library: the whole render in one
-// batch, up to 2^26 paths (15.6 GB of queues) and a quarter of the device memory free for the
+// batch, up to 2^26 paths (13.4 GB of queues) and a quarter of the device memory free for the
 // queues and the adjoint's per-sample totals.  Wide batches keep every segment's launch full:
 // with RR the late segments of a 2^21-path batch hold a few hundred thousand paths, fewer than
 // the persistent traversal grid has lanes.
@@ -1719,31 +1738,32 @@ struct Pipeline {
         for (int k = 0; k < segments; k++) {
             const Queue& qi = b.q[k & 1];
             const Queue& qo = b.q[(k + 1) & 1];
+            const float tmin = is_pt && k == 0 ? 0.f : kEps;  // pt's camera rays (pathtrace.cpp:187-192) start at 0
             // Scenes of at most kBruteMaxTris triangles: the shading kernel traces the segment's
             // rays itself (kFuse), so there is no extension launch and no hit record.
             if (!brute) {
                 e = timed(ctx, kKExtend, [&]() {
                     if (counting)
-                        hipLaunchKernelGGL(k_extend<true>, grid_t, dim3(kTraceBlock), 0, s, c.bvh, qi,
+                        hipLaunchKernelGGL(k_extend<true>, grid_t, dim3(kTraceBlock), 0, s, c.bvh, qi, tmin,
                                            b.counters + k, b.counters + 2 * kMaxSegments + k, b.hits, ext_counts);
                     else
-                        hipLaunchKernelGGL(k_extend<false>, grid_t, dim3(kTraceBlock), 0, s, c.bvh, qi,
+                        hipLaunchKernelGGL(k_extend<false>, grid_t, dim3(kTraceBlock), 0, s, c.bvh, qi, tmin,
                                            b.counters + k, b.counters + 2 * kMaxSegments + k, b.hits, ext_counts);
                 });
                 if (e != hipSuccess) return hip_fail(ctx, e, "k_extend");
             }
             e = timed(ctx, kKShade, [&]() {
                 if (is_pt && brute)
-                    hipLaunchKernelGGL((k_shade_pt<kMode, true>), grid_s, dim3(kPTBlock), 0, s, c, qi, b.counters + k,
+                    hipLaunchKernelGGL((k_shade_pt<kMode, true>), grid_s, dim3(kPTBlock), 0, s, c, qi, tmin, b.counters + k,
                                        b.hits, qo, b.counters + k + 1);
                 else if (is_pt)
-                    hipLaunchKernelGGL(k_shade_pt<kMode>, grid_s, dim3(kPTBlock), 0, s, c, qi, b.counters + k, b.hits,
+                    hipLaunchKernelGGL(k_shade_pt<kMode>, grid_s, dim3(kPTBlock), 0, s, c, qi, tmin, b.counters + k, b.hits,
                                        qo, b.counters + k + 1);
                 else if (brute)
-                    hipLaunchKernelGGL((k_shade_nee<kMode, true>), grid_s, dim3(kPTBlock), 0, s, c, qi, b.counters + k,
+                    hipLaunchKernelGGL((k_shade_nee<kMode, true>), grid_s, dim3(kPTBlock), 0, s, c, qi, tmin, b.counters + k,
                                        b.hits, qo, b.counters + k + 1, b.sq, b.counters + kMaxSegments + k + 1);
                 else
-                    hipLaunchKernelGGL(k_shade_nee<kMode>, grid_s, dim3(kPTBlock), 0, s, c, qi, b.counters + k,
+                    hipLaunchKernelGGL(k_shade_nee<kMode>, grid_s, dim3(kPTBlock), 0, s, c, qi, tmin, b.counters + k,
                                        b.hits, qo, b.counters + k + 1, b.sq, b.counters + kMaxSegments + k + 1);
             });
             if (e != hipSuccess) return hip_fail(ctx, e, "k_shade");
