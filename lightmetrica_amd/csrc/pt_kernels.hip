@@ -167,15 +167,19 @@ __device__ __forceinline__ uint32_t block_append(uint32_t* counter, bool pred) {
     return base + wave_off[wave] + uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
 }
 
+// The rounding error of the FP32 sum old + x.
+__device__ __forceinline__ float two_sum_error(float old, float x) {
+    const float s = old + x;  // the value the atomic stored (round to nearest even)
+    const float bp = s - old;
+    return (old - (s - bp)) + (x - bp);
+}
+
 // Compensated FP32 accumulation: the atomic returns the sum it replaced, so the rounding
 // error of the stored sum is recovered exactly by TwoSum (Knuth, TAOCP vol. 2, 4.2.2) and
 // accumulated in a second FP32 array; the film value is sum + error.
 __device__ __forceinline__ void comp_add(float* sum, float* err, float x) {
     if (x == 0.f) return;
-    const float old = unsafeAtomicAdd(sum, x);
-    const float s = old + x;  // the value the atomic stored (round to nearest even)
-    const float bp = s - old;
-    const float e = (old - (s - bp)) + (x - bp);
+    const float e = two_sum_error(unsafeAtomicAdd(sum, x), x);
     if (e != 0.f) unsafeAtomicAdd(err, e);
 }
 
@@ -298,8 +302,8 @@ __device__ __forceinline__ void gc_init(GradCache& g) {
     __syncthreads();
 }
 
-__device__ __forceinline__ void gc_add(GradCache& g, const PTConsts& c, uint32_t key, double x, double y, double z) {
-    if (x == 0.0 && y == 0.0 && z == 0.0) return;
+// Adds to the sums of `key`; false if there is no slot for it.
+__device__ __forceinline__ bool gc_put(GradCache& g, uint32_t key, double x, double y, double z) {
     uint32_t slot = (key * 2654435761u) >> 23;  // 9 bits: kGradSlots = 512
     for (int probe = 0; probe < kGradProbes; probe++) {
         uint32_t k = __hip_atomic_load(&g.keys[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -311,10 +315,16 @@ __device__ __forceinline__ void gc_add(GradCache& g, const PTConsts& c, uint32_t
             atomicAdd(&g.vals[3 * slot + 0], x);
             atomicAdd(&g.vals[3 * slot + 1], y);
             atomicAdd(&g.vals[3 * slot + 2], z);
-            return;
+            return true;
         }
         slot = (slot + 1) & (kGradSlots - 1);
     }
+    return false;
+}
+
+__device__ __forceinline__ void gc_add(GradCache& g, const PTConsts& c, uint32_t key, double x, double y, double z) {
+    if (x == 0.0 && y == 0.0 && z == 0.0) return;
+    if (gc_put(g, key, x, y, z)) return;
     double* d = grad_target(c, key);
     if (x != 0.0) unsafeAtomicAdd(d + 0, x);
     if (y != 0.0) unsafeAtomicAdd(d + 1, y);
@@ -330,6 +340,50 @@ __device__ __forceinline__ void gc_flush(GradCache& g, const PTConsts& c) {
         for (int k = 0; k < 3; k++)
             if (g.vals[3 * i + k] != 0.0) unsafeAtomicAdd(d + k, g.vals[3 * i + k]);
     }
+}
+
+// The same table over the pixels on which a tile of paths ends (keys: pixel indices), added to an
+// FP64 or compensated film once per tile and emptied.  Paths in screen-tile order end four to a
+// pixel and tile, and the film's atomics, six a path where it is compensated, took longer than all
+// the rest of the shading: 1920 x 1080 x 8 of the terrain 2.90 -> 1.22 ms compensated, 2.04 ->
+// 1.07 FP64 (0.81 without a film).  An FP32 film keeps its sums' order, and its atomics.
+__device__ __forceinline__ void film_flush(GradCache& g, const PTConsts& c) {
+    constexpr int kEach = 3 * kGradSlots / kPTBlock;
+    static_assert(kEach * kPTBlock == 3 * kGradSlots, "a thread flushes kEach values");
+    __syncthreads();
+    double x[kEach];
+    uint32_t pixel[kEach];
+    auto channel = [](int j) { return uint32_t(j * kPTBlock + int(threadIdx.x)) % 3u; };
+#pragma unroll
+    for (int j = 0; j < kEach; j++) {
+        const int i = j * kPTBlock + int(threadIdx.x);
+        pixel[j] = g.keys[i / 3];
+        x[j] = 0.0;
+        if (pixel[j] == kEmptyKey) continue;
+        x[j] = g.vals[i];
+        g.vals[i] = 0.0;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kGradSlots; i += kPTBlock) g.keys[i] = kEmptyKey;
+    if (c.film_mode == LMGPU_FILM_FP64) {
+#pragma unroll
+        for (int j = 0; j < kEach; j++)
+            if (x[j] != 0.0) unsafeAtomicAdd(static_cast<double*>(c.film) + 3ull * pixel[j] + channel(j), x[j]);
+    } else {
+        // comp_add, with all the sums' old values under way before the first is needed.
+        float old[kEach];
+#pragma unroll
+        for (int j = 0; j < kEach; j++)
+            if (x[j] != 0.0) old[j] = unsafeAtomicAdd(static_cast<float*>(c.film) + 3ull * pixel[j] + channel(j), float(x[j]));
+#pragma unroll
+        for (int j = 0; j < kEach; j++) {
+            if (x[j] == 0.0) continue;
+            const float v = float(x[j]);
+            const float e = two_sum_error(old[j], v) + float(x[j] - double(v));
+            if (e != 0.f) unsafeAtomicAdd(c.film_comp + 3ull * pixel[j] + channel(j), e);
+        }
+    }
+    __syncthreads();
 }
 
 // dL/dLe of a contribution v = w * Le (w: the contribution without Le) of light `li`.
@@ -943,7 +997,8 @@ __device__ __forceinline__ uint32_t lanes_per_path(uint32_t count) {
 // over a device-filling grid (16 blocks per CU; 4 for the gradient pass, so that each
 // block's gradient table collects many paths before it is flushed): a late segment's
 // nearly empty queue then costs a launch of that grid, not of one block per queue slot.
-template <int kMode, bool kFuse = false>
+// kTable: the film's sums go through film_flush.
+template <int kMode, bool kFuse = false, bool kTable = false>
 __global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, float tmin, const uint32_t* __restrict__ in_count,
                                                        const float4* __restrict__ hits, Queue out,
                                                        uint32_t* out_count) {
@@ -955,7 +1010,7 @@ __global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, flo
     __shared__ XformRecord xf_lds[kFuse ? kBruteMaxTrisPt : 1];
     const XformRecord* xf = kFuse ? stage_xform<kBruteMaxTrisPt>(c, xf_lds) : c.xform;
     __shared__ GradCache gc;
-    if (kMode == kAdjGrad) gc_init(gc);
+    if (kMode == kAdjGrad || kTable) gc_init(gc);
     auto tile_body = [&](uint32_t tile) {
     const uint32_t i = tile * per_tile + threadIdx.x / group;
     const uint32_t sub = threadIdx.x & (group - 1u);
@@ -994,9 +1049,10 @@ __global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, flo
         store_path(out, slot, v.s.p, v.wo, T, meta.x, path_bits(uint32_t(n), lit ? kFlagLit : 0u, rng.dim), meta.z);
         if (lit) out.aux[slot] = make_float4(L.x, L.y, L.z, 0.f);
     } else if (kMode == kRender && valid && lead) {
-        film_add(c, meta.z, L);
+        if (!kTable || is_zero(L) || !gc_put(gc, meta.z, L.x, L.y, L.z)) film_add(c, meta.z, L);
         if (c.record) c.record[meta.x] = make_float4(L.x, L.y, L.z, __uint_as_float(meta.z));
     }
+    if (kTable) film_flush(gc, c);
     };
     for (uint32_t tile = blockIdx.x; tile * per_tile < count; tile += gridDim.x) tile_body(tile);
     if (kMode == kAdjGrad) gc_flush(gc, c);
@@ -1756,6 +1812,9 @@ struct Pipeline {
                 if (is_pt && brute)
                     hipLaunchKernelGGL((k_shade_pt<kMode, true>), grid_s, dim3(kPTBlock), 0, s, c, qi, tmin, b.counters + k,
                                        b.hits, qo, b.counters + k + 1);
+                else if (is_pt && kMode == kRender && c.order && c.film_mode != LMGPU_FILM_FP32)
+                    hipLaunchKernelGGL((k_shade_pt<kMode, false, kMode == kRender>), grid_s, dim3(kPTBlock), 0, s, c, qi,
+                                       tmin, b.counters + k, b.hits, qo, b.counters + k + 1);
                 else if (is_pt)
                     hipLaunchKernelGGL(k_shade_pt<kMode>, grid_s, dim3(kPTBlock), 0, s, c, qi, tmin, b.counters + k, b.hits,
                                        qo, b.counters + k + 1);
