@@ -40,6 +40,7 @@
 #include "traverse.hpp"
 
 #include <algorithm>
+#include <type_traits>
 #include <cmath>
 #include <chrono>
 
@@ -208,7 +209,7 @@ __device__ __forceinline__ void film_add(const PTConsts& c, uint32_t pixel, V3 v
 // show the lights, so their film atomics pile onto a few cache lines and serialise there.
 // Block b adds them to replica b mod splat_k (a multiple of the 8 XCDs when at least 8, so
 // each replica is written from one XCD) of the film rectangle that the lights project to,
-// and k_splat_fold sums the replicas into the film after the last batch.  A pixel outside
+// and k_resolve adds the replicas to the film's values after the last batch.  A pixel outside
 // the rectangle (never, up to rounding) goes to the film directly.
 __device__ __forceinline__ void splat_add(const PTConsts& c, uint32_t pixel, V3 v) {
     if (v.x == 0.f && v.y == 0.f && v.z == 0.f) return;
@@ -1330,64 +1331,85 @@ __global__ void k_zero_bytes(uint4* p, size_t n16) {
     if (i < n16) p[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
+// What a render or an adjoint starts from: two accumulators and the path buffers' counters and
+// totals, cleared in one launch.  Launches are what a small render waits for, some 5 us each: 64 x 64 x 8
+// with 18 of them took 195 us, with 12 180.
+__global__ void k_clear(uint4* a, size_t na, uint4* b, size_t nb, uint32_t* words, uint32_t nw) {
+    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < na) a[i] = make_uint4(0u, 0u, 0u, 0u);
+    else if (i - na < nb) b[i - na] = make_uint4(0u, 0u, 0u, 0u);
+    if (i < nw) words[i] = 0u;
+}
+
+// Adds a batch's queue sizes to the totals, by the first wave of a launch; `out` may be `totals`.
+__device__ __forceinline__ void add_totals(const uint32_t* counters, int segments, const unsigned long long* totals,
+                                           unsigned long long* out) {
+    unsigned long long a = 0, b = 0;
+    for (int k = int(threadIdx.x); k < segments; k += 64) {
+        a += counters[k];
+        b += counters[kMaxSegments + k];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_xor(a, off, 64);
+        b += __shfl_xor(b, off, 64);
+    }
+    if (threadIdx.x == 0) {
+        out[0] = totals[0] + a;
+        out[1] = totals[1] + b;
+    }
+}
+
+// After every batch but the last, whose counters the run's last kernel adds.
 __global__ void k_accumulate_totals(const uint32_t* counters, int segments, unsigned long long* totals) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        unsigned long long a = 0, b = 0;
-        for (int k = 0; k < segments; k++) {
-            a += counters[k];
-            b += counters[kMaxSegments + k];
-        }
-        totals[0] += a;
-        totals[1] += b;
-    }
+    add_totals(counters, segments, totals, totals);
 }
 
-// HDRBitmapFilm::Rescale after the master-film reduction (sched.mt.cpp:250-256):
-// weight = Float(W*H) / Float(N), data *= weight, in the film's arithmetic type.
-template <class Acc, class Out>
-__global__ void k_resolve(const Acc* __restrict__ acc, Out* __restrict__ out, size_t n, Acc weight) {
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = Out(acc[i] * weight);
-}
+struct RunTotals {
+    const uint32_t* counters;
+    int segments;
+    const unsigned long long* totals;
+    unsigned long long* out;  // device or pinned host memory
+};
 
-// Compensated FP32 film: (sum + error) * weight, evaluated in FP64 and rounded once.
-template <class Out>
-__global__ void k_resolve_comp(const float* __restrict__ acc, const float* __restrict__ err, Out* __restrict__ out,
-                               size_t n, double weight) {
+// HDRBitmapFilm::Rescale after the master-film reduction (sched.mt.cpp:250-256): weight =
+// Float(W*H) / Float(N), data *= weight, in the film's arithmetic type; the compensated FP32 film
+// as (sum + error) * weight, evaluated in FP64 and rounded once.  kSplat: the replicas of splat_add
+// are first added to the film's values in their rectangle; the compensated film takes sum + error
+// + replicas in FP64, rounded to an FP32 pair.
+template <class Acc, class Out, bool kComp, bool kSplat>
+__global__ void k_resolve(PTConsts c, Out* __restrict__ out, size_t n, std::conditional_t<kComp, double, Acc> weight,
+                          RunTotals run) {
     const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = Out((double(acc[i]) + double(err[i])) * weight);
-}
-
-// The film replicas of splat_add summed into the film accumulator (value i of every
-// replica, i < 3 * splat_w * splat_h), once, after the last batch: stream order makes plain
-// read-modify-writes safe.  The compensated film takes sum + error + replicas in FP64,
-// stored back as an FP32 pair.
-__global__ void k_splat_fold(PTConsts c, size_t n) {
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0 && threadIdx.x < 64) add_totals(run.counters, run.segments, run.totals, run.out);
     if (i >= n) return;
-    const uint32_t local = uint32_t(i / 3), ch = uint32_t(i % 3);
-    const size_t j = 3ull * ((c.splat_y0 + local / c.splat_w) * size_t(c.cam.width) + c.splat_x0 + local % c.splat_w) + ch;
-    if (c.film_mode == LMGPU_FILM_FP32) {
-        const float* r = static_cast<const float*>(c.splat) + i;
-        float s = 0.f;
+    using Rep = std::conditional_t<kComp, double, Acc>;  // the replicas' type
+    Rep s = Rep(0);
+    bool in = false;
+    if constexpr (kSplat) {
+        const uint32_t w = uint32_t(c.cam.width);
+        const uint32_t pixel = uint32_t(i / 3), ch = uint32_t(i % 3);
+        const uint32_t x = pixel % w - c.splat_x0, y = pixel / w - c.splat_y0;  // wraps below the rectangle
+        in = x < c.splat_w && y < c.splat_h;
+        if (in) {
+            const Rep* r = static_cast<const Rep*>(c.splat) + 3ull * (y * c.splat_w + x) + ch;
 #pragma unroll 8
-        for (uint32_t k = 0; k < c.splat_k; k++) s += r[k * c.splat_vals];
-        static_cast<float*>(c.film)[j] += s;
-        return;
+            for (uint32_t k = 0; k < c.splat_k; k++) s += r[k * c.splat_vals];
+        }
     }
-    const double* r = static_cast<const double*>(c.splat) + i;
-    double s = 0.0;
-#pragma unroll 8
-    for (uint32_t k = 0; k < c.splat_k; k++) s += r[k * c.splat_vals];
-    if (c.film_mode == LMGPU_FILM_FP64) {
-        static_cast<double*>(c.film)[j] += s;
+    if constexpr (kComp) {
+        const float f = static_cast<const float*>(c.film)[i], e = c.film_comp[i];
+        double v = double(f) + double(e);
+        if (in) {
+            const double t = v + s;
+            const float hi = float(t);
+            v = double(hi) + double(float(t - double(hi)));
+        }
+        out[i] = Out(v * weight);
     } else {
-        float* f = static_cast<float*>(c.film) + j;
-        float* e = c.film_comp + j;
-        const double t = double(*f) + double(*e) + s;
-        const float hi = float(t);
-        *f = hi;
-        *e = float(t - double(hi));
+        Acc v = static_cast<const Acc*>(c.film)[i];
+        if (in) v += s;
+        out[i] = Out(v * weight);
     }
 }
 
@@ -1428,12 +1450,9 @@ __global__ __launch_bounds__(kPTBlock) void k_conn_reduce(PTConsts c, const floa
         if (acc[k] != Acc(0)) unsafeAtomicAdd(rep + k, acc[k]);
 }
 
-// sum over samples of |Q.x| + |Q.y| + |Q.z| (the replay check of the adjoint).
-__global__ __launch_bounds__(256) void k_abs_sum(const double* __restrict__ q, uint32_t n, double* out) {
+// *out += the sum of v over a block of 256 threads.
+__device__ __forceinline__ void block_sum_to(double v, double* out) {
     __shared__ double part[256 / 64];
-    double v = 0.0;
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
-        v += fabs(q[4ull * i]) + fabs(q[4ull * i + 1]) + fabs(q[4ull * i + 2]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     if (__lane_id() == 0) part[threadIdx.x >> 6] = v;
@@ -1441,32 +1460,50 @@ __global__ __launch_bounds__(256) void k_abs_sum(const double* __restrict__ q, u
     if (threadIdx.x == 0) unsafeAtomicAdd(out, part[0] + part[1] + part[2] + part[3]);
 }
 
+// sum over samples of |Q.x| + |Q.y| + |Q.z| (the replay check of the adjoint).
+__global__ __launch_bounds__(256) void k_abs_sum(const double* __restrict__ q, uint32_t n, double* out) {
+    double v = 0.0;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
+        v += fabs(q[4ull * i]) + fabs(q[4ull * i + 1]) + fabs(q[4ull * i + 2]);
+    block_sum_to(v, out);
+}
+
 // Adjoint pass 1 from a sample record (`stride` float4 per sample):
 // Q = sum over the record's pixels of dL/dI[pixel] * contribution.
 // A pixel index outside the film (a record the render did not write) contributes nothing.
-__global__ void k_q_from_record(const float4* __restrict__ rec, uint32_t stride, const float* __restrict__ dLdI,
-                                uint32_t npix, uint32_t n, double* __restrict__ q) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double x = 0.0, y = 0.0, z = 0.0;
-    for (uint32_t k = 0; k < stride; k++) {
-        const float4 r = rec[size_t(stride) * i + k];
-        const uint32_t pixel = __float_as_uint(r.w);
-        if (pixel >= npix) continue;
-        const float* g = dLdI + 3ull * pixel;
-        x += double(g[0]) * double(r.x);
-        y += double(g[1]) * double(r.y);
-        z += double(g[2]) * double(r.z);
+// *sum += its k_abs_sum (one atomic a block, of 4096 at most).
+__global__ __launch_bounds__(256) void k_q_from_record(const float4* __restrict__ rec, uint32_t stride, const float* __restrict__ dLdI,
+                                uint32_t npix, uint32_t n, double* __restrict__ q, double* sum) {
+    double total = 0.0;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        double x = 0.0, y = 0.0, z = 0.0;
+        for (uint32_t k = 0; k < stride; k++) {
+            const float4 r = rec[size_t(stride) * i + k];
+            const uint32_t pixel = __float_as_uint(r.w);
+            if (pixel >= npix) continue;
+            const float* g = dLdI + 3ull * pixel;
+            x += double(g[0]) * double(r.x);
+            y += double(g[1]) * double(r.y);
+            z += double(g[2]) * double(r.z);
+        }
+        q[4ull * i + 0] = x;
+        q[4ull * i + 1] = y;
+        q[4ull * i + 2] = z;
+        q[4ull * i + 3] = 0.0;
+        total += fabs(x) + fabs(y) + fabs(z);
     }
-    q[4ull * i + 0] = x;
-    q[4ull * i + 1] = y;
-    q[4ull * i + 2] = z;
-    q[4ull * i + 3] = 0.0;
+    block_sum_to(total, sum);
 }
 
-__global__ void k_scale_f64(double* p, uint32_t n, double w) {
+// The gradients (materials, then lights) times w, to where they go; the replay check's sums and the
+// totals after them.
+__global__ void k_grad_out(const double* p, uint32_t nmat, uint32_t n, double w, double* mat, double* light,
+                           const double* sums, double* sums_out, RunTotals run) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] *= w;
+    if (blockIdx.x == 0 && threadIdx.x < 64) add_totals(run.counters, run.segments, run.totals, run.out);
+    if (i < 2) sums_out[i] = sums[i];
+    if (i < nmat) mat[i] = p[i] * w;
+    else if (i < n) light[i - nmat] = p[i] * w;
 }
 
 // ---------------------------------------------------------------------------------
@@ -1632,6 +1669,17 @@ struct Pipeline {
     size_t sort_temp_bytes = 0;
     int key_bits = 0;
     int key_skip = 0;
+    bool counters_clear = false;  // the next batch need not clear them
+
+    // Clears what a run starts from (k_clear).
+    void clear(void* a, size_t a_bytes, void* b2, size_t b2_bytes) {
+        const size_t na = a_bytes / 16, nb = b2_bytes / 16;
+        const uint32_t nw = (4096u + 64u) / 4u;
+        hipLaunchKernelGGL(k_clear, dim3(uint32_t((std::max<size_t>(na + nb, nw) + 255) / 256)), dim3(256), 0, ctx->stream,
+                           static_cast<uint4*>(a), na, static_cast<uint4*>(b2), nb, b.counters, nw);
+        counters_clear = true;
+    }
+    RunTotals run_totals(unsigned long long* out) const { return {b.counters, segments + 1, b.totals, out}; }
 
     lmgpu_status setup(const lmgpu_pt_params* p) {
         cap = p->wavefront_width ? p->wavefront_width : auto_width(ctx, p->num_samples);
@@ -1700,11 +1748,14 @@ struct Pipeline {
     // One batch [base, base + nb) of the global sample range through every stage.
     // counters[k]: queue entering segment k; counters[kMaxSegments + k]: shadow rays emitted
     // before segment k; [2 kMaxSegments, 4 kMaxSegments + 1): work counters of the launches.
-    template <int kMode> lmgpu_status batch(uint64_t base, uint32_t nb) {
+    // `last`: the run's last kernel adds its counters to the totals.
+    template <int kMode> lmgpu_status batch(uint64_t base, uint32_t nb, bool last) {
         hipStream_t s = ctx->stream;
         c.base = base;
         c.batch = nb;
-        hipLaunchKernelGGL(k_zero_u32, dim3(2), dim3(256), 0, s, b.counters, uint32_t(4 * kMaxSegments));
+        if (!counters_clear)
+            hipLaunchKernelGGL(k_zero_u32, dim3(2), dim3(256), 0, s, b.counters, uint32_t(4 * kMaxSegments));
+        counters_clear = false;
         const dim3 grid_b((nb + kPTBlock - 1) / kPTBlock), grid_c((cap + kPTBlock - 1) / kPTBlock);
         // Persistent traversal grids: the device fill, never more than the queue capacity needs with a
         // wave per ray.
@@ -1836,7 +1887,7 @@ struct Pipeline {
         }
         // k_shade_pt never enqueues a path whose vertex count reached max_path_vertices, so
         // the final queue is empty.
-        hipLaunchKernelGGL(k_accumulate_totals, dim3(1), dim3(64), 0, s, b.counters, segments + 1, b.totals);
+        if (!last) hipLaunchKernelGGL(k_accumulate_totals, dim3(1), dim3(64), 0, s, b.counters, segments + 1, b.totals);
         e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(ctx, e, "k_accumulate_totals");
         return LMGPU_OK;
@@ -1959,57 +2010,39 @@ lmgpu_status run_pt(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_film* film, 
 
     hipStream_t s = ctx->stream;
     (void)hipEventRecord(ctx->run0, s);
-    hipLaunchKernelGGL(k_zero_bytes, dim3(uint32_t((acc_bytes / 16 + 255) / 256)), dim3(256), 0, s,
-                       static_cast<uint4*>(ctx->film_acc), acc_bytes / 16);
-    if (splat_bytes)
-        hipLaunchKernelGGL(k_zero_bytes, dim3(uint32_t((splat_bytes / 16 + 255) / 256)), dim3(256), 0, s,
-                           static_cast<uint4*>(ctx->splat_buf), splat_bytes / 16);
-    hipLaunchKernelGGL(k_zero_u32, dim3(5), dim3(256), 0, s, pl.b.counters, (4096u + 64u) / 4u);
+    pl.clear(ctx->film_acc, acc_bytes, ctx->splat_buf, splat_bytes);
     const uint32_t rec_stride = p->renderer == LMGPU_PT ? 1u : 2u;  // float4 per sample in the record
     for (uint64_t base = 0; base < p->num_samples && st == LMGPU_OK; base += pl.cap) {
         pl.c.record = p->sample_record ? static_cast<float4*>(p->sample_record) + rec_stride * base : nullptr;
-        st = pl.batch<kRender>(p->sample_offset + base, uint32_t(std::min<uint64_t>(pl.cap, p->num_samples - base)));
+        const uint32_t nb = uint32_t(std::min<uint64_t>(pl.cap, p->num_samples - base));
+        st = pl.batch<kRender>(p->sample_offset + base, nb, base + nb == p->num_samples);
     }
     if (st == LMGPU_OK) {
         // Resolve: sums * W*H/N into the output film.
         const dim3 rg(uint32_t((nval + 255) / 256));
-        if (splat_bytes)
-            hipLaunchKernelGGL(k_splat_fold, dim3(uint32_t((splat_vals + 255) / 256)), dim3(256), 0, s, pl.c, splat_vals);
-        if (comp) {
-            const double w = double(npix) / double(p->num_samples);
-            const float* acc = static_cast<const float*>(ctx->film_acc);
-            if (film->precision == LMGPU_FILM_FP64)
-                hipLaunchKernelGGL(k_resolve_comp<double>, rg, dim3(256), 0, s, acc, pl.c.film_comp,
-                                   static_cast<double*>(out_dev), nval, w);
-            else
-                hipLaunchKernelGGL(k_resolve_comp<float>, rg, dim3(256), 0, s, acc, pl.c.film_comp,
-                                   static_cast<float*>(out_dev), nval, w);
-        } else if (p->film_precision == LMGPU_FILM_FP64) {
-            const double w = double(npix) / double(p->num_samples);
-            const double* acc = static_cast<const double*>(ctx->film_acc);
-            if (film->precision == LMGPU_FILM_FP64)
-                hipLaunchKernelGGL((k_resolve<double, double>), rg, dim3(256), 0, s, acc, static_cast<double*>(out_dev),
-                                   nval, w);
-            else
-                hipLaunchKernelGGL((k_resolve<double, float>), rg, dim3(256), 0, s, acc, static_cast<float*>(out_dev),
-                                   nval, w);
-        } else {
-            const float w = float(npix) / float(p->num_samples);
-            const float* acc = static_cast<const float*>(ctx->film_acc);
-            if (film->precision == LMGPU_FILM_FP64)
-                hipLaunchKernelGGL((k_resolve<float, double>), rg, dim3(256), 0, s, acc, static_cast<double*>(out_dev),
-                                   nval, w);
-            else
-                hipLaunchKernelGGL((k_resolve<float, float>), rg, dim3(256), 0, s, acc, static_cast<float*>(out_dev),
-                                   nval, w);
-        }
+        const double w = double(npix) / double(p->num_samples);
+        const RunTotals run = pl.run_totals(pinned ? static_cast<unsigned long long*>(words) : pl.b.totals);
+        auto resolve = [&](auto kernel, auto* out, auto weight) {
+            hipLaunchKernelGGL(kernel, rg, dim3(256), 0, s, pl.c, out, nval, weight, run);
+        };
+        auto resolve_to = [&](auto* out) {
+            using Out = std::remove_pointer_t<decltype(out)>;
+            if (comp && splat_bytes) resolve(k_resolve<float, Out, true, true>, out, w);
+            else if (comp) resolve(k_resolve<float, Out, true, false>, out, w);
+            else if (p->film_precision == LMGPU_FILM_FP64 && splat_bytes) resolve(k_resolve<double, Out, false, true>, out, w);
+            else if (p->film_precision == LMGPU_FILM_FP64) resolve(k_resolve<double, Out, false, false>, out, w);
+            else if (splat_bytes) resolve(k_resolve<float, Out, false, true>, out, float(npix) / float(p->num_samples));
+            else resolve(k_resolve<float, Out, false, false>, out, float(npix) / float(p->num_samples));
+        };
+        if (film->precision == LMGPU_FILM_FP64) resolve_to(static_cast<double*>(out_dev));
+        else resolve_to(static_cast<float*>(out_dev));
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) st = hip_fail(ctx, e, "k_resolve");
     }
     (void)hipEventRecord(ctx->run1, s);
     unsigned long long totals[2] = {0, 0};
     if (st == LMGPU_OK) {
-        hipError_t e = hipMemcpyAsync(words, pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
+        hipError_t e = pinned ? hipSuccess : hipMemcpyAsync(words, pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = film->device || direct ? hipStreamSynchronize(s) : read_back(ctx, film->data, out_dev, out_bytes);
         if (e != hipSuccess) st = hip_fail(ctx, e, "pt readback");
         else std::memcpy(totals, words, sizeof(totals));
@@ -2068,17 +2101,16 @@ lmgpu_status run_pt_backward(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_adj
     pl.c.film_mode = LMGPU_FILM_FP32;
 
     (void)hipEventRecord(ctx->run0, s);
-    hipLaunchKernelGGL(k_zero_bytes, dim3(uint32_t(((g_bytes + 16) / 16 + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<uint4*>(grad), (g_bytes + 16) / 16);
-    hipLaunchKernelGGL(k_zero_u32, dim3(5), dim3(256), 0, s, pl.b.counters, (4096u + 64u) / 4u);
+    pl.clear(grad, g_bytes + 16, nullptr, 0);
     const uint32_t rec_stride = p->renderer == LMGPU_PT ? 1u : 2u;  // float4 per sample in the record
     for (uint64_t base = 0; base < p->num_samples && st == LMGPU_OK; base += pl.cap) {
         const uint32_t nb = uint32_t(std::min<uint64_t>(pl.cap, p->num_samples - base));
+        const dim3 grid_sum(std::min<uint32_t>((nb + 255) / 256, 256u));
         if (p->sample_record) {
             // The forward's record holds every sample's contributions: Q without a replay.
-            hipLaunchKernelGGL(k_q_from_record, dim3((nb + 255) / 256), dim3(256), 0, s,
+            hipLaunchKernelGGL(k_q_from_record, dim3(std::min<uint32_t>((nb + 255) / 256, 4096u)), dim3(256), 0, s,
                                static_cast<const float4*>(p->sample_record) + rec_stride * base, rec_stride,
-                               pl.c.dLdI, uint32_t(npix), nb, pl.c.qacc);
+                               pl.c.dLdI, uint32_t(npix), nb, pl.c.qacc, sums + 0);
             e = hipGetLastError();
             if (e != hipSuccess) {
                 st = hip_fail(ctx, e, "k_q_from_record");
@@ -2087,40 +2119,46 @@ lmgpu_status run_pt_backward(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_adj
         } else {
             hipLaunchKernelGGL(k_zero_bytes, dim3(uint32_t((size_t(nb) * 2 + 255) / 256)), dim3(256), 0, s,
                                reinterpret_cast<uint4*>(pl.c.qacc), size_t(nb) * 2);
-            st = pl.batch<kAdjTotal>(p->sample_offset + base, nb);
+            st = pl.batch<kAdjTotal>(p->sample_offset + base, nb, false);
             if (st != LMGPU_OK) break;
+            hipLaunchKernelGGL(k_abs_sum, grid_sum, dim3(256), 0, s, pl.c.qacc, nb, sums + 0);
         }
-        const dim3 grid_sum(std::min<uint32_t>((nb + 255) / 256, 256u));
-        hipLaunchKernelGGL(k_abs_sum, grid_sum, dim3(256), 0, s, pl.c.qacc, nb, sums + 0);
-        st = pl.batch<kAdjGrad>(p->sample_offset + base, nb);
+        st = pl.batch<kAdjGrad>(p->sample_offset + base, nb, base + nb == p->num_samples);
         if (st != LMGPU_OK) break;
         hipLaunchKernelGGL(k_abs_sum, grid_sum, dim3(256), 0, s, pl.c.qacc, nb, sums + 1);
     }
-    if (st == LMGPU_OK) {
-        // The film is Sum * W*H/N (sched.mt.cpp:256): the same factor scales its gradient.
-        hipLaunchKernelGGL(k_scale_f64, dim3((ngrad + 255) / 256), dim3(256), 0, s, grad, ngrad,
-                           double(npix) / double(p->num_samples));
-        e = hipGetLastError();
-        if (e != hipSuccess) st = hip_fail(ctx, e, "k_scale_f64");
-    }
-    (void)hipEventRecord(ctx->run1, s);
     unsigned long long totals[2] = {0, 0};
     double hs[2] = {0.0, 0.0};
-    char words_here[sizeof(hs) + sizeof(totals)];
-    char* const words = ensure_pinned(ctx, kPinnedWords) ? static_cast<char*>(ctx->io->pinned) : words_here;
+    const uint32_t nmat = 3u * ctx->num_materials, nlight = ngrad - nmat;
+    const bool pinned = ensure_pinned(ctx, kPinnedWords);
+    // The sums and the totals, on the device where there is no pinned memory.
+    double* const hs_out = pinned ? static_cast<double*>(ctx->io->pinned) : sums;
+    unsigned long long* const totals_out = pinned ? reinterpret_cast<unsigned long long*>(hs_out + 2) : pl.b.totals;
     if (st == LMGPU_OK) {
-        const hipMemcpyKind k = adj->grad_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-        e = hipMemcpyAsync(adj->d_albedo, grad, size_t(ctx->num_materials) * 24, k, s);
-        if (e == hipSuccess && ctx->num_lights > 0)
-            e = hipMemcpyAsync(adj->d_emission, pl.c.grad_light, size_t(ctx->num_lights) * 24, k, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(words, sums, sizeof(hs), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(words + sizeof(hs), pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
+        // The film is Sum * W*H/N (sched.mt.cpp:256): the same factor scales its gradient.
+        hipLaunchKernelGGL(k_grad_out, dim3((ngrad + 255) / 256), dim3(256), 0, s, grad, nmat, ngrad,
+                           double(npix) / double(p->num_samples), adj->grad_device ? adj->d_albedo : grad,
+                           adj->grad_device ? adj->d_emission : grad + nmat, sums, hs_out, pl.run_totals(totals_out));
+        e = hipGetLastError();
+        if (e != hipSuccess) st = hip_fail(ctx, e, "k_grad_out");
+    }
+    (void)hipEventRecord(ctx->run1, s);
+    if (st == LMGPU_OK) {
+        if (!adj->grad_device) {
+            e = hipMemcpyAsync(adj->d_albedo, grad, size_t(nmat) * 8, hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess && nlight > 0)
+                e = hipMemcpyAsync(adj->d_emission, grad + nmat, size_t(nlight) * 8, hipMemcpyDeviceToHost, s);
+        }
+        if (!pinned) {
+            if (e == hipSuccess) e = hipMemcpyAsync(hs, sums, sizeof(hs), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipMemcpyAsync(totals, pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
+        }
         if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) st = hip_fail(ctx, e, "adjoint readback");
-        else {
-            std::memcpy(hs, words, sizeof(hs));
-            std::memcpy(totals, words + sizeof(hs), sizeof(totals));
+        if (e != hipSuccess) {
+            st = hip_fail(ctx, e, "adjoint readback");
+        } else if (pinned) {
+            std::memcpy(hs, hs_out, sizeof(hs));
+            std::memcpy(totals, totals_out, sizeof(totals));
         }
     }
     float ms = 0.f;
