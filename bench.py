@@ -19,7 +19,7 @@ against central differences on 64 parameters.
 
 `roofline` is measured live: HIP events around every traversal launch (the traversal
 kernel and the FP64 pass) on the launch stream give the average duration; algorithmic
-bytes per launch come from the kernel's own counting run (node visits x 112 B + triangle
+bytes per launch come from the kernel's own counting run (node visits x 64 B + triangle
 tests x 48 B + 32 B ray + 16 B hit per ray) plus the FP64 pass (4 B per ray; ray, FP32
 result, triangle record and result per hit).  `cpu_baseline` times the CPU restatement (FP32 4-wide QBVH with SSE,
 OpenMP over the host cores) on the same rays.
@@ -38,24 +38,24 @@ sys.path.insert(0, str(ROOT))
 
 METRIC = "M path-samples/s + Mrays/s on 1 MI355X at fixed RMSE; backward/forward ratio"
 HBM_PEAK_GBS = 8000.0
-NODE_BYTES = 112  # bytes of a 4-wide node the kernel loads (6 box planes x 4 + 4 child words)
-TRI_BYTES = 48    # one triangle record
+NODE_BYTES = 64   # a packed 4-wide node (origin, steps, 24 8-bit planes, 4 child words)
+TRI_BYTES = 48    # the vertices and index of a triangle record
 RAY_BYTES = 32    # o, d, tmin, tmax
 HIT_BYTES = 16    # t, b0, b1, prim
 
 
 # Algorithmic bytes of the path tracer's stages (SoA path queues of 16-byte records):
-#   extension ray: ray in (origin + tmin, direction + pdf) 32 B, hit out 16 B, plus the nodes and
+#   extension ray: ray in (origin and direction records) 32 B, hit out 16 B, plus the nodes and
 #     triangle records its traversal visits;
 #   shadow ray: record in (origin + tmax, direction + pixel, contribution + light) 48 B, one film
 #     update 12 B, plus its traversal;
-#   pt shading of one path: path in 80 B (5 records), hit 16 B, shading record 64 B, material 16 B;
-#     a surviving path out 80 B, an ending path one film update 12 B;
-#   camera stage: one path out, 80 B.
+#   pt shading of one path: path in 48 B (3 records), hit 16 B, shading record 64 B, material 16 B;
+#     a surviving path out 48 B, an ending path one film update 12 B;
+#   camera stage: one path out, 48 B.
 EXT_RAY_BYTES = 32 + 16
 SHADOW_RAY_BYTES = 48 + 12
-SHADE_IN_BYTES = 80 + 16 + 64 + 16
-PATH_BYTES = 80
+SHADE_IN_BYTES = 48 + 16 + 64 + 16
+PATH_BYTES = 48
 FILM_ADD_BYTES = 12
 CLOCK_GHZ = 2.4  # MI355X peak engine clock
 NUM_CUS = 256
@@ -260,7 +260,7 @@ def run_traversal(args, torch, Device, scenes):
         "host_buffers": {"Mrays_per_s": round(n / host_s / 1e6, 1), "seconds": round(host_s, 4),
                          "same_hits_as_device_buffers": host_same,
                          "note": "lmgpu_trace_closest on pageable host arrays (32 B per ray in, 16 B per hit "
-                                 "out over PCIe, in 2M-ray chunks through pinned memory), one call over the "
+                                 "out over PCIe, in 512k-ray chunks through pinned memory), one call over the "
                                  "same rays"},
         "modes": extra,
         "gpu_hits": gpu_hits,
@@ -871,7 +871,7 @@ def main():
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic,
-            "kernel": "k_trace_closest<true> + k_refine_fp64",
+            "kernel": "k_trace_record + k_refine_fp64",
             "kernel_ms": round(res["kernel_ms"], 4),
             "alg_bytes_per_launch": int(res["alg_bytes"]),
         },

@@ -120,10 +120,10 @@ typedef struct lmgpu_bvh_params {
 } lmgpu_bvh_params;
 
 typedef struct lmgpu_bvh_info {
-    uint32_t num_nodes;       /* 4-wide nodes (128 B each) */
+    uint32_t num_nodes;       /* 4-wide nodes (64 B packed, and 128 B as built) */
     uint32_t num_leaves;
     uint32_t max_depth;       /* inner-node levels on the deepest path */
-    uint32_t num_tri_records; /* 48 B each */
+    uint32_t num_tri_records; /* 64 B each, leaves on 128-byte lines */
     double build_seconds;
     double sah_cost;
     uint64_t device_bytes;
@@ -221,9 +221,10 @@ lmgpu_status lmgpu_scene_upload(lmgpu_ctx* ctx, const lmgpu_scene_desc* desc);
 lmgpu_status lmgpu_bvh_build(lmgpu_ctx* ctx, const lmgpu_bvh_params* params, lmgpu_bvh_info* info);
 
 /* ---- traversal ---------------------------------------------------------------- */
-/* Host rays and results (device flags clear) are staged through the device; from 2^20 rays
- * on they move in chunks through pinned host memory, copied by up to 8 host threads, with
- * uploads, kernels and read-backs overlapped on two extra streams of the context.  The call
+/* Host rays and results (device flags clear) go through pinned host memory, copied by up to 8
+ * host threads: up to 1024 rays are read and written there by the kernels, up to 65536 are
+ * copied to the device and back in one piece, more in chunks, with uploads, kernels and
+ * read-backs overlapped on two extra streams of the context.  The call
  * returns when the host results are written; with device buffers it only enqueues. */
 lmgpu_status lmgpu_trace_closest(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uint32_t n, lmgpu_hits_soa* hits,
                                  uint32_t flags);

@@ -1691,7 +1691,7 @@ struct Pipeline {
         carve(ctx->pt_buf, cap, b);
         c = PTConsts{};
         c.bvh = bvh_of(ctx);
-            c.xform = ctx->xform.ptr;
+        c.xform = ctx->xform.ptr;
         c.shade = ctx->shade.ptr;
         c.mats = ctx->mats.ptr;
         c.lights = ctx->lights.ptr;
