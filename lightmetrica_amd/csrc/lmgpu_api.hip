@@ -888,7 +888,7 @@ lmgpu_status lmgpu_trace_closest(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uin
                                             reinterpret_cast<float*>(o[2]), reinterpret_cast<int32_t*>(o[3]), refine,
                                             ctx->next_counter);
             },
-            "k_trace_closest (host buffers)");
+            "closest hit (host buffers)");
         if (s != LMGPU_ERR_UNSUPPORTED) return s;
     }
     const float* dev[8];
@@ -904,7 +904,7 @@ lmgpu_status lmgpu_trace_closest(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uin
         prim = reinterpret_cast<int32_t*>(b1 + n);
     }
     hipError_t e = launch_trace_closest(ctx, dev, n, t, b0, b1, prim, refine, ctx->next_counter);
-    if (e != hipSuccess) return hip_fail(ctx, e, "k_trace_closest");
+    if (e != hipSuccess) return hip_fail(ctx, e, "closest hit");
     if (!hits->device) {
         const void* srcs[4] = {t, b0, b1, prim};
         void* dsts[4] = {hits->t, hits->b0, hits->b1, hits->prim};
@@ -946,7 +946,7 @@ lmgpu_status lmgpu_trace_closest_noalloc(lmgpu_ctx* ctx, const lmgpu_rays_soa* r
     // before the traversal) is word 0 of this device's static scratch array.
     hipError_t e = launch_trace_closest(ctx, dev, n, hits->t, hits->b0, hits->b1, hits->prim,
                                         (flags & LMGPU_TRACE_REFINE_FP64) != 0, ctx->noalloc_scratch);
-    if (e != hipSuccess) return hip_fail(ctx, e, "k_trace_closest");
+    if (e != hipSuccess) return hip_fail(ctx, e, "closest hit");
     return LMGPU_OK;
 }
 
