@@ -45,16 +45,16 @@ HIT_BYTES = 16    # t, b0, b1, prim
 
 
 # Algorithmic bytes of the path tracer's stages (SoA path queues of 16-byte records):
-#   extension ray: ray in (origin and direction records) 32 B, hit out 16 B, plus the nodes and
+#   extension ray: ray in (origin and direction records) 32 B, hit out 4 B (its record), plus the nodes and
 #     triangle records its traversal visits;
 #   shadow ray: record in (origin + tmax, direction + pixel, contribution + light) 48 B, one film
 #     update 12 B, plus its traversal;
-#   pt shading of one path: path in 48 B (3 records), hit 16 B, shading record 64 B, material 16 B;
+#   pt shading of one path: path in 48 B (3 records), hit 4 B, triangle 48 B, shading record 64 B, material 16 B;
 #     a surviving path out 48 B, an ending path one film update 12 B;
 #   camera stage: one path out, 48 B.
-EXT_RAY_BYTES = 32 + 16
+EXT_RAY_BYTES = 32 + 4
 SHADOW_RAY_BYTES = 48 + 12
-SHADE_IN_BYTES = 48 + 16 + 64 + 16
+SHADE_IN_BYTES = 48 + 4 + 48 + 64 + 16
 PATH_BYTES = 48
 FILM_ADD_BYTES = 12
 CLOCK_GHZ = 2.4  # MI355X peak engine clock

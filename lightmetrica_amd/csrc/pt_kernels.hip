@@ -124,7 +124,7 @@ struct ShadowQueue {
 
 struct PTBuffers {
     Queue q[2];
-    float4* hits;  // t, b0, b1, prim (bits)
+    uint32_t* hits;  // records of the segment's hits
     ShadowQueue sq;
     uint32_t* counters;  // [0, 64): live-queue sizes per segment, [64, 128): shadow sizes per segment,
                          // [128, 192): work counters of the extension launches, [192, 257): of the shadow launches
@@ -866,19 +866,27 @@ struct QueueSource {
     }
 };
 
+// A segment's hits: the winner's record (kMiss for none), a word per path.  The shading stages repeat
+// its test (hit_of), which gives the traversal's t and weights: a training step's extension rays
+// 10.52 -> 10.15 ms without the four-word results and their registers, its shading 4.10 -> 4.18.
 struct HitSink {
-    const LeafTri* tris;
-    float4* hits;
-    __device__ __forceinline__ void operator()(uint32_t i, bool found, const HitOut& h, const RayIn& r) const {
-        float4 out = make_float4(0.f, 0.f, 0.f, __uint_as_float(kMiss));
-        if (found) {
-            float t, b0, b1;
-            winner_barycentrics(tris, r, h, false, t, b0, b1);
-            out = make_float4(t, b0, b1, __uint_as_float(h.prim));
-        }
-        hits[i] = out;
+    uint32_t* recs;
+    __device__ __forceinline__ void operator()(uint32_t i, bool found, const HitOut& h, const RayIn&) const {
+        recs[i] = found ? h.rec : kMiss;
     }
 };
+
+// (t, b0, b1, triangle bits) of record `rec` along r.
+__device__ __forceinline__ float4 hit_of(const LeafTri* tris, uint32_t rec, const RayIn& r) {
+    if (rec == kMiss) return make_float4(0.f, 0.f, 0.f, __uint_as_float(kMiss));
+    const float4* tp = reinterpret_cast<const float4*>(tris + rec);
+    const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
+    HitOut h{};
+    float U;
+    (void)watertight(make_shear_cyclic(r), v0, v1, v2, r.tmin, r.tmax, h.t, U, h.b0, h.b1, h.det);
+    hit_weights(h);
+    return make_float4(h.t, h.b0, h.b1, v0.w);
+}
 
 // The LDS of a stage that traces a queue, whatever the number of rays makes of it: late bounces
 // hold few rays, which several lanes follow each (trace_grouped).
@@ -908,11 +916,11 @@ __device__ __forceinline__ void add_wave_counts(const TraceCounters& cnt, unsign
 template <bool kCount = false>
 __global__ __launch_bounds__(kTraceBlock, 6) void k_extend(BvhDev bvh, Queue q, float tmin,
                                                         const uint32_t* __restrict__ count, uint32_t* next,
-                                                        float4* __restrict__ hits, unsigned long long* counts) {
+                                                        uint32_t* __restrict__ hits, unsigned long long* counts) {
     __shared__ QueueShared<true> sm;
     const uint32_t n = *count;
     QueueSource src{q, tmin};
-    HitSink sink{bvh.tris, hits};
+    HitSink sink{hits};
     TraceCounters cnt{0, 0};
     if (n <= kGroup64Rays) trace_grouped<false, kCount, 64>(bvh, n, sm.group64, src, sink, cnt);
     else if (n <= kGroup16Closest) trace_grouped<false, kCount, 16>(bvh, n, sm.group16, src, sink, cnt);
@@ -1001,7 +1009,7 @@ __device__ __forceinline__ uint32_t lanes_per_path(uint32_t count) {
 // kTable: the film's sums go through film_flush.
 template <int kMode, bool kFuse = false, bool kTable = false>
 __global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, float tmin, const uint32_t* __restrict__ in_count,
-                                                       const float4* __restrict__ hits, Queue out,
+                                                       const uint32_t* __restrict__ hits, Queue out,
                                                        uint32_t* out_count) {
     const uint32_t count = *in_count;
     // kFuse: a segment of few paths gives each path a group of lanes (lanes_per_path).
@@ -1032,7 +1040,7 @@ __global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, flo
     // kFuse (scenes of at most kBruteMaxTris triangles): the segment's ray is traced here
     // instead of by a separate extension launch.
     const RayIn ray{ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, tmin, kInf};
-    const float4 hit = kFuse ? xform_closest(xf, c.ntris, ray, valid, group, sub) : hits[j];
+    const float4 hit = kFuse ? xform_closest(xf, c.ntris, ray, valid, group, sub) : hit_of(c.bvh.tris, hits[j], ray);
     // Every lane of a group shades the same path the same way; the lead lane applies it.
     const PtVertex v = pt_vertex(c, o, d, tmin, hit, valid, T, n, rng);
     if (v.emits) {
@@ -1066,7 +1074,7 @@ __global__ __launch_bounds__(kPTBlock) void k_shade_pt(PTConsts c, Queue in, flo
 // the room's pt.direct / pt.mis renders 3 % faster).
 template <int kMode, bool kFuse = false>
 __global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in, float tmin, const uint32_t* __restrict__ in_count,
-                                                        const float4* __restrict__ hits, Queue out,
+                                                        const uint32_t* __restrict__ hits, Queue out,
                                                         uint32_t* out_count, ShadowQueue sq, uint32_t* shadow_count) {
     const uint32_t count = *in_count;
     // kFuse: a segment of few paths gives each path a group of lanes (lanes_per_path).
@@ -1098,7 +1106,7 @@ __global__ __launch_bounds__(kPTBlock, 5) void k_shade_nee(PTConsts c, Queue in,
     s.mat = kBlackMat;
     s.light = -1;
     const RayIn ray{ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, tmin, kInf};
-    const float4 hit = kFuse ? xform_closest(xf, c.ntris, ray, valid, group, sub) : hits[j];
+    const float4 hit = kFuse ? xform_closest(xf, c.ntris, ray, valid, group, sub) : hit_of(c.bvh.tris, hits[j], ray);
     bool alive = valid && surface_at(c, o, d, tmin, hit, s);
     bool emits = false;
     V3 Le_w = v3s(0.f);
@@ -1565,6 +1573,7 @@ static void connection_rect(const lmgpu_ctx* ctx, uint32_t r[4]) {
 }
 
 static size_t queue_bytes(uint32_t cap) { return size_t(cap) * 16 * 4; }
+static size_t hit_bytes(uint32_t cap) { return (size_t(cap) * 4 + 15) / 16 * 16; }
 
 static void carve(void* base, uint32_t cap, PTBuffers& b) {
     char* p = static_cast<char*>(base);
@@ -1574,7 +1583,7 @@ static void carve(void* base, uint32_t cap, PTBuffers& b) {
         b.q[k].aux = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
         b.q[k].meta = reinterpret_cast<uint4*>(p); p += size_t(cap) * 16;
     }
-    b.hits = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
+    b.hits = reinterpret_cast<uint32_t*>(p); p += hit_bytes(cap);
     b.sq.o = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
     b.sq.d = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
     b.sq.c = reinterpret_cast<float4*>(p); p += size_t(cap) * 16;
@@ -1584,10 +1593,10 @@ static void carve(void* base, uint32_t cap, PTBuffers& b) {
     b.totals = reinterpret_cast<unsigned long long*>(p);
 }
 
-static size_t pt_bytes(uint32_t cap) { return 2 * queue_bytes(cap) + size_t(cap) * (16 * 4 + 8) + 4096 + 64; }
+static size_t pt_bytes(uint32_t cap) { return 2 * queue_bytes(cap) + hit_bytes(cap) + size_t(cap) * (16 * 3 + 8) + 4096 + 64; }
 
 // Paths in flight per batch when the caller leaves it to the library: the whole render in one
-// batch, up to 2^26 paths (13.4 GB of queues) and a quarter of the device memory free for the
+// batch, up to 2^26 paths (12.6 GB of queues) and a quarter of the device memory free for the
 // queues and the adjoint's per-sample totals.  Wide batches keep every segment's launch full:
 // with RR the late segments of a 2^21-path batch hold a few hundred thousand paths, fewer than
 // the persistent traversal grid has lanes.
