@@ -149,10 +149,15 @@ bool ensure_io_events(lmgpu_ctx* ctx) {
 // memory the runtime copies with one thread: the FP64 film of a 1920 x 1080 render (50 MB) took
 // 4.8 ms, 1 to 3 so (the caller's pages are made on the way); a raycast of 1280 x 720 (11 MB), its
 // kernel included, 0.89 -> 0.51 ms.  Slots of 512 KB: 0.83 ms, a copy has its own cost on the link.
+// Fewer bytes than this are left to the runtime, which maps the caller's pages at once: raycasts of
+// 133, 537 and 1004 KB take 38, 66 and 91 us so, 45, 83 and 101 through the ring; 1312 KB 121 and
+// 108, 1735 KB 139 and 126.
+constexpr size_t kRingFrom = size_t(1152) << 10;
 hipError_t read_back(lmgpu_ctx* ctx, void* dst, const void* src, size_t bytes) {
     const hipStream_t s = ctx->stream;
     const size_t chunks = (bytes + kReadSlot - 1) / kReadSlot;
-    if (!ensure_pinned(ctx, kPinnedWords + std::min(bytes, kReadSlots * kReadSlot)) || !ensure_io_events(ctx)) {
+    if (bytes < kRingFrom ||
+        !ensure_pinned(ctx, kPinnedWords + std::min(bytes, kReadSlots * kReadSlot)) || !ensure_io_events(ctx)) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
