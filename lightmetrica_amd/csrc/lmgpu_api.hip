@@ -690,11 +690,12 @@ lmgpu_status prepare_rays(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uint32_t n
 // Host rays with host results go through pinned memory.  Up to kDirectRays the kernels read and
 // write it themselves: a copy costs more than they wait for the link.  Up to kPipeMinChunk are
 // copied to the device and back in one piece each.  More move through the device in chunks of a
-// quarter of the batch (between kPipeMinChunk and kPipeChunk rays), two of them at a time in pinned memory and in the device staging, on three streams: uploads on one
-// copy stream, the kernels on the context's stream, read-backs on the other copy stream, so the
-// two transfer directions and the kernels overlap, while the host threads copy chunk c + 1 in from
-// the caller's arrays and chunk c - 1 out to them.  Each ray is traced by the same kernels as in
-// one batch, so the results are the same.
+// quarter of the batch (between kPipeMinChunk and kPipeChunk rays), two of them at a time in pinned
+// memory and in the device staging, on three streams: uploads on one copy stream, the kernels on the
+// context's stream, read-backs on the other copy stream, so the two transfer directions and the
+// kernels overlap, while the host threads copy chunk c + 1 in from the caller's arrays and chunk
+// c - 1 out to them.  A chunk may go to another kernel than the whole batch would (a last one of few
+// rays, several lanes to each); a ray's result is the same in every one (hit_order, traverse.hpp).
 // 81 rays 210 -> 34 us (eight copies in and four out before); 512 rays direct 36 us, copied 39; 4000
 // rays 63 and 61.  65536 rays 445 -> 255 us, 1M rays 2.7 -> 1.6 ms.
 constexpr uint32_t kDirectRays = 1024;

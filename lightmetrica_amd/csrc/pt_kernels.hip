@@ -879,13 +879,8 @@ struct HitSink {
 // (t, b0, b1, triangle bits) of record `rec` along r.
 __device__ __forceinline__ float4 hit_of(const LeafTri* tris, uint32_t rec, const RayIn& r) {
     if (rec == kMiss) return make_float4(0.f, 0.f, 0.f, __uint_as_float(kMiss));
-    const float4* tp = reinterpret_cast<const float4*>(tris + rec);
-    const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
-    HitOut h{};
-    float U;
-    (void)watertight(make_shear_cyclic(r), v0, v1, v2, r.tmin, r.tmax, h.t, U, h.b0, h.b1, h.det);
-    hit_weights(h);
-    return make_float4(h.t, h.b0, h.b1, v0.w);
+    const HitOut h = hit_at(tris, rec, r);
+    return make_float4(h.t, h.b0, h.b1, __uint_as_float(h.prim));
 }
 
 // The LDS of a stage that traces a queue, whatever the number of rays makes of it: late bounces
@@ -1303,12 +1298,7 @@ struct RaycastSink {
     Out* out;
     __device__ __forceinline__ void operator()(uint32_t i, bool found, const HitOut& h, const RayIn& r) const {
         const V3 o = v3(r.ox, r.oy, r.oz), d = v3(r.dx, r.dy, r.dz);
-        float4 hit = make_float4(0.f, 0.f, 0.f, __uint_as_float(kMiss));
-        if (found) {
-            float t, b0, b1;
-            winner_barycentrics(c.bvh.tris, r, h, false, t, b0, b1);
-            hit = make_float4(t, b0, b1, __uint_as_float(h.prim));
-        }
+        const float4 hit = hit_of(c.bvh.tris, found ? h.rec : kMiss, r);
         Surf s;
         float v = 0.f;
         if (surface_at(c, o, d, 0.f, hit, s)) v = fabsf(dot(s.f.sn, -d));

@@ -3,6 +3,7 @@
 #include "traverse.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace lmgpu {
 
@@ -29,8 +30,10 @@ template <bool kRefine, class Tri> struct ClosestSink {
     const Tri* tris;
     float *t_out, *b0_out, *b1_out;
     int32_t* prim_out;
-    __device__ __forceinline__ void operator()(uint32_t i, bool found, const HitOut& h, const RayIn& r) const {
+    __device__ __forceinline__ void operator()(uint32_t i, bool found, const HitOut& hit, const RayIn& r) const {
         if (found) {
+            HitOut h = hit;
+            if constexpr (std::is_same_v<Tri, LeafTri>) h = hit_at(tris, hit.rec, r);
             float t, b0, b1;
             winner_barycentrics(tris, r, h, kRefine, t, b0, b1);
             t_out[i] = t;
@@ -130,8 +133,6 @@ __global__ __launch_bounds__(256) void k_result_fp32(const LeafTri* __restrict__
     float t = -1.f, b0 = 0.f, b1 = 0.f;
     int32_t prim = -1;
     if (rec >= 0) {
-        const float4* tp = reinterpret_cast<const float4*>(tris + rec);
-        const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
         RayIn r;
         r.ox = __builtin_nontemporal_load(rays.ox + i); r.oy = __builtin_nontemporal_load(rays.oy + i);
         r.oz = __builtin_nontemporal_load(rays.oz + i);
@@ -139,16 +140,11 @@ __global__ __launch_bounds__(256) void k_result_fp32(const LeafTri* __restrict__
         r.dz = __builtin_nontemporal_load(rays.dz + i);
         r.tmin = __builtin_nontemporal_load(rays.tmin + i);
         r.tmax = __builtin_nontemporal_load(rays.tmax + i);
-        HitOut h;
-        float V = 0.f, W = 0.f, U, det = 1.f;
-        (void)watertight(make_shear_cyclic(r), v0, v1, v2, r.tmin, r.tmax, t, U, V, W, det);
-        h.b0 = V;
-        h.b1 = W;
-        h.det = det;
-        hit_weights(h);
+        const HitOut h = hit_at(tris, uint32_t(rec), r);
+        t = h.t;
         b0 = h.b0;
         b1 = h.b1;
-        prim = __float_as_int(v0.w);
+        prim = int32_t(h.prim);
     }
     __builtin_nontemporal_store(t, t_out + i);
     __builtin_nontemporal_store(b0, b0_out + i);

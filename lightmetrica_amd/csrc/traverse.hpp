@@ -23,11 +23,11 @@
 //   * triangles use the watertight test of Woop, Benthin and Wald (JCGT 2013), with
 //     the FP64 fallback for edge functions that evaluate to exactly zero.
 // Measured on 16M incoherent rays against 1M triangles (closest hit with the FP64 pass):
-// 3.98 ms with separate node and leaf loops over 128-byte nodes and unaligned leaves, 3.06 ms
-// so; 4M any-hit segments 1.75 -> 1.31 ms; the extension rays of a 96k-triangle room (8.4M
-// paths, 8 segments, twice) 15.2 -> 12.0 ms, of which 0.4 ms buys the built boxes' order and
-// ends (LeafTri::box_yz, trace_exact).  With 128-byte nodes in the same loop: 3.35, 1.65 and
-// 13.8 ms.
+// 3.98 ms with separate node and leaf loops over 128-byte nodes and unaligned leaves, 3.11 ms
+// so; 4M any-hit segments 1.75 -> 1.30 ms; the extension rays of a 96k-triangle room (8.4M
+// paths, 8 segments, twice) 15.2 -> 10.3 ms.  With 128-byte nodes in the same loop: 3.35, 1.65 and
+// 13.8 ms.  Of that 0.05, 0 and 0.2 ms go into checking each ray's last hit against the built boxes
+// (sound_hit); checked as each hit is met it took 0.13, 0.04 and 0.5 ms.
 // Acceptance follows the reference's QBVH: t strictly inside (tmin, tmax), the first
 // triangle found wins an exact tie (scene.qbvh.cpp:124-133).
 #pragma once
@@ -44,6 +44,7 @@ struct RayIn {
     float ox, oy, oz, dx, dy, dz, tmin, tmax;
 };
 
+// The descents of the BVH report a hit by its record alone (`rec`), which hit_at turns into the rest.
 struct HitOut {
     float t;
     uint32_t rec;  // leaf-order triangle record of the winner
@@ -207,34 +208,42 @@ __device__ __forceinline__ bool watertight_tail(float ax, float ay, float bx, fl
 
 // The winner re-evaluated in FP64 (Moeller-Trumbore form): t and the weights of v1, v2.  Reads
 // only the ray's origin and direction; leaves t, b0, b1 as they are (and returns false) when
-// the FP64 determinant is 0.
+// the FP64 determinant is 0.  Fused operations are spelled out: left to the compiler they differed
+// from kernel to kernel, and the last bit of one result in 2000 with them.
 __device__ __forceinline__ bool refine_fp64(const RayIn& r, float4 v0, float4 v1, float4 v2, float& t, float& b0,
                                             float& b1) {
-    const double ox = r.ox, oy = r.oy, oz = r.oz, dx = r.dx, dy = r.dy, dz = r.dz;
-    const double p0x = v0.x, p0y = v0.y, p0z = v0.z;
-    const double e1x = double(v1.x) - p0x, e1y = double(v1.y) - p0y, e1z = double(v1.z) - p0z;
-    const double e2x = double(v2.x) - p0x, e2y = double(v2.y) - p0y, e2z = double(v2.z) - p0z;
-    const double s1x = dy * e2z - dz * e2y, s1y = dz * e2x - dx * e2z, s1z = dx * e2y - dy * e2x;
-    const double div = s1x * e1x + s1y * e1y + s1z * e1z;
+#pragma clang fp contract(off)
+    struct D3 {
+        double x, y, z;
+    };
+    auto cross = [](const D3& a, const D3& b) {
+        return D3{fma(a.y, b.z, -(a.z * b.y)), fma(a.z, b.x, -(a.x * b.z)), fma(a.x, b.y, -(a.y * b.x))};
+    };
+    auto dot = [](const D3& a, const D3& b) { return fma(a.z, b.z, fma(a.x, b.x, a.y * b.y)); };
+    const D3 d{r.dx, r.dy, r.dz}, p0{v0.x, v0.y, v0.z};
+    const D3 e1{double(v1.x) - p0.x, double(v1.y) - p0.y, double(v1.z) - p0.z};
+    const D3 e2{double(v2.x) - p0.x, double(v2.y) - p0.y, double(v2.z) - p0.z};
+    const D3 s1 = cross(d, e2);
+    const double div = dot(s1, e1);
     if (div == 0.0) return false;
     const double inv = 1.0 / div;
-    const double qx = ox - p0x, qy = oy - p0y, qz = oz - p0z;
-    const double u = (qx * s1x + qy * s1y + qz * s1z) * inv;
-    const double s2x = qy * e1z - qz * e1y, s2y = qz * e1x - qx * e1z, s2z = qx * e1y - qy * e1x;
-    const double v = (dx * s2x + dy * s2y + dz * s2z) * inv;
-    const double tt = (e2x * s2x + e2y * s2y + e2z * s2z) * inv;
-    t = float(tt);
-    b0 = float(u);
-    b1 = float(v);
+    const D3 q{r.ox - p0.x, r.oy - p0.y, r.oz - p0.z};
+    const D3 s2 = cross(q, e1);
+    t = float(dot(e2, s2) * inv);
+    b0 = float(dot(q, s1) * inv);
+    b1 = float(dot(d, s2) * inv);
     return true;
 }
 
-// 1 + 2 gamma(6), gamma(n) = n u / (1 - n u), u = 2^-24: the hardware reciprocal is within 1 ulp
-// (2u), the node's offset fma(origin, inv, offset) and the plane distance round once each, and
-// so does the threshold product.
-constexpr float kBoxRobust = 1.0f + 2.0f * 3.6e-7f;
+// Packed boxes: 1 + 2 gamma(8), gamma(n) = n u / (1 - n u), u = 2^-24.  Against the built box's test
+// (1 + 2 gamma(4)) each of the two distances is off by 3 more roundings, the node's offset
+// fma(origin, inv, offset), the step's product and the plane's own FMA, beyond what the planes'
+// margin covers: whatever the built box accepts the packed one accepts.
+constexpr float kBoxRobust = 1.0f + 2.0f * 4.8e-7f;
 // The same for a box whose planes are at hand: 1 + 2 gamma(4).
 constexpr float kBoxRobustExact = 1.0f + 2.0f * 2.4e-7f;
+// 1 - 4u: see hit_order.
+constexpr float kOrderScale = 1.0f - 2.384185791015625e-7f;
 
 // Hardware reciprocal (v_rcp_f32, within 1 ulp) of a direction component kept away from 0.
 __device__ __forceinline__ float safe_rcp(float d) {
@@ -401,9 +410,9 @@ __device__ __forceinline__ void node_children(const NodeFetch& fetch, uint32_t c
     cswap(e[1], e[2]);
 }
 
-// Records an accepted triangle in h; closest hit also keeps the watertight test's scaled weights
-// V and W of v1 and v2 and their sum det, so the winner is never fetched again: hit_weights
-// turns them into barycentric weights once the ray is done.
+// Records a triangle that trace_brute accepted in h; closest hit also keeps the watertight test's
+// scaled weights V and W of v1 and v2 and their sum det, which hit_weights turns into barycentric
+// weights once the ray is done.
 template <bool kAny>
 __device__ __forceinline__ void accept_hit(HitOut& h, float t, uint32_t rec, uint32_t prim, float V, float W,
                                            float det) {
@@ -420,6 +429,17 @@ __device__ __forceinline__ void hit_weights(HitOut& h) {
     const float inv = 1.f / h.det;
     h.b0 *= inv;
     h.b1 *= inv;
+}
+
+// A BVH record's hit as the descent saw it: the same test gives the same t and weights.
+__device__ __forceinline__ HitOut hit_at(const LeafTri* tris, uint32_t rec, const RayIn& r) {
+    const float4* tp = reinterpret_cast<const float4*>(tris + rec);
+    const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
+    HitOut h{-1.f, rec, __float_as_uint(v0.w), 0.f, 0.f, 1.f};
+    float U;
+    (void)watertight(make_shear_cyclic(r), v0, v1, v2, r.tmin, r.tmax, h.t, U, h.b0, h.b1, h.det);
+    hit_weights(h);
+    return h;
 }
 
 // The LDS of one traversal block: the stacks' LDS levels ([level][thread]), for closest hit
@@ -528,37 +548,73 @@ __device__ __forceinline__ float built_child(const BvhDev& bvh, const Slab& s, u
     return child != kEmptyChild && tn <= tf * kBoxRobustExact ? tn : INFINITY;
 }
 
+// Whether a ray meets the box of a record's leaf as it was built (lx, hx: its x range, the fourth
+// column of v1 and v2), by built_child's operations, and where it enters (`tn`).  The built boxes
+// above contain this one and their tests round monotonically, so they accept whatever it accepts.
+__device__ __forceinline__ bool in_leaf_box(const LeafTri& rec, float lx, float hx, const Slab& s, float tmin, float tmax,
+                                            float& tn) {
+    const float4 b = *reinterpret_cast<const float4*>(rec.box_yz);
+    tn = fmaxf(fmaxf(fmaf(s.ix >= 0.f ? lx : hx, s.ix, s.nx), fmaf(s.iy >= 0.f ? b.x : b.y, s.iy, s.ny)),
+               fmaxf(fmaf(s.iz >= 0.f ? b.z : b.w, s.iz, s.nz), tmin));
+    const float tf = fminf(fminf(fmaf(s.ix >= 0.f ? hx : lx, s.ix, s.fx), fmaf(s.iy >= 0.f ? b.y : b.x, s.iy, s.fy)),
+                           fminf(fmaf(s.iz >= 0.f ? b.w : b.z, s.iz, s.fz), tmax));
+    return tn <= tf * kBoxRobustExact;
+}
+
+// What orders a ray's hits: the distance, but no less than where the ray enters the hit's leaf.  The
+// FP32 test of a triangle that is large, thin or seen edge-on can place a hit before its own box;
+// a descent that has met a hit between the two by then leaves the box out, another finds it first.
+// Ordered so, no box test leaves out a hit that comes before the nearest one so far, whatever the
+// order of the descent (tn * (1 - 4u) < tmax implies tn <= tmax * (1 + 8u)), and every kernel finds
+// the same one (tmin >= 0).
+__device__ __forceinline__ float hit_order(float t, float tn) { return fmaxf(t, tn * kOrderScale); }
+
+// A descent that takes hits by their distance alone, and through packed boxes, ends at the first hit
+// in that order if the record it ends at (`rec`, at distance t) is in its leaf's box and not before
+// it: another that comes before in the order is nearer too, and was not left out unless a nearer
+// one still was accepted.  The few other rays are traced again (trace_exact).  For any hit the box
+// alone counts.
+template <bool kAny>
+__device__ __forceinline__ bool sound_hit(const BvhDev& bvh, uint32_t rec, const Slab& s, const RayIn& r, float t) {
+    const LeafTri& l = bvh.tris[rec];
+    float tn;
+    return in_leaf_box(l, l.v1[3], l.v2[3], s, r.tmin, r.tmax, tn) && (kAny || tn * kOrderScale <= t);
+}
+
 // 2^-21 of the coordinates involved in a distance along r, which is known to a few units of 2^-24
 // of them.
 __device__ __forceinline__ float distance_band(const BvhDev& bvh, const RayIn& r, const ShearCyclic& sh) {
     return 4.76837158203125e-7f * fabsf(sh.Sz) * (fmaxf(fmaxf(fabsf(r.ox), fabsf(r.oy)), fabsf(r.oz)) + bvh.reach);
 }
 
-// The packed boxes hold every hit, but the order in which a ray meets them is the built boxes' to
-// say: of two triangles at the same t the one found first wins.  A ray whose nearest hit, at
-// `t_hit`, is such a tie is traced again here, one node or leaf after the other in the order of
-// the built boxes, to the first record at t_hit.  Boxes away from t_hit by more than 1e-3 of it
-// and `band`, a thousand times what a distance can be off by, are left out: after the node's
-// children are sorted, so that the others keep their order.  Should no record be found so (a box
-// that the ray misses by rounding), the whole interval is traced.
+// The built boxes say which records a ray may hit and which of two at one place in the order
+// (hit_order) comes first: the one that their descent meets first.  A ray whose hit is in doubt is
+// traced again here, one node or leaf after the other in that order (kDone: none): to the first record at `t_hit`
+// where only that is in doubt, through the whole interval where t_hit is -inf (sound_hit is false).
+// Boxes away from t_hit by more than 1e-3 of it and `band`, a thousand times what a distance
+// commonly is off by, are left out at first: after the node's children are sorted, so that the others
+// keep their order.  Should no record be found so, the whole interval is traced.
 // Ties are 1 in 10^6 of the rays in a city, but all of those that meet two lights in one plane:
 // 1.1M camera rays over 16 overlapping lights 222 us with the whole interval, 212 us so; where a group
 // of lanes looks for it together (trace_grouped), 45824 rays 70 and 37 us.
 template <class Stack>
-__device__ __forceinline__ HitOut trace_exact(const BvhDev& bvh, const RayIn& r, float t_hit, Stack& st) {
+__device__ __forceinline__ uint32_t trace_exact(const BvhDev& bvh, const RayIn& r, float t_hit, Stack& st) {
     const Slab s = make_slab(r);
     const ShearCyclic sh = make_shear_cyclic(r);
     const float band = 1000.f * distance_band(bvh, r, sh);
-    HitOut h{r.tmax, 0u, 0xffffffffu, 0.f, 0.f, 1.f};
-    float tmax = t_hit, far = fminf(fmaf(t_hit, 1.f + 1e-3f, band), r.tmax), near = fmaf(t_hit, 1.f - 1e-3f, -band);
-    bool first = true;  // the first record at t_hit is looked for
-    uint32_t cur = 0u;
+    uint32_t rec = kDone;
+    float best = t_hit, far = fminf(fmaf(t_hit, 1.f + 1e-3f, band), r.tmax), near = fmaf(t_hit, 1.f - 1e-3f, -band);
+    bool first = t_hit > -INFINITY;  // the first record at t_hit is looked for
+    uint32_t cur = first ? 0u : kDone;
+    bool all = false;  // the whole interval
     st.sp = 0u;
     for (;;) {
         if (cur == kDone) {
-            if (!first) break;
+            if (all) break;
             first = false;
-            tmax = far = r.tmax;
+            all = true;
+            best = INFINITY;
+            far = r.tmax;
             near = -INFINITY;
             cur = 0u;
         }
@@ -596,19 +652,55 @@ __device__ __forceinline__ HitOut trace_exact(const BvhDev& bvh, const RayIn& r,
             for (uint32_t k = begin; k < end; k++) {
                 const float4* tp = reinterpret_cast<const float4*>(bvh.tris + k);
                 const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
-                float t, U, V, W, det;
-                if (watertight(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det) && (first ? t == t_hit : t < tmax)) {
-                    tmax = t;
-                    accept_hit<false>(h, t, k, __float_as_uint(v0.w), V, W, det);
-                    if (first) return h;
-                    far = t;
+                float t, U, V, W, det, tn;
+                if (!watertight(sh, v0, v1, v2, r.tmin, far, t, U, V, W, det) || !(t < r.tmax)) continue;
+                (void)in_leaf_box(bvh.tris[k], v1.w, v2.w, s, r.tmin, r.tmax, tn);
+                const float at = hit_order(t, tn);
+                if (first ? at == t_hit : at < best) {
+                    best = at;
+                    far = fminf(at, r.tmax);
+                    rec = k;
+                    if (first) return rec;
                 }
             }
             cur = kDone;
         }
-        if (cur == kDone) cur = st.pop(tmax);
+        if (cur == kDone) cur = st.pop(far);
     }
-    return h;
+    return rec;
+}
+
+// The same for any hit, where no order counts: whether a record of a leaf whose built box the ray
+// meets is hit.
+template <class Stack> __device__ __forceinline__ bool occluded_exact(const BvhDev& bvh, const RayIn& r, Stack& st) {
+    const Slab s = make_slab(r);
+    const ShearCyclic sh = make_shear_cyclic(r);
+    uint32_t cur = 0u;
+    st.sp = 0u;
+    while (cur != kDone) {
+        uint32_t next = kDone;
+        if (is_inner(cur)) {
+#pragma unroll 1
+            for (uint32_t i = 0; i < 4u; i++) {
+                uint32_t child;
+                float tf;
+                if (!(built_child(bvh, s, cur, i, r.tmin, r.tmax, child, tf) < INFINITY)) continue;
+                if (next != kDone) st.push(pack_entry(-INFINITY, next));
+                next = child;
+            }
+        } else {
+            const uint32_t begin = cur & kMaxLeafFirst, end = begin + ((cur >> 27) & 0xfu) + 1u;
+#pragma unroll 1
+            for (uint32_t k = begin; k < end; k++) {
+                const float4* tp = reinterpret_cast<const float4*>(bvh.tris + k);
+                const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
+                float t, U, V, W, det;
+                if (watertight(sh, v0, v1, v2, r.tmin, r.tmax, t, U, V, W, det) && t < r.tmax) return true;
+            }
+        }
+        cur = next != kDone ? next : st.pop(r.tmax);
+    }
+    return false;
 }
 
 // A wave fetches new rays once this many of its lanes are idle: fetching costs the setup of the
@@ -653,14 +745,12 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
     float tmax = 0.f;
     Slab sl = make_slab(r);
     ShearCyclic sh = make_shear_cyclic(r);
-    HitOut h{0.f, 0u, kNone, 0.f, 0.f, 1.f};
+    HitOut h{};
     bool found = false;
-    bool tie = false;  // closest hit: another triangle at the nearest distance (trace_exact decides)
-    // Distances beyond doubt: farther than distance_band from the ends.
-    float sure_lo = 0.f, sure_hi = 0.f;
-    // Closed rays with a tie, kTies at most; a lane with a full list takes no further ray.
+    bool tie = false;  // closest hit: another triangle at the nearest distance
+    // Closed rays that trace_exact decides, kTies at most; a lane with a full list takes no further ray.
     constexpr uint32_t kTies = 4;
-    uint32_t ties[kAny ? 1 : kTies];
+    uint32_t ties[kTies];
     float ties_at[kAny ? 1 : kTies];
     uint32_t num_ties = 0u;
     uint32_t cur = kDone;   // next node or leaf reference to visit
@@ -681,34 +771,18 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
         sh = make_shear_cyclic(r);
         tmax = r.tmax;
         found = tie = false;
-        const float band = distance_band(bvh, r, sh);
-        sure_lo = r.tmin + band;
-        if (kAny) sure_hi = fmaf(r.tmax, 1.f - 1e-6f, -band);
         tri = tri_end = 0u;
         st.sp = 0u;
         cur = 0u;
     };
-    // A triangle passed at t in (tmin, tmax].  So near an end of the interval that the FP32
-    // distance may lie inside where the leaf lies outside, the leaf's built box decides.
-    auto meet = [&](uint32_t k, float t, float id_bits, float V, float W, float det) {
-        if (t < tmax && (t < sure_lo || (kAny && t > sure_hi))) {
-            const LeafTri& rec = bvh.tris[k];
-            const float4 b = *reinterpret_cast<const float4*>(rec.box_yz);
-            const float lx = rec.v1[3], hx = rec.v2[3];
-            const float tn = fmaxf(fmaxf(fmaf(sl.ix >= 0.f ? lx : hx, sl.ix, sl.nx), fmaf(sl.iy >= 0.f ? b.x : b.y, sl.iy, sl.ny)),
-                                   fmaxf(fmaf(sl.iz >= 0.f ? b.z : b.w, sl.iz, sl.nz), r.tmin));
-            const float tf = fminf(fminf(fmaf(sl.ix >= 0.f ? hx : lx, sl.ix, sl.fx), fmaf(sl.iy >= 0.f ? b.y : b.x, sl.iy, sl.fy)),
-                                   fminf(fmaf(sl.iz >= 0.f ? b.w : b.z, sl.iz, sl.fz), tmax));
-            if (!(tn <= tf * kBoxRobustExact)) return;
-        }
-        if (kAny) {
-            found = found || t < tmax;
-        } else if (t < tmax) {
+    // A triangle passed at t in (tmin, tmax].
+    auto meet = [&](uint32_t k, float t) {
+        if (t < tmax) {
             tie = false;
             found = true;
-            tmax = t;
-            accept_hit<kAny>(h, 0.f, k, __float_as_uint(id_bits), V, W, det);  // t: tmax once the ray is done
-        } else {
+            if (!kAny) tmax = t;
+            h.rec = k;
+        } else if (!kAny) {
             tie = found;
         }
     };
@@ -784,12 +858,11 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
             const uint32_t nn = uint32_t(__popcll(nm)), nl = uint32_t(__popcll(lm)), busy = uint32_t(__popcll(nm | lm | pm));
             if (busy == 0u || (!exhausted && busy <= 64u - kRefillIdle)) {
                 if (id != kNone && cur == kDone && tri >= tri_end) {
-                    if (!kAny && tie) {
-                        ties[num_ties] = id;
-                        ties_at[num_ties++] = tmax;
+                    const bool sound = !found || sound_hit<kAny>(bvh, h.rec, sl, r, tmax);
+                    if (tie || !sound) {
+                        if (!kAny) ties_at[num_ties] = sound ? tmax : -INFINITY;
+                        ties[num_ties++] = id;
                     } else {
-                        h.t = tmax;
-                        if (!kAny && found) hit_weights(h);
                         sink(id, found, h, r);
                     }
                     id = kNone;
@@ -815,11 +888,11 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
                     float t, U, V, W, det;
                     if (kCount) cnt.tris++;
                     if (watertight(sh, a0, a1, a2, r.tmin, tmax, t, U, V, W, det))
-                        meet(tri, t, a0.w, V, W, det);
+                        meet(tri, t);
                     if (two && !(kAny && found)) {
                         if (kCount) cnt.tris++;
                         if (watertight(sh, b0, b1, b2, r.tmin, tmax, t, U, V, W, det))
-                            meet(tri + 1u, t, b0.w, V, W, det);
+                            meet(tri + 1u, t);
                     }
                     tri += 2u;
                     if (kAny && found) {
@@ -834,15 +907,16 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
                 take_leaf();
             }
         }
-        if constexpr (kAny) break;
         // All lanes are idle: nothing of the loop above is live here.
         while (num_ties > 0u) {
             num_ties--;
             const RayIn q = src(ties[num_ties]);
-            HitOut hx = trace_exact(bvh, q, ties_at[num_ties], st);
-            const bool hit = hx.prim != kNone;
-            if (hit) hit_weights(hx);
-            sink(ties[num_ties], hit, hx, q);
+            if constexpr (kAny) {
+                sink(ties[num_ties], occluded_exact(bvh, q, st), h, q);
+            } else {
+                h.rec = trace_exact(bvh, q, ties_at[num_ties], st);
+                sink(ties[num_ties], h.rec != kDone, h, q);
+            }
         }
         exhausted = cur_next >= (even ? cur_end : n);
         if (exhausted) break;
@@ -850,7 +924,7 @@ __device__ __forceinline__ void trace_persistent(const BvhDev& bvh, uint32_t n, 
         sl = Slab{};
         sh = ShearCyclic{};
         h = HitOut{};
-        tmax = sure_lo = sure_hi = 0.f;
+        tmax = 0.f;
         found = tie = false;
         id = kNone;
         cur = kDone;
@@ -910,8 +984,8 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
         const Slab sl = make_slab(r);
         const ShearCyclic sh = make_shear_cyclic(r);
         float tmax = r.tmax;
-        HitOut h{0.f, 0u, 0xffffffffu, 0.f, 0.f, 1.f};
-        bool mine = false;                // this lane met a triangle
+        HitOut h{};
+        float nearest = INFINITY;         // of the triangles this lane met: h.rec
         bool found = false, tie = false;  // of the ray
         uint32_t sp = 1u;
         wave_fence();
@@ -964,7 +1038,10 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
                         if (watertight(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det)) {
                             met = t < tmax;
                             same = !met && found;
-                            if (met) accept_hit<kAny>(h, t, tri, __float_as_uint(v0.w), V, W, det);
+                            if (met) {
+                                nearest = t;
+                                h.rec = tri;
+                            }
                         }
                     }
                     const bool any_met = ballot(met) != 0ull;
@@ -975,7 +1052,6 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
                     }
                     tie = tie || ballot(same) != 0ull;
                     if (any_met) {
-                        mine = mine || met;
                         found = true;
                         float m = met ? t : INFINITY;
 #pragma unroll
@@ -990,15 +1066,23 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
             if (lane == 0u) sink(i, found, h, r);
             continue;
         }
-        if (tie) {
-            // trace_exact's search for the first record at the nearest distance, a node's children or
-            // a leaf's records at once.
+        unsigned long long holders = ballot(found && nearest == tmax);
+        // The boxes were the built ones, but a hit before its own may have kept another from being met.
+        const bool sound = !found || ballot(nearest == tmax && !sound_hit<false>(bvh, h.rec, sl, r, tmax)) == 0ull;
+        if (tie || !sound) {
+            // As trace_exact, with a node's children or a leaf's records at once.
             const float band = 1000.f * distance_band(bvh, r, sh);
             float far = fminf(fmaf(tmax, 1.f + 1e-3f, band), r.tmax), near = fmaf(tmax, 1.f - 1e-3f, -band);
-            bool seen = false;
-            for (int pass = 0; pass < 2 && !seen; pass++, far = r.tmax, near = -INFINITY) {
+            bool first = sound;
+            for (;;) {
+                if (!first) {
+                    tmax = INFINITY;
+                    far = r.tmax;
+                    near = -INFINITY;
+                }
+                found = false;
                 if (lane == 0u) stack[0] = make_uint2(0u, 0u);
-                for (sp = 1u; sp > 0u && !seen;) {
+                for (sp = 1u; sp > 0u && !(first && found);) {
                     wave_fence();
                     const uint32_t ref = stack[--sp].x;
                     wave_fence();
@@ -1023,26 +1107,37 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
                         }
                     } else {
                         const uint32_t tri = (ref & kMaxLeafFirst) + lane;
-                        bool here = false;
-                        float t, U, V, W, det;
+                        float at = INFINITY;
                         if (lane <= ((ref >> 27) & 0xfu)) {
                             const float4* tp = reinterpret_cast<const float4*>(bvh.tris + tri);
                             const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
-                            here = watertight(sh, v0, v1, v2, r.tmin, tmax, t, U, V, W, det) && t == tmax;
-                            if (here) accept_hit<false>(h, t, tri, __float_as_uint(v0.w), V, W, det);
+                            float t, U, V, W, det, tn;
+                            if (watertight(sh, v0, v1, v2, r.tmin, far, t, U, V, W, det) && t < r.tmax) {
+                                (void)in_leaf_box(bvh.tris[tri], v1.w, v2.w, sl, r.tmin, r.tmax, tn);
+                                at = hit_order(t, tn);
+                            }
                         }
-                        const unsigned long long m = ballot(here);
-                        seen = m != 0ull;
-                        if (seen) mine = lane == uint32_t(__ffsll(static_cast<long long>(m)) - 1);
+                        float best = at;
+#pragma unroll
+                        for (int off = kLanes / 2; off > 0; off >>= 1) best = fminf(best, __shfl_xor(best, off, 64));
+                        if (first ? ballot(at == tmax) != 0ull : best < tmax) {
+                            if (!first) {
+                                tmax = best;
+                                far = fminf(best, r.tmax);
+                            }
+                            found = true;
+                            // Of equal ones the first record, the lowest lane's.
+                            holders = ballot(at == tmax);
+                            if (at == tmax) h.rec = tri;
+                        }
                     }
                 }
+                if (found || !first) break;
+                first = false;
             }
         }
-        const unsigned long long holders = ballot(mine && h.t == tmax);
         const bool lead = found ? lane == uint32_t(__ffsll(static_cast<long long>(holders)) - 1) : lane == 0u;
-        if (!lead) continue;
-        if (found) hit_weights(h);
-        sink(i, found, h, r);
+        if (lead) sink(i, found, h, r);
     }
 }
 
