@@ -104,11 +104,24 @@ def build_bvh_check() -> Path:
     return BVH_CHECK
 
 
+PACKED_CHECK = ROOT / "tests" / "native" / "packed_check"
+
+
+def build_packed_check() -> Path:
+    """The host-side checker of the packed nodes (the kernels' box arithmetic compiled in, no GPU)."""
+    tmp = PACKED_CHECK.with_name(PACKED_CHECK.name + ".tmp")
+    _run(["g++", *HOST_FLAGS, str(ROOT / "tests" / "native" / "packed_check.cpp"), str(CSRC / "bvh_build.cpp"), "-o",
+          str(tmp), "-lpthread"])
+    os.replace(tmp, PACKED_CHECK)
+    return PACKED_CHECK
+
+
 def build_all(jobs: int = 4) -> None:
     build_lib(jobs)
     build_plugin()
     build_driver()
     build_bvh_check()
+    build_packed_check()
 
 
 if __name__ == "__main__":

@@ -32,6 +32,7 @@
 // triangle found wins an exact tie (scene.qbvh.cpp:124-133).
 #pragma once
 
+#include "boxes.hpp"
 #include "bvh_build.h"
 #include "device_math.hpp"
 
@@ -235,53 +236,13 @@ __device__ __forceinline__ bool refine_fp64(const RayIn& r, float4 v0, float4 v1
     return true;
 }
 
-// Packed boxes: 1 + 2 gamma(8), gamma(n) = n u / (1 - n u), u = 2^-24.  Against the built box's test
-// (1 + 2 gamma(4)) each of the two distances is off by 3 more roundings, the node's offset
-// fma(origin, inv, offset), the step's product and the plane's own FMA, beyond what the planes'
-// margin covers: whatever the built box accepts the packed one accepts.
-constexpr float kBoxRobust = 1.0f + 2.0f * 4.8e-7f;
-// The same for a box whose planes are at hand: 1 + 2 gamma(4).
-constexpr float kBoxRobustExact = 1.0f + 2.0f * 2.4e-7f;
-// 1 - 4u: see hit_order.
-constexpr float kOrderScale = 1.0f - 2.384185791015625e-7f;
-
 // Hardware reciprocal (v_rcp_f32, within 1 ulp) of a direction component kept away from 0.
 __device__ __forceinline__ float safe_rcp(float d) {
     return __builtin_amdgcn_rcpf(fabsf(d) > 1e-30f ? d : copysignf(1e-30f, d));
 }
 
-// Per-ray constants of the slab test.  A plane at coordinate x is reached at
-// t = fma(x, inv, offset).  The offset fma(-o, inv, -+e) is -o * inv -+ e rounded once, so
-// fma(x, inv, offset) equals (x - o) * inv -+ e up to one rounding of the result and an
-// absolute error of about u |o * inv| (the offset's rounding); e = 4u |p| = 2^-22 |p|, with
-// p = o * inv, exceeds it, so moving the plane that is entered first (lo when inv >= 0)
-// earlier by e and the plane that is left last later by e leaves the entry and exit distances
-// with relative errors only, which kBoxRobust covers.  Coordinates are assumed below 1e8 in
-// magnitude so that o * inv stays finite for the clamped reciprocal (<= 1e30).
-// Per axis the ray knows which plane it enters first (lo when inv >= 0), so a select per axis
-// and node takes the near and far planes of all four children and no min / max orders them.
-struct Slab {
-    float ix, iy, iz;
-    float nx, fx, ny, fy, nz, fz;  // offsets of the near and far planes per axis
-};
-
-__device__ __forceinline__ void slab_axis(float o, float inv, float& near_off, float& far_off) {
-    const float e = fabsf(o * inv) * 2.384185791015625e-7f;  // 2^-22 |p|
-    const float lo = fmaf(-o, inv, inv >= 0.f ? -e : e);       // lo plane, moved away from the box's inside
-    const float hi = fmaf(-o, inv, inv >= 0.f ? e : -e);
-    near_off = inv >= 0.f ? lo : hi;
-    far_off = inv >= 0.f ? hi : lo;
-}
-
 __device__ __forceinline__ Slab make_slab(const RayIn& r) {
-    Slab s;
-    s.ix = safe_rcp(r.dx);
-    s.iy = safe_rcp(r.dy);
-    s.iz = safe_rcp(r.dz);
-    slab_axis(r.ox, s.ix, s.nx, s.fx);
-    slab_axis(r.oy, s.iy, s.ny, s.fy);
-    slab_axis(r.oz, s.iz, s.nz, s.fz);
-    return s;
+    return make_slab(r.ox, r.oy, r.oz, safe_rcp(r.dx), safe_rcp(r.dy), safe_rcp(r.dz));
 }
 
 // Orders two (key, reference) pairs, nearer first.  A pair is one 64-bit value, the key in the
@@ -307,60 +268,11 @@ constexpr uint32_t kPop = 0xfffffffeu;   // the next reference is on the stack (
 __device__ __forceinline__ bool is_inner(uint32_t ref) { return int(ref) >= 0; }
 __device__ __forceinline__ bool is_leaf(uint32_t ref) { return ref >= kLeafBit && ref < kPop; }
 
-// A node of the built tree in the form the kernels read.  Along each axis the children's planes
-// are 8-bit steps of ext / 254.9 from the lowest plane, lo planes rounded down and hi planes up
-// and moved out by at least kPlaneMargin steps more, which exceeds what evaluating
-// origin + q * scale along a ray can lose against the extent (3 roundings of 255 steps).
-// Step 0 is the lowest plane itself.  An empty slot's box is inverted (255, 0) and its child
-// word a one-record leaf: where rounding or NaN lets a ray in, the record's own test decides.
-constexpr double kPlaneMargin = 1.0 / 512;
-__device__ __forceinline__ NodeQ pack_node(const Node4& n) {
-    NodeQ q;
-    const float* lo[3] = {n.lo_x, n.lo_y, n.lo_z};
-    const float* hi[3] = {n.hi_x, n.hi_y, n.hi_z};
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        float l = INFINITY, h = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            if (n.child[i] == kEmptyChild) continue;
-            l = fminf(l, lo[a][i]);
-            h = fmaxf(h, hi[a][i]);
-        }
-        const double ext = double(h) - double(l);
-        const float step = ext > 0.0 ? fmaxf(float(ext * (1.0 / 254.9)), 1.17549435e-38f) : 0.f;
-        uint32_t ql = 0u, qh = 0u;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            uint32_t b0 = 255u, b1 = 0u;
-            if (n.child[i] != kEmptyChild) {
-                b0 = 0u;
-                if (step > 0.f) {
-                    const double s0 = (double(lo[a][i]) - double(l)) / double(step) - kPlaneMargin;
-                    const double s1 = (double(hi[a][i]) - double(l)) / double(step) + kPlaneMargin;
-                    b0 = uint32_t(fmax(floor(s0), 0.0));
-                    b1 = uint32_t(fmin(ceil(s1), 255.0));
-                }
-            }
-            ql |= b0 << (8 * i);
-            qh |= b1 << (8 * i);
-        }
-        q.origin[a] = l;
-        q.step[a] = step;
-        q.planes[a][0] = ql;
-        q.planes[a][1] = qh;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) q.child[i] = n.child[i] == kEmptyChild ? kLeafBit : n.child[i];
-    return q;
-}
-
 // Node words are fetched through a buffer resource over the node array: the
 // constant part of each fetch's offset goes into the instruction's offset field, so a fetch
 // costs one 32-bit address add (a global load needs 64-bit address arithmetic to fold it),
 // and the 64-bit temporaries' registers are freed.  The resource's record count, 2^32 - 1
-// bytes, lets every fetch of a tree within kMaxNodes nodes through (the last node's words
-// end 16 bytes before 2^32).
+// bytes, lets every fetch of a tree through: kMaxNodes packed nodes end at 2^31.
 struct NodeFetch {
     __amdgpu_buffer_rsrc_t rsrc;
     __device__ __forceinline__ explicit NodeFetch(const NodeQ* nodes)
@@ -371,36 +283,23 @@ struct NodeFetch {
     }
 };
 
-// Slab tests of the four children of node `cur` (Node4 words read by `fetch`), sorted into
-// entries (key = entry distance, reference), nearest first; a missed child's key is +inf.  Each
-// lane fetches the plane it enters first and the plane it leaves last per axis (byte offsets
-// from the ray's direction signs), so the entry and exit distances need no min / max per axis;
-// for a non-empty box they equal what ordering the two planes would give (fma rounds
-// monotonically), and the inverted box of an empty slot is never entered.
+// Slab tests of the four children of packed node `cur`, sorted into entries (key = entry distance,
+// reference), nearest first; a missed child's key is +inf.  Per axis the direction's sign selects
+// the planes entered first and left last of all four children, so the entry and exit distances
+// need no min / max per axis; the inverted box of an empty slot is entered only by rounding or NaN.
 __device__ __forceinline__ void node_children(const NodeFetch& fetch, uint32_t cur, const Slab& s, float tmin, float tmax,
                                               double e[4]) {
     // 32-bit byte offsets from the node array (at most kMaxNodes nodes, checked by the builder).
     const uint32_t o = cur * uint32_t(sizeof(NodeQ));
     const float4 q0 = fetch(o), q1 = fetch(o + 16u), q2 = fetch(o + 32u), q3 = fetch(o + 48u);
-    // The planes are origin + q * scale: along the ray fma(q, scale * inv, fma(origin, inv, offset)).
-    const float ax = q0.w * s.ix, ay = q1.x * s.iy, az = q1.y * s.iz;
-    const float bnx = fmaf(q0.x, s.ix, s.nx), bfx = fmaf(q0.x, s.ix, s.fx);
-    const float bny = fmaf(q0.y, s.iy, s.ny), bfy = fmaf(q0.y, s.iy, s.fy);
-    const float bnz = fmaf(q0.z, s.iz, s.nz), bfz = fmaf(q0.z, s.iz, s.fz);
-    const uint32_t lx = __float_as_uint(q1.z), hx = __float_as_uint(q1.w);
-    const uint32_t ly = __float_as_uint(q2.x), hy = __float_as_uint(q2.y);
-    const uint32_t lz = __float_as_uint(q2.z), hz = __float_as_uint(q2.w);
-    const uint32_t nx = s.ix >= 0.f ? lx : hx, fx = s.ix >= 0.f ? hx : lx;
-    const uint32_t ny = s.iy >= 0.f ? ly : hy, fy = s.iy >= 0.f ? hy : ly;
-    const uint32_t nz = s.iz >= 0.f ? lz : hz, fz = s.iz >= 0.f ? hz : lz;
+    const PackedAxis x = packed_axis(q0.x, q0.w, __float_as_uint(q1.z), __float_as_uint(q1.w), s.ix, s.nx, s.fx);
+    const PackedAxis y = packed_axis(q0.y, q1.x, __float_as_uint(q2.x), __float_as_uint(q2.y), s.iy, s.ny, s.fy);
+    const PackedAxis z = packed_axis(q0.z, q1.y, __float_as_uint(q2.z), __float_as_uint(q2.w), s.iz, s.nz, s.fz);
     const float c[4] = {q3.x, q3.y, q3.z, q3.w};
-    auto plane = [](uint32_t q, int i) { return float((q >> (8 * i)) & 0xffu); };
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const float tn = fmaxf(fmaxf(fmaf(plane(nx, i), ax, bnx), fmaf(plane(ny, i), ay, bny)),
-                               fmaxf(fmaf(plane(nz, i), az, bnz), tmin));
-        const float tf = fminf(fminf(fmaf(plane(fx, i), ax, bfx), fmaf(plane(fy, i), ay, bfy)),
-                               fminf(fmaf(plane(fz, i), az, bfz), tmax));
+        float tn, tf;
+        packed_span(x, y, z, i, tmin, tmax, tn, tf);
         e[i] = pack_entry(tn <= tf * kBoxRobust ? tn : INFINITY, __float_as_uint(c[i]));
     }
     cswap(e[0], e[1]);
@@ -539,12 +438,9 @@ __device__ __forceinline__ void sort4(float key[4], uint32_t val[4]) {
 __device__ __forceinline__ float built_child(const BvhDev& bvh, const Slab& s, uint32_t node, uint32_t i, float tmin,
                                              float tmax, uint32_t& child, float& tf) {
     const float* nd = reinterpret_cast<const float*>(bvh.exact + node) + i;
-    const float lx = nd[0], hx = nd[4], ly = nd[8], hy = nd[12], lz = nd[16], hz = nd[20];
     child = __float_as_uint(nd[24]);
-    const float tn = fmaxf(fmaxf(fmaf(s.ix >= 0.f ? lx : hx, s.ix, s.nx), fmaf(s.iy >= 0.f ? ly : hy, s.iy, s.ny)),
-                           fmaxf(fmaf(s.iz >= 0.f ? lz : hz, s.iz, s.nz), tmin));
-    tf = fminf(fminf(fmaf(s.ix >= 0.f ? hx : lx, s.ix, s.fx), fmaf(s.iy >= 0.f ? hy : ly, s.iy, s.fy)),
-               fminf(fmaf(s.iz >= 0.f ? hz : lz, s.iz, s.fz), tmax));
+    float tn;
+    box_span(s, nd[0], nd[4], nd[8], nd[12], nd[16], nd[20], tmin, tmax, tn, tf);
     return child != kEmptyChild && tn <= tf * kBoxRobustExact ? tn : INFINITY;
 }
 
@@ -554,10 +450,8 @@ __device__ __forceinline__ float built_child(const BvhDev& bvh, const Slab& s, u
 __device__ __forceinline__ bool in_leaf_box(const LeafTri& rec, float lx, float hx, const Slab& s, float tmin, float tmax,
                                             float& tn) {
     const float4 b = *reinterpret_cast<const float4*>(rec.box_yz);
-    tn = fmaxf(fmaxf(fmaf(s.ix >= 0.f ? lx : hx, s.ix, s.nx), fmaf(s.iy >= 0.f ? b.x : b.y, s.iy, s.ny)),
-               fmaxf(fmaf(s.iz >= 0.f ? b.z : b.w, s.iz, s.nz), tmin));
-    const float tf = fminf(fminf(fmaf(s.ix >= 0.f ? hx : lx, s.ix, s.fx), fmaf(s.iy >= 0.f ? b.y : b.x, s.iy, s.fy)),
-                           fminf(fmaf(s.iz >= 0.f ? b.w : b.z, s.iz, s.fz), tmax));
+    float tf;
+    box_span(s, lx, hx, b.x, b.y, b.z, b.w, tmin, tmax, tn, tf);
     return tn <= tf * kBoxRobustExact;
 }
 
