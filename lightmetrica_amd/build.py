@@ -116,12 +116,24 @@ def build_packed_check() -> Path:
     return PACKED_CHECK
 
 
+HOST_IO_CHECK = ROOT / "tests" / "native" / "host_io_check"
+
+
+def build_host_io_check() -> Path:
+    """The checker of the host copy team (no GPU)."""
+    tmp = HOST_IO_CHECK.with_name(HOST_IO_CHECK.name + ".tmp")
+    _run(["g++", *HOST_FLAGS, str(ROOT / "tests" / "native" / "host_io_check.cpp"), "-o", str(tmp), "-lpthread"])
+    os.replace(tmp, HOST_IO_CHECK)
+    return HOST_IO_CHECK
+
+
 def build_all(jobs: int = 4) -> None:
     build_lib(jobs)
     build_plugin()
     build_driver()
     build_bvh_check()
     build_packed_check()
+    build_host_io_check()
 
 
 if __name__ == "__main__":

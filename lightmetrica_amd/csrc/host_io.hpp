@@ -6,6 +6,7 @@
 #include <cstddef>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <unistd.h>
 #include <vector>
@@ -21,21 +22,19 @@ struct CopyJob {
 // Copies with up to kTeam host threads: one thread's memcpy is slower than the link, most of all
 // into pages that the caller has not touched yet.  The helpers are started by copies of at least
 // kShared bytes and stay until the team is destroyed; starting seven threads for each copy took
-// 0.1 to 0.3 ms.  Called by one thread at a time.
+// 0.1 to 0.3 ms.  Called by one thread at a time.  In a process forked from the one that started
+// them there are no helpers: a team copies alone there and leaves what the helpers wait on as it is.
 class CopyTeam {
 public:
     ~CopyTeam() {
-        if (helpers_.empty()) return;
-        if (getpid() != owner_) {  // a forked child has no such threads
-            for (auto& t : helpers_) t.detach();
-            return;
-        }
+        if (!crew_ || getpid() != owner_) return;
         {
-            std::lock_guard<std::mutex> lock(m_);
-            quit_ = true;
+            std::lock_guard<std::mutex> lock(crew_->m);
+            crew_->quit = true;
         }
-        wake_.notify_all();
-        for (auto& t : helpers_) t.join();
+        crew_->wake.notify_all();
+        for (auto& t : crew_->helpers) t.join();
+        delete crew_;
     }
 
     void run(const CopyJob* jobs, int njobs) {
@@ -45,19 +44,20 @@ public:
             for (int j = 0; j < njobs; j++) std::memcpy(jobs[j].dst, jobs[j].src, jobs[j].bytes);
             return;
         }
+        Crew& c = *crew_;
         {
-            std::lock_guard<std::mutex> lock(m_);
-            jobs_ = jobs;
-            njobs_ = njobs;
-            next_.store(0, std::memory_order_relaxed);
-            open_ = true;
-            call_++;
+            std::lock_guard<std::mutex> lock(c.m);
+            c.jobs = jobs;
+            c.njobs = njobs;
+            c.next.store(0, std::memory_order_relaxed);
+            c.open = true;
+            c.call++;
         }
-        wake_.notify_all();
-        work(jobs, njobs);
-        std::unique_lock<std::mutex> lock(m_);
-        open_ = false;  // a helper that wakes up later finds nothing to do
-        idle_.wait(lock, [&] { return working_ == 0; });
+        c.wake.notify_all();
+        c.work(jobs, njobs);
+        std::unique_lock<std::mutex> lock(c.m);
+        c.open = false;  // a helper that wakes up later finds nothing to do
+        c.idle.wait(lock, [&] { return c.working == 0; });
     }
 
 private:
@@ -65,60 +65,72 @@ private:
     static constexpr size_t kShared = size_t(512) << 10;  // below, waking the helpers costs more than it gives
     static constexpr size_t kPiece = size_t(256) << 10;
 
-    // Two more helpers a copy until the team is whole: starting one takes some 20 us.
+    // The helpers and what they share, on the heap: a forked process can destroy neither a thread that
+    // it does not have nor a condition that such a thread waits on.
+    struct Crew {
+        std::vector<std::thread> helpers;
+        std::mutex m;
+        std::condition_variable wake, idle;
+        const CopyJob* jobs = nullptr;
+        int njobs = 0;
+        std::atomic<size_t> next{0};
+        unsigned long long call = 0;
+        unsigned working = 0;
+        bool open = false, quit = false;
+
+        void work(const CopyJob* list, int n) {
+            for (;;) {
+                size_t p = next.fetch_add(1, std::memory_order_relaxed);
+                int j = 0;
+                for (; j < n; j++) {
+                    const size_t pieces = (list[j].bytes + kPiece - 1) / kPiece;
+                    if (p < pieces) break;
+                    p -= pieces;
+                }
+                if (j == n) return;
+                const size_t off = p * kPiece;
+                std::memcpy(list[j].dst + off, list[j].src + off, std::min(kPiece, list[j].bytes - off));
+            }
+        }
+
+        void help() {
+            unsigned long long seen = 0;
+            std::unique_lock<std::mutex> lock(m);
+            for (;;) {
+                wake.wait(lock, [&] { return quit || call != seen; });
+                if (quit) return;
+                seen = call;
+                if (!open) continue;
+                const CopyJob* list = jobs;
+                const int n = njobs;
+                working++;
+                lock.unlock();
+                work(list, n);
+                lock.lock();
+                if (--working == 0) idle.notify_one();
+            }
+        }
+    };
+
+    // Two more helpers a copy until the team is whole: starting one takes some 20 us.  False if there
+    // is none.
     bool start() {
-        owner_ = getpid();
+        if (!crew_) {
+            crew_ = new (std::nothrow) Crew;
+            owner_ = getpid();
+        }
+        if (!crew_ || getpid() != owner_) return false;
+        Crew* const c = crew_;
         const unsigned n = std::min(kTeam, std::max(1u, std::thread::hardware_concurrency())) - 1;
         try {
-            for (unsigned t = 0; t < 2 && helpers_.size() < n; t++) helpers_.emplace_back([this] { helper(); });
+            for (unsigned t = 0; t < 2 && c->helpers.size() < n; t++) c->helpers.emplace_back([c] { c->help(); });
         } catch (...) {
             // fewer helpers
         }
-        return !helpers_.empty();
+        return !c->helpers.empty();
     }
 
-    void work(const CopyJob* jobs, int njobs) {
-        for (;;) {
-            size_t p = next_.fetch_add(1, std::memory_order_relaxed);
-            int j = 0;
-            for (; j < njobs; j++) {
-                const size_t pieces = (jobs[j].bytes + kPiece - 1) / kPiece;
-                if (p < pieces) break;
-                p -= pieces;
-            }
-            if (j == njobs) return;
-            const size_t off = p * kPiece;
-            std::memcpy(jobs[j].dst + off, jobs[j].src + off, std::min(kPiece, jobs[j].bytes - off));
-        }
-    }
-
-    void helper() {
-        unsigned long long seen = 0;
-        std::unique_lock<std::mutex> lock(m_);
-        for (;;) {
-            wake_.wait(lock, [&] { return quit_ || call_ != seen; });
-            if (quit_) return;
-            seen = call_;
-            if (!open_) continue;
-            const CopyJob* jobs = jobs_;
-            const int njobs = njobs_;
-            working_++;
-            lock.unlock();
-            work(jobs, njobs);
-            lock.lock();
-            if (--working_ == 0) idle_.notify_one();
-        }
-    }
-
-    std::vector<std::thread> helpers_;
-    std::mutex m_;
-    std::condition_variable wake_, idle_;
-    const CopyJob* jobs_ = nullptr;
-    int njobs_ = 0;
-    std::atomic<size_t> next_{0};
-    unsigned long long call_ = 0;
-    unsigned working_ = 0;
-    bool open_ = false, quit_ = false;
+    Crew* crew_ = nullptr;
     pid_t owner_ = 0;
 };
 

@@ -1,0 +1,60 @@
+// Host-side check of the copy team (no GPU), run by tests/test_host_io.py:
+//   1. copies of any size and number arrive whole;
+//   2. a process forked from one whose team has helpers copies and destroys the team: the helpers are
+//      not its own, and it neither waits for them nor ends by them;
+//   3. nor when it destroys the team without a copy.
+#include <cstdio>
+#include <cstdlib>
+#include <sys/wait.h>
+
+#include "../../lightmetrica_amd/csrc/host_io.hpp"
+
+using namespace lmgpu;
+
+static bool copies(CopyTeam& team) {
+    bool ok = true;
+    for (size_t bytes : {size_t(1), size_t(1000), size_t(512) << 10, (size_t(512) << 10) + 1, (size_t(9) << 20) + 17}) {
+        std::vector<char> a(bytes), b(bytes + 2, 7), c(bytes / 3 + 1), d(bytes / 3 + 1, 9);
+        for (size_t i = 0; i < bytes; i++) a[i] = char(i * 31 + (i >> 9));
+        for (size_t i = 0; i < c.size(); i++) c[i] = char(i * 13 + 5);
+        const CopyJob jobs[2] = {{b.data() + 1, a.data(), bytes}, {d.data(), c.data(), c.size()}};
+        team.run(jobs, 2);
+        ok = ok && std::memcmp(a.data(), b.data() + 1, bytes) == 0 && b[0] == 7 && b[bytes + 1] == 7 && c == d;
+    }
+    return ok;
+}
+
+// Runs `child` in a forked process of a few seconds at most; its exit status, or -1 if a signal ended it.
+template <class F> static int forked(F&& child) {
+    std::fflush(stdout);
+    const pid_t pid = fork();
+    if (pid == 0) {
+        alarm(5);
+        _exit(child());
+    }
+    int status = 0;
+    waitpid(pid, &status, 0);
+    return WIFEXITED(status) ? WEXITSTATUS(status) : -1;
+}
+
+int main() {
+    int failures = 0;
+    CopyTeam* team = new CopyTeam;
+    for (int k = 0; k < 8; k++)
+        if (!copies(*team)) failures++, std::printf("copies differ\n");
+    if (forked([&] {
+            const bool ok = copies(*team);
+            delete team;
+            return ok ? 0 : 2;
+        }) != 0)
+        failures++, std::printf("a forked process that copied did not end well\n");
+    if (forked([&] {
+            delete team;
+            return 0;
+        }) != 0)
+        failures++, std::printf("a forked process that did not copy did not end well\n");
+    if (!copies(*team)) failures++, std::printf("copies differ after the forks\n");
+    delete team;
+    std::printf(failures ? "host_io_check: FAILED\n" : "host_io_check: OK\n");
+    return failures ? 1 : 0;
+}
