@@ -8,6 +8,7 @@
 #include <mutex>
 #include <new>
 #include <thread>
+#include <type_traits>
 #include <unistd.h>
 #include <vector>
 
@@ -146,6 +147,37 @@ struct HostIo {
 constexpr size_t kPinnedWords = 256;
 constexpr size_t kIdleIos = 4;
 constexpr size_t kIdlePinned = size_t(64) << 20;
+// The pool itself, which knows no HIP: release() hands back what is to be freed.  Nothing in it throws
+// (a context is destroyed through a C entry), and it is trivially destroyed: contexts may be destroyed
+// after static objects are.
+class HostIoPool {
+public:
+    void context() {
+        std::lock_guard<std::mutex> lock(m_);
+        contexts_++;
+    }
+    HostIo* acquire() {  // nullptr if there is no memory for it
+        std::lock_guard<std::mutex> lock(m_);
+        return num_idle_ ? idle_[--num_idle_] : new (std::nothrow) HostIo;
+    }
+    // A context is destroyed; io may be nullptr.  Returns how many of `gone` are to be freed.
+    size_t release(HostIo* io, HostIo* (&gone)[kIdleIos + 1]) {
+        std::lock_guard<std::mutex> lock(m_);
+        size_t n = 0;
+        if (io && num_idle_ < kIdleIos && io->bytes <= kIdlePinned) idle_[num_idle_++] = io;
+        else if (io) gone[n++] = io;
+        if (--contexts_ == 0)
+            while (num_idle_) gone[n++] = idle_[--num_idle_];
+        return n;
+    }
+
+private:
+    std::mutex m_;
+    HostIo* idle_[kIdleIos] = {};
+    size_t num_idle_ = 0, contexts_ = 0;
+};
+static_assert(std::is_trivially_destructible_v<HostIoPool>, "the pool outlives static objects");
+
 void host_io_context();  // a context is created
 HostIo* host_io_acquire();  // nullptr if there is no memory for it
 void host_io_release(HostIo* io);  // a context is destroyed; io may be nullptr

@@ -69,49 +69,16 @@ void dev_free(void* p) {
     if (p) (void)hipFree(p);
 }
 
-// Left to the process at its end: the runtime may be gone before static objects are.
-struct HostIoPool {
-    std::mutex m;
-    std::vector<HostIo*> idle;
-    size_t contexts = 0;
-};
-static HostIoPool& host_io_pool() {
-    static HostIoPool* pool = new HostIoPool;
-    return *pool;
-}
-static void host_io_free(HostIo* io) {
-    if (io->pinned) (void)hipHostFree(io->pinned);
-    delete io;
-}
-
-void host_io_context() {
-    HostIoPool& pool = host_io_pool();
-    std::lock_guard<std::mutex> lock(pool.m);
-    pool.contexts++;
-}
-
-HostIo* host_io_acquire() {
-    HostIoPool& pool = host_io_pool();
-    std::lock_guard<std::mutex> lock(pool.m);
-    if (pool.idle.empty()) return new (std::nothrow) HostIo;
-    HostIo* io = pool.idle.back();
-    pool.idle.pop_back();
-    return io;
-}
-
+static HostIoPool g_host_io_pool;
+void host_io_context() { g_host_io_pool.context(); }
+HostIo* host_io_acquire() { return g_host_io_pool.acquire(); }
 void host_io_release(HostIo* io) {
-    HostIoPool& pool = host_io_pool();
-    std::vector<HostIo*> gone;
-    {
-        std::lock_guard<std::mutex> lock(pool.m);
-        if (io && pool.idle.size() < kIdleIos && io->bytes <= kIdlePinned) pool.idle.push_back(io);
-        else if (io) gone.push_back(io);
-        if (--pool.contexts == 0) {
-            gone.insert(gone.end(), pool.idle.begin(), pool.idle.end());
-            pool.idle.clear();
-        }
+    HostIo* gone[kIdleIos + 1];
+    const size_t n = g_host_io_pool.release(io, gone);
+    for (size_t k = 0; k < n; k++) {
+        if (gone[k]->pinned) (void)hipHostFree(gone[k]->pinned);
+        delete gone[k];
     }
-    for (HostIo* g : gone) host_io_free(g);
 }
 
 bool ensure_pinned(lmgpu_ctx* ctx, size_t bytes) {

@@ -2,7 +2,9 @@
 //   1. copies of any size and number arrive whole;
 //   2. a process forked from one whose team has helpers copies and destroys the team: the helpers are
 //      not its own, and it neither waits for them nor ends by them;
-//   3. nor when it destroys the team without a copy.
+//   3. nor when it destroys the team without a copy;
+//   4. the pool keeps at most kIdleIos of what contexts leave, gives all back with the last of them, and
+//      needs no memory to do so.
 #include <cstdio>
 #include <cstdlib>
 #include <sys/wait.h>
@@ -10,6 +12,42 @@
 #include "../../lightmetrica_amd/csrc/host_io.hpp"
 
 using namespace lmgpu;
+
+static bool no_memory = false;
+__attribute__((noinline)) void* operator new(size_t n) {
+    void* p = no_memory ? nullptr : std::malloc(n);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+__attribute__((noinline)) void operator delete(void* p) noexcept { std::free(p); }
+__attribute__((noinline)) void operator delete(void* p, size_t) noexcept { std::free(p); }
+
+static bool pool_gives_back() {
+    HostIoPool pool;
+    HostIo* ios[kIdleIos + 3];
+    HostIo* gone[kIdleIos + 1];
+    bool ok = true;
+    size_t freed = 0;
+    for (HostIo*& io : ios) {
+        pool.context();
+        ok = ok && (io = pool.acquire()) != nullptr;
+    }
+    ios[0]->bytes = kIdlePinned + 1;
+    no_memory = true;
+    try {
+        for (HostIo* io : ios) {
+            const size_t n = pool.release(io, gone);
+            for (size_t k = 0; k < n; k++) delete gone[k];
+            freed += n;
+            const bool last = io == ios[kIdleIos + 2];
+            ok = ok && (last || n == (io == ios[0] || io == ios[kIdleIos + 1] ? 1u : 0u));
+        }
+    } catch (...) {
+        ok = false;
+    }
+    no_memory = false;
+    return ok && freed == kIdleIos + 3;
+}
 
 static bool copies(CopyTeam& team) {
     bool ok = true;
@@ -55,6 +93,7 @@ int main() {
         failures++, std::printf("a forked process that did not copy did not end well\n");
     if (!copies(*team)) failures++, std::printf("copies differ after the forks\n");
     delete team;
+    if (!pool_gives_back()) failures++, std::printf("the pool keeps or loses something\n");
     std::printf(failures ? "host_io_check: FAILED\n" : "host_io_check: OK\n");
     return failures ? 1 : 0;
 }
