@@ -224,8 +224,10 @@ lmgpu_status lmgpu_bvh_build(lmgpu_ctx* ctx, const lmgpu_bvh_params* params, lmg
 /* Host rays and results (device flags clear) go through pinned host memory, copied by up to 8
  * host threads: up to 1024 rays are read and written there by the kernels, up to 65536 are
  * copied to the device and back in one piece, more in chunks, with uploads, kernels and
- * read-backs overlapped on two extra streams of the context.  The call
- * returns when the host results are written; with device buffers it only enqueues. */
+ * read-backs overlapped on two extra streams of the context.  Below 2^20 rays a context takes
+ * more than 512 KB of pinned memory only after calls enough to pay for it; until then it uses the
+ * runtime's copies, with the same results.  The call returns when the host results are written;
+ * with device buffers it only enqueues. */
 lmgpu_status lmgpu_trace_closest(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uint32_t n, lmgpu_hits_soa* hits,
                                  uint32_t flags);
 lmgpu_status lmgpu_trace_any(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uint32_t n, uint8_t* occluded,

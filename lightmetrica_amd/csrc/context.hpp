@@ -180,12 +180,17 @@ void dev_free(void* p);
 // Grows the context's pinned memory to at least `bytes` (its contents are lost); false if it cannot
 // be had.
 bool ensure_pinned(lmgpu_ctx* ctx, size_t bytes);
+// HostIo::pays of the context's pinned memory.
+bool pinned_pays(lmgpu_ctx* ctx, size_t need, double saved_us, double more_us = 0.0);
 bool ensure_io_events(lmgpu_ctx* ctx);
 constexpr size_t kReadSlot = size_t(2) << 20;
 constexpr size_t kReadSlots = 4;
+// Whether read_back takes a film of this many bytes through the ring of pinned slots (of at most
+// kPinnedWords + kReadSlots * kReadSlot bytes).
+bool ring_pays(lmgpu_ctx* ctx, size_t bytes);
 // Copies device results to a host array, behind the work on the context's stream; returns when
 // they are there.
-hipError_t read_back(lmgpu_ctx* ctx, void* dst, const void* src, size_t bytes);
+hipError_t read_back(lmgpu_ctx* ctx, void* dst, const void* src, size_t bytes, bool ring);
 
 // Times `launch` with HIP events on the context stream when timing is enabled.
 template <class Fn> hipError_t timed(lmgpu_ctx* ctx, int cls, Fn&& launch) {

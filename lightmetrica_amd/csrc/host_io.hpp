@@ -137,12 +137,34 @@ private:
 
 // What a context needs to move host arrays: pinned memory, its first kPinnedWords bytes for small
 // results, and a team.  A destroyed context leaves it to the next one, since fresh pinned memory
-// costs 0.4 ms a megabyte when the host first touches it: at most kIdleIos of them are kept, with
+// costs 0.39 ms a MiB when the host first touches it: at most kIdleIos of them are kept, with
 // up to kIdlePinned bytes each, and all are freed with the last context (host_io_release).
 struct HostIo {
     void* pinned = nullptr;
     size_t bytes = 0;
     CopyTeam team;
+
+    // Whether a call that would save `saved_us` takes its way through `need` bytes of pinned memory,
+    // which `more_us` of other preparation (0 once done) has to go before.  Fresh pinned pages cost the
+    // host 0.39 ms a MiB (kTouchUs: 8 MiB 2.9 ms, 31 MiB 12.2), many times what one call saves, so calls
+    // take the runtime's way until what they would have saved has paid for them: a program that renders
+    // one image loses nothing, one that goes on never more than it spent.  First calls in a process
+    // with all of it pinned at once, and before (us): a raycast of 1280 x 720 2600, 1040; 65000 rays
+    // 1000, 510; 300,000 rays 13,000, 1380.  Up to kPinAtOnce the two are alike (10,000 rays 356, 358).
+    bool pays(size_t need, double saved_us, double more_us = 0.0) {
+        const bool fresh = need > bytes && need > kPinAtOnce;
+        if (!fresh && more_us == 0.0) return true;
+        saved_ += saved_us;
+        if (saved_ < (fresh ? double(need) * (kTouchUs / (1 << 20)) : 0.0) + more_us) return false;
+        saved_ = 0.0;
+        return true;
+    }
+
+    static constexpr double kTouchUs = 390.0;  // a MiB
+    static constexpr size_t kPinAtOnce = size_t(512) << 10;
+
+private:
+    double saved_ = 0.0;
 };
 constexpr size_t kPinnedWords = 256;
 constexpr size_t kIdleIos = 4;

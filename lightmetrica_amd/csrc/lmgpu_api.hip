@@ -81,6 +81,11 @@ void host_io_release(HostIo* io) {
     }
 }
 
+bool pinned_pays(lmgpu_ctx* ctx, size_t need, double saved_us, double more_us) {
+    if (!ctx->io && !(ctx->io = host_io_acquire())) return false;
+    return ctx->io->pays(need, saved_us, more_us);
+}
+
 bool ensure_pinned(lmgpu_ctx* ctx, size_t bytes) {
     if (!ctx->io && !(ctx->io = host_io_acquire())) return false;
     HostIo& io = *ctx->io;
@@ -120,11 +125,16 @@ bool ensure_io_events(lmgpu_ctx* ctx) {
 // 133, 537 and 1004 KB take 38, 66 and 91 us so, 45, 83 and 101 through the ring; 1312 KB 121 and
 // 108, 1735 KB 139 and 126.
 constexpr size_t kRingFrom = size_t(1152) << 10;
-hipError_t read_back(lmgpu_ctx* ctx, void* dst, const void* src, size_t bytes) {
+bool ring_pays(lmgpu_ctx* ctx, size_t bytes) {
+    // 36 us a MiB saved by the raycast above, 90 by the film of 50 MB.
+    return bytes >= kRingFrom && pinned_pays(ctx, kPinnedWords + std::min(bytes, kReadSlots * kReadSlot),
+                                             double(bytes) * (36.0 / (1 << 20)));
+}
+
+hipError_t read_back(lmgpu_ctx* ctx, void* dst, const void* src, size_t bytes, bool ring) {
     const hipStream_t s = ctx->stream;
     const size_t chunks = (bytes + kReadSlot - 1) / kReadSlot;
-    if (bytes < kRingFrom ||
-        !ensure_pinned(ctx, kPinnedWords + std::min(bytes, kReadSlots * kReadSlot)) || !ensure_io_events(ctx)) {
+    if (!ring || !ensure_pinned(ctx, kPinnedWords + std::min(bytes, kReadSlots * kReadSlot)) || !ensure_io_events(ctx)) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
@@ -664,7 +674,11 @@ lmgpu_status prepare_rays(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uint32_t n
 // c - 1 out to them.  A chunk may go to another kernel than the whole batch would (a last one of few
 // rays, several lanes to each); a ray's result is the same in every one (hit_order, traverse.hpp).
 // 81 rays 210 -> 34 us (eight copies in and four out before); 512 rays direct 36 us, copied 39; 4000
-// rays 63 and 61.  65536 rays 445 -> 255 us, 1M rays 2.7 -> 1.6 ms.
+// rays 63 and 61.  65,000 rays 421 -> 240 us, 300,000 rays 900 -> 755 us, 1M rays 2.7 -> 1.6 ms; so
+// much is saved a MiB, and once it has paid for the pinned memory and the two streams (3 to 6 ms
+// each to make) a batch goes this way (HostIo::pays), from kPipeAlways rays on at once.
+constexpr double kPieceUs = 58.0, kChunksUs = 15.0, kStreamsUs = 7000.0;
+constexpr uint32_t kPipeAlways = 1u << 20;
 constexpr uint32_t kDirectRays = 1024;
 constexpr uint32_t kPipeChunk = 1u << 19;
 constexpr uint32_t kPipeMinChunk = 1u << 16;
@@ -690,7 +704,7 @@ struct HostOut {
 // Traces n host rays in chunks (see kPipeChunk); `launch(dev_rays, m, dev_out)` enqueues on
 // the context's stream the kernels for m rays whose eight columns are dev_rays[0..7] and
 // whose result columns start at dev_out[j].  Returns LMGPU_ERR_UNSUPPORTED, having done
-// nothing, when the pinned memory or the copy streams cannot be had.
+// nothing, when the pinned memory or the copy streams cannot be had or do not pay yet.
 template <class Launch>
 lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, uint32_t n, const HostOut* outs,
                                   int nout, Launch&& launch, const char* what) {
@@ -701,7 +715,8 @@ lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, ui
     for (int j = 0; j < nout; j++) elems += outs[j].elem;
     if (n <= kPipeMinChunk) {
         const size_t in = size_t(n) * 32, out = size_t(n) * elems;
-        if (!ensure_pinned(ctx, in + out)) return LMGPU_ERR_UNSUPPORTED;
+        if (!pinned_pays(ctx, in + out, double(in + out) * (kPieceUs / (1 << 20))) || !ensure_pinned(ctx, in + out))
+            return LMGPU_ERR_UNSUPPORTED;
         char* const pinned = static_cast<char*>(ctx->io->pinned);
         char* dev = pinned;
         CopyJob jobs[8];
@@ -735,6 +750,9 @@ lmgpu_status trace_host_pipelined(lmgpu_ctx* ctx, const lmgpu_rays_soa* rays, ui
     const size_t quarter = (size_t(n) + 4 * kPipeMinChunk - 1) / (4 * kPipeMinChunk) * kPipeMinChunk;
     const size_t chunk = std::min<size_t>(kPipeChunk, std::max<size_t>(kPipeMinChunk, quarter));
     const size_t slot = (chunk * (32 + elems) + 255) / 256 * 256;
+    if (n < kPipeAlways && !pinned_pays(ctx, 2 * slot, double(n) * double(32 + elems) * (kChunksUs / (1 << 20)),
+                                        ctx->copy_streams[1] ? 0.0 : kStreamsUs))
+        return LMGPU_ERR_UNSUPPORTED;
     if (!ensure_pipeline(ctx, 2 * slot)) return LMGPU_ERR_UNSUPPORTED;
     lmgpu_status st = stage(ctx, 2 * slot);
     if (st != LMGPU_OK) return st;

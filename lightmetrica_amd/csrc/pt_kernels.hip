@@ -1896,6 +1896,7 @@ struct Pipeline {
 // A film of up to this many bytes is resolved into pinned host memory: the link takes it as fast as
 // a copy would, without the copy's launch.
 constexpr size_t kDirectFilm = (size_t(1) << 20) - kPinnedWords;
+constexpr double kDirectUs = 80.0;  // a MiB so saved: the room at 256 x 256 (768 KB) 395 -> 335 us
 
 lmgpu_status run_raycast(lmgpu_ctx* ctx, lmgpu_film* film) {
     if (!ctx->has_bvh) return fail(ctx, LMGPU_ERR_NO_BVH, "lmgpu_raycast_render: build the BVH first");
@@ -1938,7 +1939,7 @@ lmgpu_status run_raycast(lmgpu_ctx* ctx, lmgpu_film* film) {
                                static_cast<float*>(out_dev));
     });
     if (e != hipSuccess) return hip_fail(ctx, e, "k_raycast");
-    e = film->device ? hipStreamSynchronize(s) : read_back(ctx, film->data, out_dev, out_bytes);
+    e = film->device ? hipStreamSynchronize(s) : read_back(ctx, film->data, out_dev, out_bytes, ring_pays(ctx, out_bytes));
     if (e != hipSuccess) return hip_fail(ctx, e, "raycast readback");
     return LMGPU_OK;
 }
@@ -1967,8 +1968,10 @@ lmgpu_status run_pt(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_film* film, 
     void* out_dev = film->data;
     // The pinned memory is grown here, before it holds the words.
     const bool small = !film->device && out_bytes <= kDirectFilm;
-    const bool pinned = ensure_pinned(ctx, kPinnedWords + (film->device ? 0 : std::min(out_bytes, kReadSlots * kReadSlot)));
-    const bool direct = small && pinned;
+    const bool ring = !film->device && ring_pays(ctx, out_bytes);
+    const bool in_place = small && pinned_pays(ctx, kPinnedWords + out_bytes, double(out_bytes) * (kDirectUs / (1 << 20)));
+    const bool pinned = ensure_pinned(ctx, kPinnedWords + (ring || in_place ? std::min(out_bytes, kReadSlots * kReadSlot) : 0));
+    const bool direct = in_place && pinned;
     unsigned long long words_here[4];
     void* const words = pinned ? ctx->io->pinned : words_here;
     if (direct) {
@@ -2042,7 +2045,7 @@ lmgpu_status run_pt(lmgpu_ctx* ctx, const lmgpu_pt_params* p, lmgpu_film* film, 
     unsigned long long totals[2] = {0, 0};
     if (st == LMGPU_OK) {
         hipError_t e = pinned ? hipSuccess : hipMemcpyAsync(words, pl.b.totals, sizeof(totals), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = film->device || direct ? hipStreamSynchronize(s) : read_back(ctx, film->data, out_dev, out_bytes);
+        if (e == hipSuccess) e = film->device || direct ? hipStreamSynchronize(s) : read_back(ctx, film->data, out_dev, out_bytes, ring);
         if (e != hipSuccess) st = hip_fail(ctx, e, "pt readback");
         else std::memcpy(totals, words, sizeof(totals));
         if (e == hipSuccess && direct) {

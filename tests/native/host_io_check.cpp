@@ -4,7 +4,9 @@
 //      not its own, and it neither waits for them nor ends by them;
 //   3. nor when it destroys the team without a copy;
 //   4. the pool keeps at most kIdleIos of what contexts leave, gives all back with the last of them, and
-//      needs no memory to do so.
+//      needs no memory to do so;
+//   5. pinned memory is taken once the calls without it have paid for it, and at once where it is there
+//      or small.
 #include <cstdio>
 #include <cstdlib>
 #include <sys/wait.h>
@@ -62,6 +64,23 @@ static bool copies(CopyTeam& team) {
     return ok;
 }
 
+static bool pays_in_time() {
+    const size_t mib = size_t(1) << 20;
+    HostIo io;
+    bool ok = io.pays(HostIo::kPinAtOnce, 0.0);
+    // 8 MiB for calls that save 400 us each: 3120 us, the eighth call's.
+    for (int k = 1; k <= 8; k++) ok = ok && io.pays(8 * mib, 400.0) == (k == 8);
+    ok = ok && !io.pays(8 * mib, 400.0);  // not had, for want of memory: asked for again as seldom
+    io.bytes = 8 * mib;
+    ok = ok && io.pays(8 * mib, 0.0) && io.pays(3 * mib, 0.0);
+    HostIo streams;  // with 7000 us to prepare besides, then without
+    streams.bytes = 8 * mib;
+    for (int k = 1; k <= 7; k++) ok = ok && streams.pays(8 * mib, 1000.0, 7000.0) == (k == 7);
+    ok = ok && streams.pays(8 * mib, 1.0);
+    HostIo large;  // a call that pays for it by itself
+    return ok && large.pays(8 * mib, 4000.0);
+}
+
 // Runs `child` in a forked process of a few seconds at most; its exit status, or -1 if a signal ended it.
 template <class F> static int forked(F&& child) {
     std::fflush(stdout);
@@ -94,6 +113,7 @@ int main() {
     if (!copies(*team)) failures++, std::printf("copies differ after the forks\n");
     delete team;
     if (!pool_gives_back()) failures++, std::printf("the pool keeps or loses something\n");
+    if (!pays_in_time()) failures++, std::printf("pinned memory is taken too early or too late\n");
     std::printf(failures ? "host_io_check: FAILED\n" : "host_io_check: OK\n");
     return failures ? 1 : 0;
 }
