@@ -125,11 +125,11 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_any_grouped(BvhDev bvh, R
 // t and weights.  Otherwise as k_refine_fp64.  16M rays against 1M triangles, the traversal storing
 // all four results: 3.20 ms, with this pass 3.09; 70k to 1M rays the same either way.
 __global__ __launch_bounds__(256) void k_result_fp32(const LeafTri* __restrict__ tris, RaysSoA rays, uint32_t n,
-                                                     float* __restrict__ t_out, float* __restrict__ b0_out,
-                                                     float* __restrict__ b1_out, int32_t* __restrict__ prim_out) {
+                                                     const int32_t* rec_in, float* t_out, float* b0_out,
+                                                     float* b1_out, int32_t* prim_out) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n) return;
-    const int32_t rec = __builtin_nontemporal_load(prim_out + i);
+    const int32_t rec = __builtin_nontemporal_load(rec_in + i);
     float t = -1.f, b0 = 0.f, b1 = 0.f;
     int32_t prim = -1;
     if (rec >= 0) {
@@ -152,19 +152,20 @@ __global__ __launch_bounds__(256) void k_result_fp32(const LeafTri* __restrict__
     __builtin_nontemporal_store(prim, prim_out + i);
 }
 
-// The hits of k_trace_record, evaluated in FP64 (refine_fp64): prim holds the leaf-order record
-// of the winner (-1 for a miss), replaced here by its scene-order id.  Only the origin and
+// The hits of k_trace_record, evaluated in FP64 (refine_fp64): rec_in, one of the results' columns,
+// holds the leaf-order record of the winner (-1 for a miss).  Only the origin and
 // direction of a hit ray are read.  Where the FP64 determinant is 0 the traversal's FP32
 // values are computed again.  The streamed arrays are read and written non-temporally, which
 // keeps more of the BVH cached for the next traversal (-1.3 % for the pair of kernels on the
 // 16M-ray batch).
 __global__ __launch_bounds__(256) void k_refine_fp64(const LeafTri* __restrict__ tris, RaysSoA rays, uint32_t n,
-                                                     float* __restrict__ t_out, float* __restrict__ b0_out,
-                                                     float* __restrict__ b1_out, int32_t* __restrict__ prim_out) {
+                                                     const int32_t* rec_in, float* t_out, float* b0_out,
+                                                     float* b1_out, int32_t* prim_out) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n) return;
-    const int32_t rec = __builtin_nontemporal_load(prim_out + i);
+    const int32_t rec = __builtin_nontemporal_load(rec_in + i);
     float t = -1.f, b0 = 0.f, b1 = 0.f;
+    int32_t prim = -1;
     if (rec >= 0) {
         const float4* tp = reinterpret_cast<const float4*>(tris + rec);
         const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
@@ -183,11 +184,12 @@ __global__ __launch_bounds__(256) void k_refine_fp64(const LeafTri* __restrict__
             b0 = h.b0;
             b1 = h.b1;
         }
-        __builtin_nontemporal_store(__float_as_int(v0.w), prim_out + i);
+        prim = __float_as_int(v0.w);
     }
     __builtin_nontemporal_store(t, t_out + i);
     __builtin_nontemporal_store(b0, b0_out + i);
     __builtin_nontemporal_store(b1, b1_out + i);
+    if (rec >= 0 || rec_in != prim_out) __builtin_nontemporal_store(prim, prim_out + i);
 }
 
 __global__ __launch_bounds__(kTraceBlock) void k_trace_any_brute(const TriRecord* __restrict__ tris, uint32_t ntris,
@@ -298,6 +300,22 @@ hipError_t launch_pack_nodes(lmgpu_ctx* ctx) {
     return hipGetLastError();
 }
 
+// The results' column that carries the records from the traversal to the pass after it, which reads the
+// rays again: one that lies in none of the rays' (a caller may have its results written over its rays);
+// nullptr if there is none.
+static int32_t* record_column(const float* const* rays, uint32_t n, float* t, float* b0, float* b1, int32_t* prim) {
+    for (void* c : {static_cast<void*>(prim), static_cast<void*>(t), static_cast<void*>(b0), static_cast<void*>(b1)}) {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(c), bytes = uintptr_t(n) * 4u;
+        bool apart = true;
+        for (int k = 0; k < 8; k++) {
+            const uintptr_t r = reinterpret_cast<uintptr_t>(rays[k]);
+            apart = apart && (at + bytes <= r || r + bytes <= at);
+        }
+        if (apart) return static_cast<int32_t*>(c);
+    }
+    return nullptr;
+}
+
 hipError_t launch_trace_closest(lmgpu_ctx* ctx, const float* const* rays, uint32_t n, float* t, float* b0, float* b1,
                                 int32_t* prim, bool refine, uint32_t* next) {
     if (n > kMaxBatch) {
@@ -317,7 +335,8 @@ hipError_t launch_trace_closest(lmgpu_ctx* ctx, const float* const* rays, uint32
                 hipLaunchKernelGGL(k_trace_closest_brute<false>, dim3(brute_blocks(ctx, n)), block, 0, ctx->stream,
                                    ctx->tris.ptr, ntris, soa_of(rays), n, t, b0, b1, prim);
         });
-    if (n <= kGroup16Closest)
+    int32_t* const rec = record_column(rays, n, t, b0, b1, prim);
+    if (n <= kGroup16Closest || !rec)  // the grouped kernels write a ray's results when they have read it
         return timed(ctx, kKTraceClosest, [&]() {
             const bool whole = n <= kGroup64Rays;
             auto kernel = refine ? (whole ? k_trace_closest_grouped<true, 64> : k_trace_closest_grouped<true, 16>)
@@ -328,9 +347,9 @@ hipError_t launch_trace_closest(lmgpu_ctx* ctx, const float* const* rays, uint32
     return timed(ctx, kKTraceClosest, [&]() {
         hipLaunchKernelGGL(k_zero_next, dim3(1), dim3(64), 0, ctx->stream, next);
         hipLaunchKernelGGL(k_trace_record, dim3(persistent_blocks(ctx, k_trace_record, n)), block, 0, ctx->stream,
-                           bvh_of(ctx), soa_of(rays), n, next, prim);
+                           bvh_of(ctx), soa_of(rays), n, next, rec);
         hipLaunchKernelGGL(refine ? k_refine_fp64 : k_result_fp32, dim3((n + 255u) / 256u), dim3(256), 0, ctx->stream,
-                           ctx->leaf_tris.ptr, soa_of(rays), n, t, b0, b1, prim);
+                           ctx->leaf_tris.ptr, soa_of(rays), n, rec, t, b0, b1, prim);
     });
 }
 
