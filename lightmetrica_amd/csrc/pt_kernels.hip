@@ -1507,9 +1507,14 @@ __global__ void k_grad_out(const double* p, uint32_t nmat, uint32_t n, double w,
 // ---------------------------------------------------------------------------------
 // Host driver
 
-// The camera stage orders its rays by screen tile when the BVH is at least as large as one XCD's
-// L2 (4 MB); a smaller one stays in the caches whatever the order, and the sort would only
-// add its own time (room: 0.90 -> 1.01 ms; 7.4 MB gradient scene: 11.35 -> 10.72 ms).
+// The camera stage orders its rays by screen tile from this size of the tree as it is built (Node4 and
+// TriRecord, some 55,000 triangles) on.  One XCD's L2 is as large; with the 128-byte nodes that the
+// kernels read when the line was drawn a smaller tree stayed in the caches whatever the order (room:
+// 0.90 -> 1.01 ms; 96k triangles: 11.35 -> 10.72).  With packed nodes the samples matter more than
+// the tree, in ms ordered and not: 4.1M samples, terrain of 0.5M triangles 2.09 and 1.91 (compensated
+// film 1.90 and 2.02), city of 1M 2.22 and 1.98, 48k to 55k triangles 3.61 and 3.36; 8.4M, 96k
+// triangles 7.22 and 6.98; 7.4M, city of 1M 3.04 and 3.14; 16.6M, terrain 6.08 and 6.29 (FP64 film
+// 5.29 and 6.07); 66M, city of 16M 26.6 and 29.4; 133M, terrain of 2M 42.0 and 48.2.
 constexpr uint64_t kOrderMinBvhBytes = uint64_t(4) << 20;
 
 hipError_t sort_tile_keys(void* temp, size_t& temp_bytes, const uint32_t* keys_in, uint32_t* keys_out,
@@ -1721,7 +1726,7 @@ struct Pipeline {
         // raster numbers follow key_skip others in each stream.
         c.order = nullptr;
         key_skip = is_pt ? 0 : 4 + (p->rr_depth != -1 && p->rr_depth <= 1 ? 1 : 0);
-        const uint64_t bvh_bytes = uint64_t(ctx->nodes.count) * sizeof(NodeQ) + uint64_t(ctx->leaf_tris.count) * sizeof(LeafTri);
+        const uint64_t bvh_bytes = uint64_t(ctx->nodes.count) * sizeof(Node4) + uint64_t(ctx->num_records) * sizeof(TriRecord);
         if (bvh_bytes >= kOrderMinBvhBytes) {
             const uint32_t tiles = uint32_t(std::max((ctx->cam.width + 7) / 8, (ctx->cam.height + 7) / 8));
             key_bits = 2;
@@ -1755,7 +1760,7 @@ struct Pipeline {
         if (!counters_clear)
             hipLaunchKernelGGL(k_zero_u32, dim3(2), dim3(256), 0, s, b.counters, uint32_t(4 * kMaxSegments));
         counters_clear = false;
-        const dim3 grid_b((nb + kPTBlock - 1) / kPTBlock), grid_c((cap + kPTBlock - 1) / kPTBlock);
+        const dim3 grid_b((nb + kPTBlock - 1) / kPTBlock);
         // Persistent traversal grids: the device fill, never more than the queue capacity needs with a
         // wave per ray.
         const dim3 grid_t(std::min<uint32_t>((cap + kTraceBlock / 64 - 1) / (kTraceBlock / 64), trace_grid));
