@@ -1040,10 +1040,16 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
 // idles in a divergent descent -- the loop of the reference's NaiveScene
 // (scene.naive.cpp:31-124) with the watertight test.  A box room of a few dozen triangles
 // costs a BVH descent through overlapping wall boxes that several times this loop costs.
-// Measured crossovers (the room with extra boxes, 256x256x16, BVH -> every triangle): ray
-// batches as pt's extension stage, 138 triangles 1.09 -> 1.06 ms, 234: 1.15 -> 1.51; pt with
-// the rays traced inside its shading kernel, 138: 1.09 -> 0.81, 234: 1.15 -> 1.21; pt.direct
-// (a closest and an any hit per vertex), 36: 1.47 -> 0.73, 138: 1.92 -> 2.03.
+// Every triangle against the BVH today, us: 1M closest hits (FP64) 42 triangles of the room 68 and
+// 99, 90 113 and 103, soups of 60 84 and 106, 90 116 and 123, 128 157 and 149; any hits 42 60 and
+// 55, soups of 36 52 and 58, 60 79 and 79, 128 159 and 111; 65,549 closest hits 42 19 and 34,
+// 128 43 and 60.  Batches of up to 8192 rays are faster through trace_grouped at any size (81 rays:
+// 36 triangles 13 and 8, 128 40 and 9), but a scene takes one way for all its batches: the two tests
+// round differently, and a ray's result must not depend on its batch.  Renders of 256 x 256 x 16:
+// pt 42 335 and 738, 138 511 and 698, 186 616 and 765; pt.direct 810 and 1520, 1226 and 1472, 1470
+// and 1571.  The lines are those drawn on the descent of 128-byte nodes, where pt.direct crossed at
+// 130 triangles and closest hits at 140; on today's closest hits cross at 75 to 110, any hits at 40
+// to 60 and pt.direct beyond 186.
 constexpr uint32_t kBruteMaxTris = 128;    // ray batches, pt.direct / pt.mis
 constexpr uint32_t kBruteMaxTrisPt = 192;  // pt (and the LDS copy of the records)
 
