@@ -24,6 +24,9 @@ namespace lmgpu {
 constexpr float kBoxRobust = 1.0f + 2.0f * 4.8e-7f;
 // The same for a box whose planes are at hand: 1 + 2 gamma(4).
 constexpr float kBoxRobustExact = 1.0f + 2.0f * 2.4e-7f;
+// t moved up by k's excess over 1 of itself: t * k, also behind the origin, where a product would
+// move it down.
+LMGPU_HD float widened(float t, float k) { return fmaf(fabsf(t), k - 1.0f, t); }
 // 1 - 4u: see hit_order.
 constexpr float kOrderScale = 1.0f - 2.384185791015625e-7f;
 
@@ -62,8 +65,8 @@ LMGPU_HD Slab make_slab(float ox, float oy, float oz, float ix, float iy, float 
     return s;
 }
 
-// Where a ray enters and leaves a box within [tmin, tmax]; it meets the box if tn <= tf *
-// kBoxRobustExact.  Monotone in every plane: a box that contains this one is met too.
+// Where a ray enters and leaves a box within [tmin, tmax]; it meets the box if
+// tn <= widened(tf, kBoxRobustExact).  Monotone in every plane: a box that contains this one is met too.
 LMGPU_HD void box_span(const Slab& s, float lx, float hx, float ly, float hy, float lz, float hz, float tmin, float tmax,
                        float& tn, float& tf) {
     tn = fmaxf(fmaxf(fmaf(s.ix >= 0.f ? lx : hx, s.ix, s.nx), fmaf(s.iy >= 0.f ? ly : hy, s.iy, s.ny)),
@@ -83,7 +86,8 @@ LMGPU_HD PackedAxis packed_axis(float origin, float step, uint32_t lo, uint32_t 
     return PackedAxis{step * inv, fmaf(origin, inv, near_off), fmaf(origin, inv, far_off), inv >= 0.f ? lo : hi,
                       inv >= 0.f ? hi : lo};
 }
-// Child i's span within [tmin, tmax]; the ray may meet the child if tn <= tf * kBoxRobust.
+// Child i's span within [tmin, tmax]; the ray may meet the child if
+// tn <= widened(tf, kBoxRobust).
 LMGPU_HD void packed_span(const PackedAxis& x, const PackedAxis& y, const PackedAxis& z, int i, float tmin, float tmax,
                           float& tn, float& tf) {
     auto at = [i](uint32_t q, float a, float off) { return fmaf(float((q >> (8 * i)) & 0xffu), a, off); };

@@ -300,7 +300,7 @@ __device__ __forceinline__ void node_children(const NodeFetch& fetch, uint32_t c
     for (int i = 0; i < 4; i++) {
         float tn, tf;
         packed_span(x, y, z, i, tmin, tmax, tn, tf);
-        e[i] = pack_entry(tn <= tf * kBoxRobust ? tn : INFINITY, __float_as_uint(c[i]));
+        e[i] = pack_entry(tn <= widened(tf, kBoxRobust) ? tn : INFINITY, __float_as_uint(c[i]));
     }
     cswap(e[0], e[1]);
     cswap(e[2], e[3]);
@@ -441,7 +441,7 @@ __device__ __forceinline__ float built_child(const BvhDev& bvh, const Slab& s, u
     child = __float_as_uint(nd[24]);
     float tn;
     box_span(s, nd[0], nd[4], nd[8], nd[12], nd[16], nd[20], tmin, tmax, tn, tf);
-    return child != kEmptyChild && tn <= tf * kBoxRobustExact ? tn : INFINITY;
+    return child != kEmptyChild && tn <= widened(tf, kBoxRobustExact) ? tn : INFINITY;
 }
 
 // Whether a ray meets the box of a record's leaf as it was built (lx, hx: its x range, the fourth
@@ -452,15 +452,15 @@ __device__ __forceinline__ bool in_leaf_box(const LeafTri& rec, float lx, float 
     const float4 b = *reinterpret_cast<const float4*>(rec.box_yz);
     float tf;
     box_span(s, lx, hx, b.x, b.y, b.z, b.w, tmin, tmax, tn, tf);
-    return tn <= tf * kBoxRobustExact;
+    return tn <= widened(tf, kBoxRobustExact);
 }
 
 // What orders a ray's hits: the distance, but no less than where the ray enters the hit's leaf.  The
 // FP32 test of a triangle that is large, thin or seen edge-on can place a hit before its own box;
 // a descent that has met a hit between the two by then leaves the box out, another finds it first.
 // Ordered so, no box test leaves out a hit that comes before the nearest one so far, whatever the
-// order of the descent (tn * (1 - 4u) < tmax implies tn <= tmax * (1 + 8u)), and every kernel finds
-// the same one (tmin >= 0).
+// order of the descent (tn * (1 - 4u) < tmax implies tn <= tmax + 8u |tmax|), and every kernel finds
+// the same one.
 __device__ __forceinline__ float hit_order(float t, float tn) { return fmaxf(t, tn * kOrderScale); }
 
 // A descent that takes hits by their distance alone, and through packed boxes, ends at the first hit
@@ -530,7 +530,7 @@ __device__ __forceinline__ uint32_t trace_exact(const BvhDev& bvh, const RayIn& 
                 const float tf = fminf(fminf(fmaf(fx[i], s.ix, s.fx), fmaf(fy[i], s.iy, s.fy)),
                                        fminf(fmaf(fz[i], s.iz, s.fz), far));
                 val[i] = __float_as_uint(c[i]);
-                key[i] = val[i] != kEmptyChild && tn <= tf * kBoxRobustExact ? tn : INFINITY;
+                key[i] = val[i] != kEmptyChild && tn <= widened(tf, kBoxRobustExact) ? tn : INFINITY;
                 if (tf < near) val[i] = kEmptyChild;
             }
             sort4(key, val);
@@ -893,7 +893,7 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
             bool hit = false;
             float tn = INFINITY;
             uint32_t child = kEmptyChild;
-            if (slot < take && !(__uint_as_float(e.y) > tmax * kBoxRobustExact)) {
+            if (slot < take && !(__uint_as_float(e.y) > widened(tmax, kBoxRobustExact))) {
                 if (kCount) cnt.nodes += sub == 0u ? 1u : 0u;
                 float tf;
                 tn = built_child(bvh, sl, e.x, sub, r.tmin, tmax, child, tf);

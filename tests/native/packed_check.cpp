@@ -11,8 +11,8 @@
 //      by the margin; empty slots are inverted one-record leaves;
 //   3. whatever ray and interval the built box's test accepts, the packed test accepts, and an entry
 //      is not taken off the stack by a hit that comes after it (hit_order): rays from inside, from
-//      faces, at corners and edges, from 1 to 1e6 extents away, in planes and with denormal
-//      direction components, with reciprocals 1 ulp off.
+//      faces, at corners and edges, from 1 to 1e6 extents away, in planes and with denormal direction
+//      components, with reciprocals 1 ulp off, forward and behind the origin.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -71,13 +71,13 @@ static void check_ray(const Node4& n, const NodeQ& q, int i, const float o[3], c
         float tn, tf, pn, pf;
         box_span(s, n.lo_x[i], n.hi_x[i], n.lo_y[i], n.hi_y[i], n.lo_z[i], n.hi_z[i], tmin, tmax, tn, tf);
         tested++;
-        if (!(tn <= tf * kBoxRobustExact)) return;
+        if (!(tn <= widened(tf, kBoxRobustExact))) return;
         accepted++;
         // As it is, and with the nearest hit so far just behind this child's earliest one.
         const float near = rep == 0 ? tmax : std::nextafter(tn * kOrderScale, INFINITY);
-        if (!(near <= tmax) || !(near > 0.f)) return;
+        if (!(near <= tmax)) return;
         packed_span(x, y, z, i, tmin, near, pn, pf);
-        CHECK(pn <= pf * kBoxRobust && !(pn > fmaxf(near * kBoxRobust, 0.f)),
+        CHECK(pn <= widened(pf, kBoxRobust) && !(pn > fmaxf(near * kBoxRobust, 0.f)),
               "child %d entered [%.9g, %.9g] (nearest %.9g), packed [%.9g, %.9g]: o %g %g %g d %g %g %g\n", i, double(tn),
               double(tf), double(near), double(pn), double(pf), double(o[0]), double(o[1]), double(o[2]), double(d[0]),
               double(d[1]), double(d[2]));
@@ -140,6 +140,9 @@ static void check_node(const Node4& n, int rays) {
             }
             const float tmin = rng() % 2 ? 0.f : float(len * U());
             check_ray(n, q, i, o, d, tmin, rng() % 2 ? 3.4028234e38f : float(len * (0.5 + U())));
+            // The same behind the origin.
+            for (float& x : d) x = -x;
+            check_ray(n, q, i, o, d, rng() % 2 ? -3.4028234e38f : float(-len * (0.5 + U())), -tmin);
         }
     }
 }

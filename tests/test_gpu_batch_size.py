@@ -93,3 +93,25 @@ def test_results_do_not_depend_on_the_batch(gpu, kind, leaf):
                 bad = np.flatnonzero(~((a == b[part]) | (np.isnan(a) & np.isnan(b[part]))))
                 assert len(bad) == 0, f"n {n} fp64 {fp64} {name}: {len(bad)} rays differ, first {bad[:3]}"
         np.testing.assert_array_equal(gpu.trace_any(many), any_want[part], err_msg=f"n {n}")
+
+
+@pytest.mark.parametrize("n", [100, 40_000, 120_000])
+def test_hits_behind_the_origin(gpu, n):
+    """Intervals of negative distances, among boxes without extent: whether -d hits in (-T, 0) is
+    whether d does in (0, T), as the triangle test is the same but for the sign of t."""
+    r = np.random.default_rng(11)
+    v = r.uniform(0, 1, (600, 1, 3)) + r.normal(size=(600, 3, 3)) * 0.1
+    flat = np.arange(600)
+    v[flat, :, flat % 3] = v[flat, :1, flat % 3]
+    P = v.reshape(-1, 3).astype(np.float32)
+    gpu.upload(scenes.Scene("flat", P, np.zeros_like(P), np.arange(len(P), dtype=np.uint32).reshape(-1, 3)))
+    gpu.build_bvh()
+    o = r.uniform(-0.5, 1.5, (n, 3)).astype(np.float32)
+    d = r.normal(size=(n, 3))
+    d = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
+    T, zero = r.uniform(0.1, 3.0, n).astype(np.float32), np.zeros(n, np.float32)
+    ahead = gpu.trace_any(scenes.Rays(o, d, zero, T))
+    back = scenes.Rays(o, -d, -T, zero)
+    assert 0.1 < ahead.mean() < 0.9
+    np.testing.assert_array_equal(gpu.trace_any(back), ahead)
+    np.testing.assert_array_equal(gpu.trace_closest(back)[3] >= 0, ahead)
