@@ -52,6 +52,8 @@ HIT_BYTES = 16    # t, b0, b1, prim
 #   pt shading of one path: path in 48 B (3 records), hit 4 B, triangle 48 B, shading record 64 B, material 16 B;
 #     a surviving path out 48 B, an ending path one film update 12 B;
 #   camera stage: one path out, 48 B.
+# A node visit counts as a packed node.  Segments of at most 65,536 rays (98,304 shadow rays) visit
+# the nodes as built, 128 B, so the stages' bytes are a lower bound.
 EXT_RAY_BYTES = 32 + 4
 SHADOW_RAY_BYTES = 48 + 12
 SHADE_IN_BYTES = 48 + 4 + 48 + 64 + 16
