@@ -17,18 +17,24 @@
 
 namespace lmgpu {
 
-// Packed boxes: 1 + 2 gamma(8), gamma(n) = n u / (1 - n u), u = 2^-24.  Against the built box's test
-// (1 + 2 gamma(4)) each of the two distances is off by 3 more roundings, the node's offset
-// fma(origin, inv, offset), the step's product and the plane's own FMA, beyond what the planes'
-// margin covers: whatever the built box accepts the packed one accepts.
-constexpr float kBoxRobust = 1.0f + 2.0f * 4.8e-7f;
-// The same for a box whose planes are at hand: 1 + 2 gamma(4).
+// u = 2^-24, gamma(n) = n u / (1 - n u).  A box whose planes are at hand is met with 1 + 2 gamma(4).
 constexpr float kBoxRobustExact = 1.0f + 2.0f * 2.4e-7f;
+// What a hit's leaf may lie behind the hit by without being taken for another order (hit_order), 64u
+// of the distance: of rays that meet a triangle in an axis-parallel plane the FP32 distance lies before
+// the plane by more than 4u for 1 in 300, by more than 64u for 1 in 12,000.
+constexpr float kOrderScale = 1.0f - 64.0f * 5.9604645e-8f;
+// A box is left out for a hit that comes before it if it lies behind that hit by more than this: 1 +
+// 72u, so that no hit that comes first in the order is (1 / kOrderScale is 1 + 64.0002u, and the
+// products round).
+constexpr float kOrderPrune = 1.0f + 72.0f * 5.9604645e-8f;
+// Packed boxes: 1 + 80u.  Against the built box's distances each of the two is off by 3 more roundings,
+// the node's offset fma(origin, inv, offset), the step's product and the plane's own FMA, beyond what
+// the planes' margin covers: whatever the built box accepts the packed one accepts, and what
+// kOrderPrune keeps it keeps.
+constexpr float kBoxRobust = 1.0f + 80.0f * 5.9604645e-8f;
 // t moved up by k's excess over 1 of itself: t * k, also behind the origin, where a product would
 // move it down.
 LMGPU_HD float widened(float t, float k) { return fmaf(fabsf(t), k - 1.0f, t); }
-// 1 - 4u: see hit_order.
-constexpr float kOrderScale = 1.0f - 2.384185791015625e-7f;
 
 // Per-ray constants of the slab test.  A plane at coordinate x is reached at
 // t = fma(x, inv, offset).  The offset fma(-o, inv, -+e) is -o * inv -+ e rounded once, so

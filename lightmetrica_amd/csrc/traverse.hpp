@@ -459,8 +459,7 @@ __device__ __forceinline__ bool in_leaf_box(const LeafTri& rec, float lx, float 
 // FP32 test of a triangle that is large, thin or seen edge-on can place a hit before its own box;
 // a descent that has met a hit between the two by then leaves the box out, another finds it first.
 // Ordered so, no box test leaves out a hit that comes before the nearest one so far, whatever the
-// order of the descent (tn * (1 - 4u) < tmax implies tn <= tmax + 8u |tmax|), and every kernel finds
-// the same one.
+// order of the descent (kOrderPrune), and every kernel finds the same one.
 __device__ __forceinline__ float hit_order(float t, float tn) { return fmaxf(t, tn * kOrderScale); }
 
 // A descent that takes hits by their distance alone, and through packed boxes, ends at the first hit
@@ -552,7 +551,7 @@ __device__ __forceinline__ uint32_t trace_exact(const BvhDev& bvh, const RayIn& 
                 const float at = hit_order(t, tn);
                 if (first ? at == t_hit : at < best) {
                     best = at;
-                    far = fminf(at, r.tmax);
+                    far = fminf(widened(at, kOrderPrune), r.tmax);
                     rec = k;
                     if (first) return rec;
                 }
@@ -877,7 +876,7 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
         const RayIn r = src(i);
         const Slab sl = make_slab(r);
         const ShearCyclic sh = make_shear_cyclic(r);
-        float tmax = r.tmax;
+        float tmax = r.tmax, limit = r.tmax;  // boxes that begin beyond `limit` hold no hit before tmax
         HitOut h{};
         float nearest = INFINITY;         // of the triangles this lane met: h.rec
         bool found = false, tie = false;  // of the ray
@@ -893,10 +892,10 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
             bool hit = false;
             float tn = INFINITY;
             uint32_t child = kEmptyChild;
-            if (slot < take && !(__uint_as_float(e.y) > widened(tmax, kBoxRobustExact))) {
+            if (slot < take && !(__uint_as_float(e.y) > widened(limit, kBoxRobustExact))) {
                 if (kCount) cnt.nodes += sub == 0u ? 1u : 0u;
                 float tf;
-                tn = built_child(bvh, sl, e.x, sub, r.tmin, tmax, child, tf);
+                tn = built_child(bvh, sl, e.x, sub, r.tmin, limit, child, tf);
                 hit = tn < INFINITY;
             }
             const bool inner = hit && is_inner(child), leaf = hit && !is_inner(child);
@@ -951,6 +950,7 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
 #pragma unroll
                         for (int off = kLanes / 2; off > 0; off >>= 1) m = fminf(m, __shfl_xor(m, off, 64));
                         tmax = m;
+                        limit = fminf(widened(m, kOrderPrune), r.tmax);
                         tie = __popcll(ballot(met && t == tmax)) > 1;
                     }
                 }
@@ -1017,7 +1017,7 @@ __device__ __forceinline__ void trace_grouped(const BvhDev& bvh, uint32_t n, Gro
                         if (first ? ballot(at == tmax) != 0ull : best < tmax) {
                             if (!first) {
                                 tmax = best;
-                                far = fminf(best, r.tmax);
+                                far = fminf(widened(best, kOrderPrune), r.tmax);
                             }
                             found = true;
                             // Of equal ones the first record, the lowest lane's.
