@@ -17,16 +17,16 @@
 //   * boxes are tested with the reciprocal-direction slab test in fused form, one FMA
 //     per plane (step * (scale * inv) + (origin * inv + offset)); the per-ray offsets -o * inv
 //     are widened by the rounding that form adds, packed planes are moved out by more than
-//     theirs, and the exit distance is scaled by 1 + 2*gamma(6), so rounding never culls a
-//     box the ray touches (Ize, "Robust BVH Ray Traversal", JCGT 2013, with the absolute
-//     error of the fused form and the 1-ulp hardware reciprocal accounted for);
+//     theirs, and the exit distance is moved up by 2 gamma(4) of itself (packed boxes: 80u), so
+//     rounding never culls a box the ray touches (Ize, "Robust BVH Ray Traversal", JCGT 2013, with
+//     the absolute error of the fused form and the 1-ulp hardware reciprocal accounted for);
 //   * triangles use the watertight test of Woop, Benthin and Wald (JCGT 2013), with
 //     the FP64 fallback for edge functions that evaluate to exactly zero.
 // Measured on 16M incoherent rays against 1M triangles (closest hit with the FP64 pass):
 // 3.98 ms with separate node and leaf loops over 128-byte nodes and unaligned leaves, 3.11 ms
-// so; 4M any-hit segments 1.75 -> 1.30 ms; the extension rays of a 96k-triangle room (8.4M
+// so; 4M any-hit segments 1.75 -> 1.29 ms; the extension rays of a 96k-triangle room (8.4M
 // paths, 8 segments, twice) 15.2 -> 10.3 ms.  With 128-byte nodes in the same loop: 3.35, 1.65 and
-// 13.8 ms.  Of that 0.05, 0 and 0.2 ms go into checking each ray's last hit against the built boxes
+// 13.8 ms.  Of that 0.05, 0 and 0.1 ms go into checking each ray's last hit against the built boxes
 // (sound_hit); checked as each hit is met it took 0.13, 0.04 and 0.5 ms.
 // Acceptance follows the reference's QBVH: t strictly inside (tmin, tmax), the first
 // triangle found wins an exact tie (scene.qbvh.cpp:124-133).
